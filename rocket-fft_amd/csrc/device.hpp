@@ -215,6 +215,9 @@ __device__ __forceinline__ void dftp(C2<T> *v, T dir, const C2<T> *__restrict__ 
 }
 
 template <int R, typename T>
+__device__ void dft_pfa(C2<T> *v, T dir);  // butterfly.hpp
+
+template <int R, typename T>
 __device__ __forceinline__ void dft(C2<T> *v, T dir, const C2<T> *g) {
   if constexpr (R == 2) dft2(v);
   else if constexpr (R == 3) dft3(v, dir);
@@ -223,6 +226,7 @@ __device__ __forceinline__ void dft(C2<T> *v, T dir, const C2<T> *g) {
   else if constexpr (R == 8) dft8(v, dir);
   else if constexpr (R == 9) dft9(v, dir);
   else if constexpr (R == 16) dft16(v, dir);
+  else if constexpr (R == 6 || R == 10 || R == 12 || R == 14 || R == 15) dft_pfa<R>(v, dir);
   else dftp<R>(v, dir, g);
 }
 
@@ -374,6 +378,7 @@ struct LineArgs {
   int shift;
   const C2<T> *t0, *t1, *t2;  // op tables
   int rot_in, rot_out;  // element-index rotations of the line set (0: none)
+  int op;
 };
 
 // (j + r) mod n for 0 <= j, r < n
@@ -453,12 +458,25 @@ __device__ __forceinline__ C2<T> expipi(int64_t num, int64_t den) {
   }
 }
 
-// Element j of the complex work line built from input line x (element
-// stride es) for the real-transform modes of PreMode; m = work length.
+// e^{i pi num / 4n}, num >= 0: computed, or from a table of the plan's (num
+// <= 2n).  The DCT / DST factors e^{i pi j / 2n} and e^{i pi (2j + 1) / 4n}.
 template <typename T>
-__device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int64_t n,
-                                          int64_t m, int64_t j, bool ortho, bool conj,
-                                          bool flip) {
+struct ComputedRoot {
+  int64_t n;
+  __device__ __forceinline__ C2<T> operator()(int64_t num) const { return expipi<T>(num, 4 * n); }
+};
+template <typename T>
+struct TableRoot {
+  const C2<T> *t;
+  __device__ __forceinline__ C2<T> operator()(int num) const { return t[num]; }
+};
+
+// Element j of the complex work line built from input line x (element
+// stride es) for the real-transform modes of PreMode; m = work length.  I: the
+// type of indices within a line.
+template <typename T, typename I, typename Rt>
+__device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, I n, I m, I j,
+                                          bool ortho, bool conj, bool flip, const Rt &root) {
   const T sqrt2 = T(1.41421356237309504880168872420969808);
   C2<T> v = {T(0), T(0)};
   switch (mode) {
@@ -470,7 +488,7 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int6
       }
       break;
     case kPreHermitian: {  // half complex input X[0..n/2]
-      const int64_t h = n / 2;
+      const I h = n / 2;
       if (j == 0) {
         v = C2<T>{x[0], T(0)};
       } else if (j < n - h || (2 * j < n)) {
@@ -479,14 +497,14 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int6
       } else if (2 * j == n) {
         v = C2<T>{x[j * es], T(0)};
       } else {
-        const int64_t k = n - j;
+        const I k = n - j;
         v = C2<T>{x[k * es], x[k * es + 1]};
         if (!conj) v.y = -v.y;
       }
       break;
     }
     case kPreDct1: {
-      const int64_t src = j < n ? j : m - j;
+      const I src = j < n ? j : m - j;
       T xv = x[src * es];
       if (ortho && (src == 0 || src == n - 1)) xv *= sqrt2;
       v.x = xv;
@@ -504,7 +522,7 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int6
         T xv = x[j * es];
         if (j == 0 && ortho) xv *= sqrt2;
         const T w = j == 0 ? T(1) : T(2);
-        v = (w * xv) * expipi<T>(j, 2 * n);
+        v = (w * xv) * root(2 * j);
       }
       break;
     case kPreDst3:
@@ -512,11 +530,11 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int6
         T xv = x[(j - 1) * es];
         if (j == 1 && ortho) xv *= sqrt2;
         const T w = j == n ? T(1) : T(2);
-        v = (w * xv) * expipi<T>(j, 2 * n);
+        v = (w * xv) * root(2 * j);
       }
       break;
     case kPreType4:
-      if (j < n) v = x[j * es] * expipi<T>(-j, 2 * n);
+      if (j < n) v = x[j * es] * conjc(root(2 * j));
       break;
     case kPreHalfcomplex: {
       if (j == 0) {
@@ -527,7 +545,7 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int6
       } else if (2 * j == n) {
         v.x = x[(n - 1) * es];
       } else {
-        const int64_t k = n - j;
+        const I k = n - j;
         v = C2<T>{x[(2 * k - 1) * es], -x[(2 * k) * es]};
         if (conj) v.y = -v.y;
       }
@@ -541,7 +559,7 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int6
       // v_j = x_2j for 2j < n, v_{n-1-j} = x_2j+1: V = FFT_n(v) gives
       // DCT-II_k = 2 Re(e^{-i pi k/2n} V_k); DST-II is DCT-II of (-1)^j x_j
       // read backwards
-      const int64_t i = 2 * j < n ? 2 * j : 2 * (n - 1 - j) + 1;
+      const I i = 2 * j < n ? 2 * j : 2 * (n - 1 - j) + 1;
       T xv = x[i * es];
       if (mode == kPreDst2N && (i & 1)) xv = -xv;
       v.x = xv;
@@ -552,21 +570,21 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, int6
       // a = x (DCT-III) or x reversed (DST-III), a_n = 0, ortho scales x_0 by
       // sqrt 2; V_j = (a_j - i a_{n-j}) e^{i pi j/2n} and the inverse FFT of
       // length n holds the even outputs up and the odd outputs down
-      auto at = [&](int64_t q) -> T {
+      auto at = [&](I q) -> T {
         if (q >= n) return T(0);
-        const int64_t src = mode == kPreDct3N ? q : n - 1 - q;
+        const I src = mode == kPreDct3N ? q : n - 1 - q;
         T xv = x[src * es];
         if (ortho && src == 0) xv *= sqrt2;
         return xv;
       };
-      v = cmul(C2<T>{at(j), -at(n - j)}, expipi<T>(j, 2 * n));
+      v = cmul(C2<T>{at(j), -at(n - j)}, root(2 * j));
       break;
     }
     case kPreHalfSpectrum: {
       // z_j = Σ_k [A_k + i e^{2πik/n} D_k] e^{2πikj/(n/2)} with A = X_k + conj X_{h-k},
       // D = X_k - conj X_{h-k}: the inverse FFT of length h = n/2 gives
       // y_2j + i y_2j+1.  Imaginary parts of bins 0 and h are ignored.
-      const int64_t h = n / 2;
+      const I h = n / 2;
       C2<T> xj = {x[j * es], x[j * es + 1]}, xm = {x[(h - j) * es], x[(h - j) * es + 1]};
       if (conj) {
         xj.y = -xj.y;
@@ -604,9 +622,9 @@ __device__ __forceinline__ C2<T> half_spectrum_bin(G &&get, int64_t n, int64_t k
 
 // Real output element k from the transformed work line (get(q) = bin q)
 // for the PostMode modes other than kPostComplexHalf; fct not applied.
-template <typename T, typename G>
-__device__ __forceinline__ T post_elem(int mode, G &&get, int64_t n, int64_t k, bool ortho,
-                                       bool flip) {
+template <typename T, typename I, typename G, typename Rt>
+__device__ __forceinline__ T post_elem(int mode, G &&get, I n, I k, bool ortho, bool flip,
+                                       const Rt &root) {
   const T isqrt2 = T(0.707106781186547524400844362104849039);
   T r = T(0);
   switch (mode) {
@@ -622,13 +640,13 @@ __device__ __forceinline__ T post_elem(int mode, G &&get, int64_t n, int64_t k, 
       r = -get(k + 1).y;
       break;
     case kPostDct2: {
-      const C2<T> z = cmul(get(k), expipi<T>(-k, 2 * n));
+      const C2<T> z = cmul(get(k), conjc(root(2 * k)));
       r = T(2) * z.x;
       if (ortho && k == 0) r *= isqrt2;
       break;
     }
     case kPostDst2: {
-      const C2<T> z = cmul(get(k + 1), expipi<T>(-(k + 1), 2 * n));
+      const C2<T> z = cmul(get(k + 1), conjc(root(2 * (k + 1))));
       r = -T(2) * z.y;
       if (ortho && k == 0) r *= isqrt2;
       break;
@@ -641,7 +659,7 @@ __device__ __forceinline__ T post_elem(int mode, G &&get, int64_t n, int64_t k, 
       break;
     case kPostDct4:
     case kPostDst4: {
-      const C2<T> z = cmul(get(k), expipi<T>(-(2 * k + 1), 4 * n));
+      const C2<T> z = cmul(get(k), conjc(root(2 * k + 1)));
       r = mode == kPostDct4 ? T(2) * z.x : -T(2) * z.y;
       break;
     }
@@ -658,8 +676,8 @@ __device__ __forceinline__ T post_elem(int mode, G &&get, int64_t n, int64_t k, 
       break;
     case kPostDct2N:
     case kPostDst2N: {
-      const int64_t q = mode == kPostDct2N ? k : n - 1 - k;
-      const C2<T> z = cmul(get(q), expipi<T>(-q, 2 * n));
+      const I q = mode == kPostDct2N ? k : n - 1 - k;
+      const C2<T> z = cmul(get(q), conjc(root(2 * q)));
       r = T(2) * z.x;
       if (ortho && k == 0) r *= isqrt2;
       break;
@@ -801,6 +819,11 @@ __device__ C2<T> *run_stages(const FftDesc &f, int s0, int s1, C2<T> *a, C2<T> *
       case 11: stage_fixed<11>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
       case 13: stage_fixed<13>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
       case 17: stage_fixed<17>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
+      case 6: stage_fixed<6>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
+      case 10: stage_fixed<10>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
+      case 12: stage_fixed<12>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
+      case 14: stage_fixed<14>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
+      case 15: stage_fixed<15>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
       case 16: stage_fixed<16>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
       default: stage_generic(a, b, L, ld, f.n, st.radix, st.ns, t, g, dir); break;
     }
@@ -891,8 +914,7 @@ __device__ __forceinline__ void line_body(const LineArgs<T> &a, int64_t tile,
       const C2<T> B = cmul(xj - conjc(xm), conjc(a.t0[j]));
       v = C2<T>{A.x - B.y, A.y + B.x};
     } else if constexpr (OP == OP_R2R) {
-      v = pre_elem<T>(a.sub & 0xff, base, a.esi, a.bign, a.f.n, j, (a.sub & R2R_ORTHO) != 0,
-                      (a.sub & R2R_CONJ) != 0, (a.sub & R2R_FLIP) != 0);
+      v = C2<T>{T(0), T(0)};
     } else {  // OP_C2R_ODD
       const int n = a.f.n;
       if (j == 0) {
@@ -1024,9 +1046,7 @@ __device__ __forceinline__ void line_body(const LineArgs<T> &a, int64_t tile,
       stc<VOUT>(base + k * a.eso, a.fct * X);
     } else if constexpr (OP == OP_R2R) {
       T *base = a.out + s_oo[l];
-      base[k * a.eso] = a.fct * post_elem<T>((a.sub >> 8) & 0xff, [&](int64_t q) { return r[q]; },
-                                             a.bign, k, (a.sub & R2R_ORTHO) != 0,
-                                             (a.sub & R2R_FLIP) != 0);
+      (void)base;
     } else {
       store(l, k, r[k]);
     }

@@ -327,8 +327,8 @@ void r2r_axis(Ctx &c, const int64_t *shape, int nd, int ax, const int64_t *si,
   LineSet g = lines_for_axis(shape, nd, ax, si, so, in, out);
   rr.n = shape[ax];
   rr.m = m;
-  auto plan = get_c2c_plan(uint64_t(m), c.dbl);
-  if (plan->kind == kDirect) {  // the whole work line fits in LDS: one launch
+  // the whole work line fits in LDS: one launch
+  if (auto plan = get_r2r_plan(uint64_t(rr.n), uint64_t(m), c.dbl)) {
     launch_r2r_fused(*plan, g, pre, post, rr, fft_forward, fct, c.s);
     return;
   }

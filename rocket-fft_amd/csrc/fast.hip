@@ -784,11 +784,13 @@ bool go_op(const LineArgs<T> &a, bool lf_in, bool lf_out, bool vin, bool vout,
 
 }  // namespace
 
+#ifndef RFH_FAST_F64
 bool g_fast_enabled = true;
 
 bool fast_interleaved_ok(uint64_t n, bool dbl) {
   return dbl ? interleaved_ok_t<double>(n) : interleaved_ok_t<float>(n);
 }
+#endif
 
 // Launches the specialised kernel for (op, length, layout) when one exists.
 template <typename T>
@@ -806,9 +808,12 @@ bool launch_fast(int op, const LineArgs<T> &a, bool lf_in, bool lf_out, bool vin
   }
 }
 
-template bool launch_fast<float>(int, const dev::LineArgs<float> &, bool, bool, bool, bool,
-                                 hipStream_t);
+#ifdef RFH_FAST_F64
 template bool launch_fast<double>(int, const dev::LineArgs<double> &, bool, bool, bool, bool,
                                   hipStream_t);
+#else
+template bool launch_fast<float>(int, const dev::LineArgs<float> &, bool, bool, bool, bool,
+                                 hipStream_t);
+#endif
 
 }  // namespace rfh

@@ -1,11 +1,11 @@
 // kernels.hip -- gfx950 kernels of the transform engine.
 //
-// The workhorse is k_lines: one workgroup owns L whole lines, loads them
-// (coalesced: consecutive lanes take consecutive elements of a line, or the
-// same element of adjacent lines when the lines are interleaved in memory),
-// runs every Stockham stage of the line FFT out of LDS (two ping-pong
-// buffers, one barrier per stage), and stores.  Per-operation load/store
-// hooks fuse the reference's pre/post processing into the same pass:
+// The workhorse is the general line kernel k_lines (mixline.hpp): one
+// workgroup owns L whole lines, loads them (coalesced: consecutive lanes take
+// consecutive elements of a line, or the same element of adjacent lines when
+// the lines are interleaved in memory), runs every stage of the line FFT out
+// of LDS and stores.  Per-operation load / store hooks fuse the reference's
+// pre/post processing into the same pass:
 //   * c2c with the output factor fct                (ExecC2C, H:3646-3659)
 //   * real -> n/2+1 bins and back through a half-length complex FFT
 //     (general_r2c / general_c2r, H:3723-3852)
@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "bufio.hpp"
+#include "mixline.hpp"
 #include "passes.hpp"
 
 namespace rfh {
@@ -32,14 +33,6 @@ namespace {
 using namespace dev;
 
 thread_local const char *t_last_family = "k_lines";  // kernel family of the last launch
-
-template <typename T, int OP, bool VIN, bool VOUT, int NT = kThreads>
-__global__ void __launch_bounds__(NT) k_lines(const LineArgs<T> a) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ int64_t s_oi[kMaxLinesPerGroup], s_oo[kMaxLinesPerGroup];
-  __shared__ int s_aux[kMaxLinesPerGroup];
-  line_body<T, OP, VIN, VOUT>(a, int64_t(xcd_tile()), smem_raw, s_oi, s_oo, s_aux);
-}
 
 // ----------------------------------------------------------- host launch
 
@@ -88,77 +81,6 @@ bool pairs_aligned(const void *p, size_t scalar, int64_t es, const int64_t *bs, 
   return true;
 }
 
-std::mutex g_attr_mu;
-std::set<std::pair<int, const void *>> g_attr_done;
-
-// Raises a kernel's dynamic-LDS ceiling to what the device allows beside the
-// kernel's static LDS (once per kernel and device).
-void allow_lds(const void *fn, size_t bytes) {
-  if (bytes <= 65536) return;
-  int dev = 0;
-  HIP_CHECK(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lk(g_attr_mu);
-  if (g_attr_done.count({dev, fn})) return;
-  hipFuncAttributes fa;
-  HIP_CHECK(hipFuncGetAttributes(&fa, fn));
-  const int dyn = int(lds_limit()) - int(fa.sharedSizeBytes);
-  if (int64_t(bytes) > dyn)
-    RFH_THROW(3, "line kernel needs " + std::to_string(bytes) + " B of LDS beside " +
-                     std::to_string(fa.sharedSizeBytes) + " B static; device allows " +
-                     std::to_string(lds_limit()));
-  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
-  if (e != hipSuccess)
-    RFH_THROW(2, std::string("hipFuncSetAttribute(MaxDynamicSharedMemorySize, ") +
-                     std::to_string(dyn) + "): " + hipGetErrorString(e));
-  g_attr_done.insert({dev, fn});
-}
-
-// Threads of the wide line workgroups: 1024 for complex64 (the float line
-// kernels stay within the 128 registers that allows), 512 for complex128
-// (within 256).
-template <typename T>
-constexpr int kWideThreads = sizeof(T) == 4 ? 1024 : 512;
-
-template <typename T, int OP, bool VIN, bool VOUT>
-void launch_one(const LineArgs<T> &a, size_t lds, hipStream_t s) {
-  const int64_t groups = (a.nlines + a.L - 1) / a.L;
-  if (groups > 0x7fffffff / kThreads) RFH_THROW(3, "batch too large for one launch");
-  bool wide = false;
-  if constexpr (OP == OP_C2C || OP == OP_BLUE) {
-    // At most one group per CU, the launch is bound by each group's stage
-    // latency (four waves per CU at the narrow width): a wider group runs a
-    // stage's butterflies in fewer rounds, as long as every thread still has
-    // two (complex64) or four (complex128) elements of the group; below that
-    // the wider barriers cost more than they save (256 lines of complex128
-    // 1536: 10.1 us narrow, 10.8 us wide).
-    constexpr int64_t kMinElems = (sizeof(T) == 4 ? 2 : 4) * kWideThreads<T>;
-    wide = groups <= bufio::device_cus() && int64_t(a.L) * a.ld >= kMinElems;
-    if (wide) {
-      allow_lds(reinterpret_cast<const void *>(&k_lines<T, OP, VIN, VOUT, kWideThreads<T>>), lds);
-      hipLaunchKernelGGL((k_lines<T, OP, VIN, VOUT, kWideThreads<T>>), dim3(unsigned(groups)),
-                         dim3(kWideThreads<T>), lds, s, a);
-    }
-  }
-  if (!wide) {
-    allow_lds(reinterpret_cast<const void *>(&k_lines<T, OP, VIN, VOUT>), lds);
-    hipLaunchKernelGGL((k_lines<T, OP, VIN, VOUT>), dim3(unsigned(groups)), dim3(kThreads), lds,
-                       s, a);
-  }
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess)
-    RFH_THROW(2, std::string("line kernel launch (") + std::to_string(groups) + " groups, " +
-                     std::to_string(lds) + " B LDS, op " + std::to_string(OP) +
-                     "): " + hipGetErrorString(e));
-}
-
-template <typename T, int OP>
-void launch_var(const LineArgs<T> &a, size_t lds, bool vin, bool vout, hipStream_t s) {
-  if (vin && vout) launch_one<T, OP, true, true>(a, lds, s);
-  else if (vin) launch_one<T, OP, true, false>(a, lds, s);
-  else if (vout) launch_one<T, OP, false, true>(a, lds, s);
-  else launch_one<T, OP, false, false>(a, lds, s);
-}
-
 }  // namespace
 
 template <typename T>
@@ -199,9 +121,25 @@ LineArgs<T> make_line_args(const PassSpec &ps, const LineSet &g) {
   a.t2 = static_cast<const C2<T> *>(ps.t2);
   a.rot_in = int(g.rot_in);
   a.rot_out = int(g.rot_out);
+  a.op = ps.op;
   return a;
 }
 
+template <typename T>
+MixGeom make_mix_geom(const PassSpec &ps, const LineArgs<T> &a) {
+  MixGeom m = mix_geometry(a.f, ps.d->pbo, sizeof(T) == 8, a.nlines, a.lfast_in || a.lfast_out,
+                           ps.lines, lds_limit());
+  if (m.L == 0) RFH_THROW(3, "line does not fit in LDS");
+  // A line of at most 8 threads: its loads and stores by place would touch one
+  // cache line per 8 lanes or fewer, so the group's lines move as one run of
+  // elements through LDS (300000 lines of 30 complex64: 53.7 -> 46.0 us).
+  m.flat = ps.op == OP_C2C && !a.lfast_in && !a.lfast_out && m.T <= 8 && a.nb <= 1 &&
+           a.esi == 2 && a.eso == 2 && !a.rot_in && !a.rot_out;
+  return m;
+}
+
+template MixGeom make_mix_geom<float>(const PassSpec &, const LineArgs<float> &);
+template MixGeom make_mix_geom<double>(const PassSpec &, const LineArgs<double> &);
 template LineArgs<float> make_line_args<float>(const PassSpec &, const LineSet &);
 template LineArgs<double> make_line_args<double>(const PassSpec &, const LineSet &);
 
@@ -339,9 +277,6 @@ void run_pass(const PassSpec &ps, const LineSet &g, hipStream_t s) {
     return;
   }
   LineArgs<T> a = make_line_args<T>(ps, g);
-  const size_t elem = 2 * sizeof(T);
-  const size_t lds = size_t(2) * a.L * a.ld * elem;
-  if (lds + kLineStaticLds > lds_limit()) RFH_THROW(3, "line does not fit in LDS");
   bool vin, vout;
   if (ps.real_in)  // real pairs: 2-wide loads when the line is contiguous
     vin = g.esi == 1 && pairs_aligned(g.in, sizeof(T), 0, g.bsi, g.nb);
@@ -369,17 +304,15 @@ void run_pass(const PassSpec &ps, const LineSet &g, hipStream_t s) {
     t_last_family = "k_fast";
     return;
   }
+  const MixGeom m = make_mix_geom(ps, a);
   switch (ps.op) {
-    case OP_C2C: launch_var<T, OP_C2C>(a, lds, vin, vout, s); break;
-    case OP_PASSA: launch_var<T, OP_PASSA>(a, lds, vin, vout, s); break;
-    case OP_PASSB: launch_var<T, OP_PASSB>(a, lds, vin, vout, s); break;
-    case OP_BLUE: launch_var<T, OP_BLUE>(a, lds, vin, vout, s); break;
-    case OP_BLUEROW: launch_var<T, OP_BLUEROW>(a, lds, vin, vout, s); break;
-    case OP_R2C_EVEN: launch_var<T, OP_R2C_EVEN>(a, lds, vin, vout, s); break;
-    case OP_R2C_ODD: launch_var<T, OP_R2C_ODD>(a, lds, false, vout, s); break;
-    case OP_C2R_EVEN: launch_var<T, OP_C2R_EVEN>(a, lds, vin, vout, s); break;
-    case OP_C2R_ODD: launch_var<T, OP_C2R_ODD>(a, lds, vin, false, s); break;
-    case OP_R2R: launch_one<T, OP_R2R, false, false>(a, lds, s); break;
+    case OP_C2C:
+    case OP_PASSA:
+    case OP_PASSB: launch_mix_c2c(ps.op, a, m, s); break;
+    case OP_BLUE:
+    case OP_BLUEROW: launch_mix_blue(ps.op, a, m, s); break;
+    case OP_R2R: launch_mix_r2r(ps.op, a, m, s); break;
+    default: launch_mix_real(ps.op, a, m, s); break;
   }
 }
 
@@ -904,10 +837,11 @@ void launch_c2c(const C2CPlan &p, const LineSet &g, int dir, double fct, hipStre
   for (const PassLaunch &pl : passes) run_pass_any(p.dbl, pl.ps, pl.g, s);
 }
 
-void launch_r2r_fused(const C2CPlan &p, const LineSet &g, PreMode pre, PostMode post,
+void launch_r2r_fused(const R2RPlan &p, const LineSet &g, PreMode pre, PostMode post,
                       const RealPrePost &rr, bool fft_forward, double fct, hipStream_t s) {
   PassSpec ps;
-  ps.d = &p.main;
+  ps.d = &p.d;
+  ps.t0 = p.roots.p;
   ps.op = OP_R2R;
   ps.dir = fft_forward ? -1 : +1;
   ps.fct = fct;
@@ -987,7 +921,8 @@ __global__ void __launch_bounds__(kThreads) k_pre(const PrePostArgs<T> a) {
     const int64_t n = a.n;
     for (int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; j < a.m;
          j += int64_t(gridDim.x) * blockDim.x) {
-      t[j] = pre_elem<T>(a.mode, x, a.es, n, a.m, j, a.ortho, a.conj, a.flip);
+      t[j] = pre_elem<T, int64_t>(a.mode, x, a.es, n, a.m, j, a.ortho, a.conj, a.flip,
+                                  ComputedRoot<T>{n});
     }
   }
 }
@@ -1009,7 +944,8 @@ __global__ void __launch_bounds__(kThreads) k_post(const PrePostArgs<T> a) {
         y[k * a.es + 1] = a.fct * v.y;
         continue;
       }
-      const T r = post_elem<T>(a.mode, [&](int64_t q) { return t[q]; }, n, k, a.ortho, a.flip);
+      const T r = post_elem<T, int64_t>(a.mode, [&](int64_t q) { return t[q]; }, n, k, a.ortho,
+                                        a.flip, ComputedRoot<T>{n});
       y[k * a.es] = a.fct * r;
     }
   }

@@ -35,8 +35,16 @@ RFH_HD inline LineOffsets line_offsets(int64_t b, int nb, const int64_t *bdim,
   LineOffsets r{0, 0, 0};
   int64_t rem = b;
   for (int d = nb - 1; d >= 0; --d) {
-    const int64_t q = rem / bdim[d];
-    const int64_t idx = rem - q * bdim[d];
+    int64_t q = 0, idx = rem;  // the outermost index is what is left: no division
+    if (d > 0) {
+      if (((rem | bdim[d]) >> 32) == 0) {  // 64-bit division is a long sequence on the GPU
+        q = int64_t(uint32_t(rem) / uint32_t(bdim[d]));
+        idx = rem - q * bdim[d];
+      } else {
+        q = rem / bdim[d];
+        idx = rem - q * bdim[d];
+      }
+    }
     rem = q;
     r.oi += idx * bsi[d];
     r.oo += idx * bso[d];

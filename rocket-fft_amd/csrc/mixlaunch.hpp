@@ -1,0 +1,53 @@
+// mixlaunch.hpp -- launch of the general line kernel (mixline.hpp) for one
+// operation; each of lines_*.hip instantiates a few operations.
+#pragma once
+
+#include <mutex>
+#include <set>
+#include <string>
+#include <utility>
+
+#include "mixline.hpp"
+#include "passes.hpp"
+
+namespace rfh {
+
+template <typename T, int OP>
+__global__ void __launch_bounds__(dev::kMixThreads<T>)
+    k_lines(const dev::LineArgs<T> a, const MixGeom m) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  dev::mix_body<T, OP>(a, m, int64_t(dev::xcd_tile()), smem_raw);
+}
+
+template <typename T, int OP>
+void launch_mix_op(const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s) {
+  const size_t lds = size_t(m.L * m.ld + m.ngen) * 2 * sizeof(T);
+  const int64_t groups = (a.nlines + m.L - 1) / m.L;
+  const int threads = (m.L * m.T + 63) / 64 * 64;
+  if (groups > 0x7fffffff / dev::kMixThreads<T>) RFH_THROW(3, "batch too large for one launch");
+  if (threads > dev::kMixThreads<T> || lds > lds_limit())
+    RFH_THROW(3, "line group of " + std::to_string(a.f.n) + " needs " + std::to_string(threads) +
+                     " threads and " + std::to_string(lds) + " B of LDS");
+  if (lds > 65536) {  // raise the kernel's dynamic-LDS ceiling once per device
+    static std::mutex mu;
+    static std::set<int> done;
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(mu);
+    if (!done.count(dev)) {
+      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_lines<T, OP>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    int(lds_limit())));
+      done.insert(dev);
+    }
+  }
+  hipLaunchKernelGGL((k_lines<T, OP>), dim3(unsigned(groups)), dim3(unsigned(threads)), lds, s, a,
+                     m);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess)
+    RFH_THROW(2, std::string("line kernel launch (") + std::to_string(groups) + " groups, " +
+                     std::to_string(lds) + " B LDS, op " + std::to_string(OP) +
+                     "): " + hipGetErrorString(e));
+}
+
+}  // namespace rfh

@@ -1,0 +1,644 @@
+// mixline.hpp -- the general line kernel: a group of L lines of any length
+// whose stages run out of ONE line buffer per line in LDS.
+//
+// Each thread owns one place j of one line and holds the elements of its
+// butterflies of a stage in registers (at most kMaxElems of them: one
+// butterfly of a large radix, several of a small one): a stage reads its
+// inputs from LDS, waits until every thread has read, and writes its outputs
+// over them.  One buffer instead of two ping-pong buffers is half the LDS per
+// line, so twice the lines (waves) are resident per CU, and a thread's place
+// in its line is found once instead of per butterfly and stage.  The radices
+// (2 .. 17, gpu_radices) are chosen so that a stage's butterflies fill the
+// line's threads: 1000 = 10 x 10 x 10 is three stages of 100 threads.
+//
+// Layout between stages.  After the stage of radix R whose predecessors
+// multiply to ns, the line is N / (ns R) blocks of ns R elements; block q
+// starts at q P with a pitch P >= ns R chosen (block_pitch) so that the
+// stage's writes (runs of ns elements, P apart) spread over the LDS banks.
+// The next stage reads element j + r N/R' of the line at
+// (j / ns') P + j mod ns' + r (N/R'/ns') P: padding changes only the strides.
+//
+// Direction.  Every stage runs the forward transform; an inverse transform
+// exchanges real and imaginary parts as elements are loaded and stored.
+//
+// Bluestein (OP_BLUE, OP_BLUEROW).  The last forward stage holds bins
+// j + r N/R in registers, which are the inputs of the first stage of the
+// inverse transform run backwards (each stage undone in reverse order:
+// butterfly, conjugate twiddles, write to where the forward stage had read).
+// So the kernel product happens in registers between two butterflies, and the
+// inverse transform needs no tables of its own: S - 1 exchanges each way.
+#pragma once
+
+#include "butterfly.hpp"
+#include "mixgeom.hpp"
+
+namespace rfh {
+
+namespace dev {
+
+template <typename T>
+constexpr int kMaxElems = mix_max_elems(sizeof(T) == 8);
+template <typename T>
+constexpr int kMixThreads = mix_max_threads(sizeof(T) == 8);
+
+// OP of a kernel that runs every operation but the real-to-real ones, by
+// LineArgs::op (the batch executor's)
+constexpr int OP_ANY = -1;
+template <int OP, typename T>
+__device__ __forceinline__ int op_of(const LineArgs<T> &a) {
+  return OP == OP_ANY ? a.op : OP;
+}
+__device__ __forceinline__ bool is_blue(int op) { return op == OP_BLUE || op == OP_BLUEROW; }
+// whether an op stores bin by bin, straight from the last stage's registers
+__device__ __forceinline__ bool elem_store(int op) { return op != OP_R2C_EVEN && op != OP_R2R; }
+
+template <typename T>
+struct MixCtx {
+  const T *in;  // this thread's line in global memory
+  T *out;
+  C2<T> *ln;    // ... and in LDS
+  int aux;      // index along the line set's auxdim (four-step row / column)
+  int j;        // place in the line
+  bool ok;      // the line exists and the thread has a place in it
+};
+
+template <typename T>
+__device__ __forceinline__ C2<T> swapri(C2<T> a, bool sw) {
+  return sw ? C2<T>{a.y, a.x} : a;
+}
+
+// Complex elements at any scalar-aligned address: a global access of two
+// (or four) dwords needs dword alignment only.
+template <typename T>
+struct __attribute__((packed, aligned(sizeof(T)))) PackedC2 {
+  T x, y;
+};
+template <typename T>
+__device__ __forceinline__ C2<T> gload(const T *p) {
+  const PackedC2<T> v = *reinterpret_cast<const PackedC2<T> *>(p);
+  return C2<T>{v.x, v.y};
+}
+template <typename T>
+__device__ __forceinline__ void gstore(T *p, C2<T> v) {
+  *reinterpret_cast<PackedC2<T> *>(p) = PackedC2<T>{v.x, v.y};
+}
+
+// W_N^e from the half-size tables
+template <typename T>
+__device__ __forceinline__ C2<T> step_twiddle(const LineArgs<T> &a, int k, int aux) {
+  const uint64_t e = uint64_t(unsigned(k)) * uint64_t(unsigned(aux));
+  const unsigned mask = (1u << a.shift) - 1u;
+  return cmul(a.t0[unsigned(e) & mask], a.t1[e >> a.shift]);
+}
+
+// Inputs j + r NR (r < R) of a line, with the op's pre-processing.
+template <typename T, int OP, int R>
+__device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c, int j, int NR,
+                                        C2<T> *v) {
+  const bool cj = (a.sub & SUB_CONJ) != 0;
+  const int64_t es = a.esi;
+  const int op = op_of<OP>(a);
+  if (op == OP_C2C || op == OP_PASSB || op == OP_BLUEROW || op == OP_PASSA) {
+    if (op == OP_PASSA && (a.sub & SUB_CHIRP)) {  // x[m] conj(chirp[m]), zero from m = n on
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int jj = j + r * NR;
+        const int64_t m = int64_t(jj) * a.other + c.aux;
+        v[r] = C2<T>{T(0), T(0)};
+        if (m < a.bign) {
+          const C2<T> w = a.t2[m];
+          v[r] = cmul(gload(c.in + blue_col_offset(jj, m, a.rot_in, a.bign, c.aux, es, a.other)),
+                      cj ? w : conjc(w));
+        }
+      }
+    } else if ((op == OP_C2C || op == OP_PASSA) && a.rot_in) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = gload(c.in + rot_index(j + r * NR, a.rot_in, a.nin) * es);
+    } else {
+      const T *p = c.in + j * es;
+      const int64_t step = NR * es;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = gload(p + r * step);
+    }
+  } else if (op == OP_BLUE) {
+    const int n = int(a.bign);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int jj = j + r * NR;
+      v[r] = C2<T>{T(0), T(0)};
+      if (jj < n) {  // element (j + rot_in) mod n, times the chirp at j
+        const C2<T> w = a.t0[jj];
+        v[r] = cmul(gload(c.in + rot_index(jj, a.rot_in, n) * es), cj ? w : conjc(w));
+      }
+    }
+  } else if (op == OP_R2C_EVEN) {
+    const T *p = c.in + 2 * j * es;
+    const int64_t step = 2 * NR * es;
+    if (es == 1) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = gload(p + r * step);
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = C2<T>{p[r * step], p[r * step + es]};
+    }
+  } else if (op == OP_R2C_ODD) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = C2<T>{c.in[(j + r * NR) * es], T(0)};
+  } else if (op == OP_C2R_EVEN) {
+    const int h = a.f.n;
+    const T *p = c.in + j * es, *pm = c.in + (h - j) * es;
+    const int64_t step = NR * es;
+    C2<T> xm[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      v[r] = gload(p + r * step);
+      xm[r] = gload(pm - r * step);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      C2<T> x = v[r], y = xm[r];
+      const int jj = j + r * NR;
+      if (!cj) y.y = -y.y;  // conj of the mirrored bin (of the conjugated input)
+      else x.y = -x.y;
+      if (jj == 0) x.y = y.y = T(0);
+      const C2<T> A = x + y;
+      const C2<T> B = cmul(x - y, conjc(a.t0[jj]));
+      v[r] = C2<T>{A.x - B.y, A.y + B.x};
+    }
+  } else if constexpr (OP == OP_R2R) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      v[r] = pre_elem<T, int>(a.sub & 0xff, c.in, es, int(a.bign), a.f.n, j + r * NR,
+                              (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_CONJ) != 0,
+                              (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0});
+  } else {  // OP_C2R_ODD
+    const int n = a.f.n;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int jj = j + r * NR;
+      if (jj == 0) {
+        v[r] = C2<T>{c.in[0], T(0)};
+      } else if (2 * jj < n) {
+        v[r] = gload(c.in + jj * es);
+        if (cj) v[r].y = -v[r].y;
+      } else {
+        v[r] = gload(c.in + (n - jj) * es);
+        if (!cj) v[r].y = -v[r].y;
+      }
+    }
+  }
+  if (op != OP_BLUE && op != OP_BLUEROW && op != OP_R2C_EVEN && op != OP_R2C_ODD) {
+    if (a.dir > T(0)) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = C2<T>{v[r].y, v[r].x};
+    }
+  }
+}
+
+// Bins j + r ns (r < R), with the op's post-processing.
+template <typename T, int OP, int R>
+__device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &c, int j, int ns,
+                                         C2<T> *v) {
+  const bool cj = (a.sub & SUB_CONJ) != 0;
+  const int64_t es = a.eso;
+  const int op = op_of<OP>(a);
+  if (is_blue(op) || (op != OP_R2C_ODD && a.dir > T(0))) {  // the inverse transform ran on exchanged parts
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = C2<T>{v[r].y, v[r].x};
+  }
+  T *p = c.out + j * es;
+  const int64_t step = ns * es;
+  if (op == OP_C2C || op == OP_PASSB) {
+    if (a.rot_out) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        gstore(c.out + rot_index(j + r * ns, a.rot_out, a.nout) * es, a.fct * v[r]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) gstore(p + r * step, a.fct * v[r]);
+    }
+  } else if (op == OP_PASSA) {
+    if (a.sub & SUB_FINAL) {  // Bluestein columns, last pass: chirp and fct, m < n
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int k = j + r * ns;
+        const int64_t m = c.aux + int64_t(k) * a.other;
+        if (m < a.bign) {
+          const C2<T> w = a.t0[m];
+          gstore(c.out + blue_col_offset(k, m, a.rot_out, a.bign, c.aux, es, a.other),
+                 a.fct * cmul(v[r], cj ? w : conjc(w)));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        gstore(p + r * step, cmul(v[r], dirw(step_twiddle(a, j + r * ns, c.aux), a.dir)));
+    }
+  } else if (op == OP_BLUEROW) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      gstore(p + r * step, cmul(v[r], conjc(step_twiddle(a, j + r * ns, c.aux))));
+  } else if (op == OP_BLUE) {  // bin k < n, chirped, to (k + rot_out) mod n
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int k = j + r * ns;
+      if (k < a.nout) {
+        const C2<T> w = a.t0[k];
+        gstore(c.out + rot_index(k, a.rot_out, a.nout) * es, a.fct * cmul(v[r], cj ? w : conjc(w)));
+      }
+    }
+  } else if (op == OP_R2C_ODD) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (j + r * ns < a.nout) {
+        if (cj) v[r].y = -v[r].y;
+        gstore(p + r * step, a.fct * v[r]);
+      }
+  } else if (op == OP_C2R_EVEN) {
+    T *q = c.out + 2 * j * es;
+    if (es == 1) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) gstore(q + 2 * r * step, a.fct * v[r]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        q[2 * r * step] = a.fct * v[r].x;
+        q[2 * r * step + es] = a.fct * v[r].y;
+      }
+    }
+  } else if (op == OP_C2R_ODD) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) p[r * step] = a.fct * v[r].x;
+  }
+}
+
+// Bluestein kernel product on bins j + r ns, leaving the parts exchanged for
+// the inverse transform.
+template <typename T, int OP, int R>
+__device__ __forceinline__ void kernel_product(const LineArgs<T> &a, const MixCtx<T> &c, int j,
+                                               int ns, C2<T> *v) {
+  const bool cj = (a.sub & SUB_CONJ) != 0;
+  const int op = op_of<OP>(a);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = j + r * ns;
+    const C2<T> w = op == OP_BLUE ? a.t1[k] : a.t2[c.aux + int64_t(k) * a.other];
+    const C2<T> y = cmul(v[r], cj ? conjc(w) : w);
+    v[r] = C2<T>{y.y, y.x};
+  }
+}
+
+// One forward stage of radix R (first: inputs from global memory; last:
+// outputs to global memory, or for Bluestein on through the kernel product
+// into the first backward stage).
+template <typename T, int OP, int R>
+__device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m,
+                                          const MixStage &st, const MixCtx<T> &c, bool first,
+                                          bool last) {
+  constexpr int QM = kMaxElems<T> / R > 0 ? kMaxElems<T> / R : 1;
+  const int op = op_of<OP>(a);
+  const int NR = st.nr, ns = st.ns;
+  const bool from_lds = !first || OP == OP_R2R || m.flat;
+  const C2<T> *tw = a.tw + st.twoff;
+  C2<T> v[QM][R];
+#pragma unroll
+  for (int q = 0; q < QM; ++q) {
+    const int j = c.j + q * m.T;
+    if (q < st.q && c.ok && j < NR) {
+      if (!from_lds) {
+        op_load<T, OP, R>(a, c, j, NR, v[q]);
+      } else {
+        const int b = fdiv(j, ns, st.invns), k = j - b * ns;
+        const C2<T> *s = c.ln + b * st.pbi + k;
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[q][r] = s[r * st.rs];
+        if (!first) {
+#pragma unroll
+          for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], tw[(r - 1) * ns + k]);
+        }
+      }
+      bfly<R>(v[q]);
+    }
+  }
+  if (elem_store(op) && !is_blue(op) && last && !m.flat) {
+#pragma unroll
+    for (int q = 0; q < QM; ++q) {
+      const int j = c.j + q * m.T;
+      if (q < st.q && c.ok && j < NR) op_store<T, OP, R>(a, c, j, ns, v[q]);
+    }
+    return;
+  }
+  if (is_blue(op)) {
+    if (last) {  // ns == NR: k == j
+#pragma unroll
+      for (int q = 0; q < QM; ++q) {
+        const int j = c.j + q * m.T;
+        if (q < st.q && c.ok && j < NR) {
+          kernel_product<T, OP, R>(a, c, j, ns, v[q]);
+          bfly<R>(v[q]);
+          if (first) {
+            op_store<T, OP, R>(a, c, j, NR, v[q]);
+          } else {
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], tw[(r - 1) * ns + j]);
+          }
+        }
+      }
+      if (first) return;
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < QM; ++q) {
+        const int j = c.j + q * m.T;
+        if (q < st.q && c.ok && j < NR) {
+          C2<T> *d = c.ln + j;
+#pragma unroll
+          for (int r = 0; r < R; ++r) d[r * st.rs] = v[q][r];
+        }
+      }
+      __syncthreads();
+      return;
+    }
+  }
+  if (from_lds) __syncthreads();
+  const bool sw = last && OP == OP_R2R && a.dir > T(0);  // read back in its own order
+#pragma unroll
+  for (int q = 0; q < QM; ++q) {
+    const int j = c.j + q * m.T;
+    if (q < st.q && c.ok && j < NR) {
+      const int b = fdiv(j, ns, st.invns), k = j - b * ns;
+      C2<T> *d = c.ln + b * st.pbo + k;
+#pragma unroll
+      for (int r = 0; r < R; ++r) d[r * ns] = swapri(v[q][r], sw);
+    }
+  }
+  __syncthreads();
+}
+
+// One stage of the Bluestein inverse transform, undone backwards: reads where
+// the forward stage wrote, butterfly, twiddles, writes where it read (the
+// first stage: to global memory).
+template <typename T, int OP, int R>
+__device__ __forceinline__ void mix_unstage(const LineArgs<T> &a, const MixGeom &m,
+                                            const MixStage &st, const MixCtx<T> &c, bool first) {
+  constexpr int QM = kMaxElems<T> / R > 0 ? kMaxElems<T> / R : 1;
+  const int NR = st.nr, ns = st.ns;
+  const C2<T> *tw = a.tw + st.twoff;
+  C2<T> v[QM][R];
+#pragma unroll
+  for (int q = 0; q < QM; ++q) {
+    const int j = c.j + q * m.T;
+    if (q < st.q && c.ok && j < NR) {
+      const int b = fdiv(j, ns, st.invns), k = j - b * ns;
+      const C2<T> *d = c.ln + b * st.pbo + k;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q][r] = d[r * ns];
+      bfly<R>(v[q]);
+      if (first) {
+        op_store<T, OP, R>(a, c, j, NR, v[q]);
+      } else {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], tw[(r - 1) * ns + k]);
+      }
+    }
+  }
+  if (first) return;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < QM; ++q) {
+    const int j = c.j + q * m.T;
+    if (q < st.q && c.ok && j < NR) {
+      const int b = fdiv(j, ns, st.invns), k = j - b * ns;
+      C2<T> *s = c.ln + b * st.pbi + k;
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r * st.rs] = v[q][r];
+    }
+  }
+  __syncthreads();
+}
+
+// The whole line to LDS, in order.
+template <typename T, int OP>
+__device__ __forceinline__ void load_line(const LineArgs<T> &a, const MixGeom &m,
+                                          const MixCtx<T> &c) {
+  if (c.ok)
+    for (int e = c.j; e < a.f.n; e += m.T) {
+      C2<T> v[1];
+      op_load<T, OP, 1>(a, c, e, 0, v);
+      c.ln[e] = v[0];
+    }
+  __syncthreads();
+}
+
+// A stage of a prime radix R above 17: st.q output pairs (kk, R - kk) of one
+// butterfly per thread, accumulated over the symmetric sums of its inputs,
+// which are read (and twiddled) once for all of them.  Unit u = chunk NR +
+// butterfly, so lanes share a chunk and the roots come from LDS as broadcasts.
+template <typename T, int OP>
+__device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixGeom &m,
+                                                const MixStage &st, const MixCtx<T> &c,
+                                                const C2<T> *roots, bool first, bool last) {
+  constexpr int PM = kMaxElems<T> / 2;
+  const int R = st.radix, NR = st.nr, ns = st.ns, H = (R - 1) / 2;
+  const C2<T> *tw = a.tw + st.twoff;
+  if (first && OP != OP_R2R && !m.flat) load_line<T, OP>(a, m, c);  // an input serves several threads
+  const int ch = fdiv(c.j, NR, 1.0f / float(NR)), j = c.j - ch * NR;
+  const int k0 = ch * st.q;  // first pair of the chunk
+  const bool on = c.ok && k0 <= H;
+  const int b = fdiv(j, ns, st.invns), k = j - b * ns;
+  const C2<T> *s = c.ln + b * st.pbi + k;
+  const C2<T> *g = roots + st.genoff;
+  C2<T> x0{T(0), T(0)}, sum{T(0), T(0)}, A[PM], B[PM];
+  if (on) {
+    x0 = sum = s[0];
+    int idx[PM];
+#pragma unroll
+    for (int p = 0; p < PM; ++p) {
+      A[p] = x0;
+      B[p] = C2<T>{T(0), T(0)};
+      idx[p] = 0;
+    }
+    for (int mm = 1; mm <= H; ++mm) {
+      C2<T> xp = s[mm * st.rs], xm = s[(R - mm) * st.rs];
+      if (ns > 1) {
+        xp = cmul(xp, tw[(mm - 1) * ns + k]);
+        xm = cmul(xm, tw[(R - mm - 1) * ns + k]);
+      }
+      const C2<T> t = xp + xm, d = xp - xm;
+      sum = sum + t;
+#pragma unroll
+      for (int p = 0; p < PM; ++p) {
+        if (p < st.q) {
+          idx[p] += k0 + p;
+          if (idx[p] >= R) idx[p] -= R;
+          const C2<T> w = g[idx[p]];
+          A[p] = A[p] + w.x * t;
+          B[p] = B[p] + w.y * d;
+        }
+      }
+    }
+  }
+  // outputs: bin kk and bin R - kk of the butterfly
+  const bool lds = !(elem_store(op_of<OP>(a)) && last && !m.flat);
+  const bool sw = lds && last && OP == OP_R2R && a.dir > T(0);
+  if (lds) __syncthreads();
+  if (on) {
+#pragma unroll
+    for (int p = 0; p < PM; ++p) {
+      const int kk = k0 + p;
+      if (p < st.q && kk <= H) {
+        C2<T> lo = {A[p].x + B[p].y, A[p].y - B[p].x}, hi = {A[p].x - B[p].y, A[p].y + B[p].x};
+        if (kk == 0) lo = sum;
+        if (lds) {
+          C2<T> *d = c.ln + b * st.pbo + k;
+          d[kk * ns] = swapri(lo, sw);
+          if (kk) d[(R - kk) * ns] = swapri(hi, sw);
+        } else {  // last stage: ns == NR, bins j + kk ns
+          op_store<T, OP, 1>(a, c, j + kk * ns, 0, &lo);
+          if (kk) op_store<T, OP, 1>(a, c, j + (R - kk) * ns, 0, &hi);
+        }
+      }
+    }
+  }
+  if (lds) __syncthreads();
+}
+
+#define RFH_MIX_RADICES(X) \
+  X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17)
+
+// The place of thread t in its group: the line it works on and its index in
+// it.  Contiguous lines: a line's threads are adjacent (runs along the line);
+// interleaved lines: adjacent threads take the same place of adjacent lines.
+template <typename T>
+__device__ __forceinline__ MixCtx<T> mix_place(const LineArgs<T> &a, const MixGeom &m,
+                                               int64_t tile, C2<T> *lds, bool lfast) {
+  const int t = threadIdx.x;
+  int l, j;
+  if (lfast) {
+    l = t & (m.L - 1);
+    j = t >> m.log2L;
+  } else {
+    l = fdiv(t, m.T, m.invT);
+    j = t - l * m.T;
+  }
+  MixCtx<T> c;
+  const int64_t b = tile * m.L + l;
+  c.ok = l < m.L && j < m.T && b < a.nlines;
+  const LineOffsets o = c.ok ? line_offsets(b, a.nb, a.bdim, a.bsi, a.bso, a.auxdim)
+                             : LineOffsets{0, 0, 0};
+  c.in = a.in + o.oi;
+  c.out = a.out + o.oo;
+  c.aux = o.aux;
+  c.j = j;
+  c.ln = lds + (c.ok ? l : 0) * m.ld;
+  return c;
+}
+
+// One tile (m.L lines from line tile m.L on) of a line set.  Ends without a
+// barrier: a caller that runs several tiles puts one between them.
+template <typename T, int OP>
+__device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m, int64_t tile,
+                                         unsigned char *smem) {
+  const int op = op_of<OP>(a);
+  C2<T> *lds = reinterpret_cast<C2<T> *>(smem);
+  MixCtx<T> c = mix_place(a, m, tile, lds, a.lfast_in != 0);
+  C2<T> *roots = lds + m.L * m.ld;
+  if (m.ngen) {
+    for (int i = threadIdx.x; i < m.ngen; i += blockDim.x) roots[i] = a.gen[i];
+    __syncthreads();
+  }
+  if (m.nst == 0) {  // lines of one element
+    if (c.ok && c.j == 0) {
+      C2<T> v[1];
+      op_load<T, OP, 1>(a, c, 0, 0, v);
+      if (is_blue(op)) kernel_product<T, OP, 1>(a, c, 0, 0, v);
+      if (elem_store(op)) op_store<T, OP, 1>(a, c, 0, 0, v);
+      else c.ln[0] = swapri(v[0], OP == OP_R2R && a.dir > T(0));
+    }
+    __syncthreads();
+  }
+  if (OP == OP_C2C && m.flat) {
+    const int n = a.f.n, nl = int(min(int64_t(m.L), a.nlines - tile * m.L));
+    const float invn = 1.0f / float(n);
+    const int64_t bs = a.nb ? a.bsi[0] : 0;
+    const T *in = a.in + tile * m.L * bs;
+    for (int e = threadIdx.x; e < nl * n; e += blockDim.x) {
+      const int l = fdiv(e, n, invn), p = e - l * n;
+      lds[l * m.ld + p] = swapri(gload(in + l * bs + 2 * p), a.dir > T(0));
+    }
+    __syncthreads();
+  }
+  // the real-to-real modes' heavier loads stay out of the unrolled stages
+  if (OP == OP_R2R && m.nst) load_line<T, OP>(a, m, c);
+  for (int s = 0; s < m.nst; ++s) {
+    const MixStage &st = m.st[s];
+    const bool first = s == 0, last = s == m.nst - 1;
+    switch (st.radix) {
+#define RFH_CASE(R) \
+  case R: mix_stage<T, OP, R>(a, m, st, c, first, last); break;
+      RFH_MIX_RADICES(RFH_CASE)
+#undef RFH_CASE
+      default:
+        if constexpr (OP != OP_BLUE && OP != OP_BLUEROW)
+          mix_prime_stage<T, OP>(a, m, st, c, roots, first, last);
+        break;
+    }
+    // from the first exchange on, threads take the places of the output side
+    if (first && !last && a.lfast_out != a.lfast_in)
+      c = mix_place(a, m, tile, lds, a.lfast_out != 0);
+  }
+  if (is_blue(op)) {
+    for (int s = m.nst - 2; s >= 0; --s) {
+      const MixStage &st = m.st[s];
+      switch (st.radix) {
+#define RFH_CASE(R) \
+  case R: mix_unstage<T, OP, R>(a, m, st, c, s == 0); break;
+        RFH_MIX_RADICES(RFH_CASE)
+#undef RFH_CASE
+        default: break;
+      }
+    }
+  }
+  if (OP == OP_C2C && m.flat && m.nst) {  // the lines' bins are in LDS, in order
+    const int n = a.f.n, nl = int(min(int64_t(m.L), a.nlines - tile * m.L));
+    const float invn = 1.0f / float(n);
+    const int64_t bs = a.nb ? a.bso[0] : 0;
+    T *out = a.out + tile * m.L * bs;
+    for (int e = threadIdx.x; e < nl * n; e += blockDim.x) {
+      const int l = fdiv(e, n, invn), p = e - l * n;
+      gstore(out + l * bs + 2 * p, a.fct * swapri(lds[l * m.ld + p], a.dir > T(0)));
+    }
+  }
+  if (op == OP_R2C_EVEN) {  // bins k and h - k of the half-length spectrum
+    if (c.ok) {
+      const int h = a.f.n;
+      const bool cj = (a.sub & SUB_CONJ) != 0;
+      for (int k = c.j; k <= h; k += m.T) {
+        C2<T> X;
+        if (k == 0 || k == h) {
+          const C2<T> z = c.ln[0];
+          X = C2<T>{k == 0 ? z.x + z.y : z.x - z.y, T(0)};
+        } else {
+          const C2<T> zk = c.ln[k], zm = conjc(c.ln[h - k]);
+          const C2<T> fe = T(0.5) * (zk + zm);
+          const C2<T> dd = zk - zm;
+          X = fe + cmul(a.t0[k], C2<T>{T(0.5) * dd.y, T(-0.5) * dd.x});
+        }
+        if (cj) X.y = -X.y;
+        gstore(c.out + k * a.eso, a.fct * X);
+      }
+    }
+  }
+  if constexpr (OP == OP_R2R) {
+    if (c.ok) {
+      const C2<T> *ln = c.ln;
+      for (int k = c.j; k < a.nout; k += m.T)
+        c.out[k * a.eso] =
+            a.fct * post_elem<T, int>((a.sub >> 8) & 0xff, [&](int q) { return ln[q]; },
+                                      int(a.bign), k, (a.sub & R2R_ORTHO) != 0,
+                                      (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0});
+    }
+  }
+}
+
+}  // namespace dev
+}  // namespace rfh

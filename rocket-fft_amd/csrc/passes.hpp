@@ -5,7 +5,7 @@
 
 #include <vector>
 
-#include "device.hpp"
+#include "mixline.hpp"
 
 namespace rfh {
 
@@ -47,5 +47,18 @@ PassLaunch describe_real_fused(const RealPlan &rp, RealOp op, const LineSet &g, 
 // Kernel arguments of a pass (lines per group chosen unless ps.lines is set).
 template <typename T>
 dev::LineArgs<T> make_line_args(const PassSpec &ps, const LineSet &g);
+// ... and its geometry on the general line kernel.
+template <typename T>
+MixGeom make_mix_geom(const PassSpec &ps, const dev::LineArgs<T> &a);
+
+// The general line kernel for one operation (lines_*.hip).
+template <typename T>
+void launch_mix_c2c(int op, const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s);
+template <typename T>
+void launch_mix_blue(int op, const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s);
+template <typename T>
+void launch_mix_real(int op, const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s);
+template <typename T>
+void launch_mix_r2r(int op, const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s);
 
 }  // namespace rfh

@@ -6,10 +6,9 @@
 //   :2629-2652) and the FFTPACK-vs-Bluestein decision (:2843-2861,
 //   :2885-2903).  The GPU follows the reference's Bluestein decision and its
 //   Bluestein length n2 = good_size_cmplx(2n-1) (:2765-2767).
-// * The GPU's own radix schedule (radix 16 first, then 8/4/2, then 9 for
-//   each pair of threes, then odd primes), independent of the reference's
-//   FFTPACK order: both compute the same DFT, the schedule only changes
-//   rounding.
+// * The GPU's own radix schedule (gpu_radices: few, even radices of 2 .. 17),
+//   independent of the reference's FFTPACK order: both compute the same DFT,
+//   the schedule only changes rounding.
 // * Twiddle, chirp and Bluestein-kernel tables generated in FP64 on the host
 //   (rounded to FP32 for complex64 plans) and kept resident in HBM for the
 //   life of the process, in a thread-safe cache keyed by (device, length,
@@ -30,6 +29,7 @@
 #include <tuple>
 #include <type_traits>
 
+#include "mixgeom.hpp"
 #include "rfh.hpp"
 
 namespace rfh {
@@ -194,36 +194,7 @@ bool plan_bluestein(uint64_t n, bool real, uint64_t *n2) {
 
 // ------------------------------------------------------------- GPU schedule
 
-std::vector<int> gpu_radices(uint64_t n) {
-  std::vector<int> r;
-  if (n <= 1) return r;
-  int twos = 0;
-  while ((n & 1) == 0) {
-    n >>= 1;
-    ++twos;
-  }
-  while (twos >= 4) {
-    r.push_back(16);
-    twos -= 4;
-  }
-  if (twos == 3) r.push_back(8);
-  if (twos == 2) r.push_back(4);
-  if (twos == 1) r.push_back(2);
-  int threes = 0;
-  while (n % 3 == 0) {
-    n /= 3;
-    ++threes;
-  }
-  for (; threes >= 2; threes -= 2) r.push_back(9);
-  if (threes) r.push_back(3);
-  for (uint64_t d = 5; d * d <= n; d += 2)
-    while (n % d == 0) {
-      r.push_back(int(d));
-      n /= d;
-    }
-  if (n > 1) r.push_back(int(n));
-  return r;
-}
+std::vector<int> gpu_radices(uint64_t n) { return mix_radices(n); }
 
 size_t lds_limit() {
   static size_t lim = [] {
@@ -290,7 +261,7 @@ static void upload_any(DevBuf &b, const std::vector<std::complex<double>> &v, bo
 }
 
 static bool has_fixed_kernel(int r) {
-  return r == 2 || r == 3 || r == 4 || r == 5 || r == 8 || r == 9 || r == 16;
+  return r <= 16 && r != 7 && r != 11 && r != 13;
 }
 
 // ---------------------------------------------------------- plan records
@@ -326,8 +297,7 @@ struct RealRec {
   std::vector<std::complex<double>> rtw;
 };
 
-static void make_direct(DirectRec &d, uint64_t n) {
-  std::vector<int> rad = gpu_radices(n);
+static void make_direct(DirectRec &d, uint64_t n, const std::vector<int> &rad) {
   if (rad.size() > size_t(kMaxStages)) RFH_THROW(3, "too many FFT stages");
   d.desc = FftDesc{};
   d.desc.n = int(n);
@@ -353,8 +323,12 @@ static void make_direct(DirectRec &d, uint64_t n) {
   if (d.gen.empty()) d.gen.push_back({1, 0});
 }
 
+static void make_direct(DirectRec &d, uint64_t n) { make_direct(d, n, gpu_radices(n)); }
+
 static void upload_direct(Direct &d, const DirectRec &r, bool dbl) {
   d.desc = r.desc;
+  for (int s = 0; s < r.desc.nst; ++s)
+    d.pbo[s] = block_pitch(r.desc.st[s].ns * r.desc.st[s].radix, r.desc.st[s].ns, dbl);
   upload_any(d.tw, r.tw, dbl);
   upload_any(d.gen, r.gen, dbl);
 }
@@ -836,6 +810,7 @@ std::mutex g_cache_mu;
 typedef std::tuple<int, uint64_t, bool, size_t, bool> PlanKey;
 std::map<PlanKey, std::shared_ptr<C2CPlan>> g_c2c;
 std::map<PlanKey, std::shared_ptr<RealPlan>> g_real;
+std::map<std::tuple<int, uint64_t, uint64_t, bool>, std::shared_ptr<R2RPlan>> g_r2r;
 std::vector<std::shared_ptr<const void>> g_retired;  // dropped from the maps
 std::string g_plan_dir;              // empty: no disk cache
 uint64_t g_disk_hits = 0, g_disk_writes = 0;
@@ -964,6 +939,31 @@ std::shared_ptr<RealPlan> get_real_plan(uint64_t n, bool dbl, size_t budget) {
   });
 }
 
+std::shared_ptr<R2RPlan> get_r2r_plan(uint64_t n, uint64_t m, bool dbl) {
+  uint64_t bn2 = 0;
+  if (m > direct_max(dbl, 1) || (m > 1 && plan_bluestein(m, false, &bn2))) return nullptr;
+  int dev = 0;
+  HIP_CHECK(hipGetDevice(&dev));
+  const auto key = std::make_tuple(dev, n, m, dbl);
+  {
+    std::lock_guard<std::mutex> lk(g_cache_mu);
+    auto it = g_r2r.find(key);
+    if (it != g_r2r.end()) return it->second;
+  }
+  auto p = std::make_shared<R2RPlan>();
+  p->n = n;
+  p->m = m;
+  p->dbl = dbl;
+  DirectRec d;
+  make_direct(d, m, even_radices(m));
+  upload_direct(p->d, d, dbl);
+  std::vector<std::complex<double>> roots(2 * n + 1);
+  for (uint64_t q = 0; q <= 2 * n; ++q) roots[q] = std::conj(wfwd(q, 8 * n));
+  upload_any(p->roots, roots, dbl);
+  std::lock_guard<std::mutex> lk(g_cache_mu);
+  return g_r2r.emplace(key, p).first->second;
+}
+
 void plan_cache_dir(const std::string &dir, bool clear_memory) {
   std::lock_guard<std::mutex> lk(g_cache_mu);
   g_plan_dir = dir;
@@ -973,8 +973,10 @@ void plan_cache_dir(const std::string &dir, bool clear_memory) {
     // graphs, may still read their device tables
     for (auto &kv : g_c2c) g_retired.push_back(kv.second);
     for (auto &kv : g_real) g_retired.push_back(kv.second);
+    for (auto &kv : g_r2r) g_retired.push_back(kv.second);
     g_c2c.clear();
     g_real.clear();
+    g_r2r.clear();
   }
 }
 

@@ -35,6 +35,7 @@
 #include <tuple>
 
 #include "../../include/rocket_fft_hip.h"
+#include "butterfly.hpp"
 #include "passes.hpp"
 
 namespace rfh {
@@ -68,8 +69,8 @@ __device__ void pre_line(const LineArgs<T> &a, int tile) {
   const int64_t j0 = int64_t(tile) * kPrePostChunk;
   const int64_t j1 = min(j0 + kPrePostChunk, int64_t(a.f.n));
   for (int64_t j = j0 + threadIdx.x; j < j1; j += blockDim.x)
-    t[j] = pre_elem<T>(mode, a.in, a.esi, a.bign, a.f.n, j, false, (a.sub & R2R_CONJ) != 0,
-                       false);
+    t[j] = pre_elem<T, int64_t>(mode, a.in, a.esi, a.bign, a.f.n, j, false,
+                                (a.sub & R2R_CONJ) != 0, false, ComputedRoot<T>{a.bign});
 }
 
 template <typename T>
@@ -92,7 +93,8 @@ __device__ void post_line(const LineArgs<T> &a, int tile) {
     const int64_t k1 = min(k0 + kPrePostChunk, n);
     for (int64_t k = k0 + threadIdx.x; k < k1; k += blockDim.x)
       a.out[k * a.eso] =
-          a.fct * post_elem<T>(mode, [&](int64_t q) { return t[q]; }, n, k, false, false);
+          a.fct * post_elem<T, int64_t>(mode, [&](int64_t q) { return t[q]; }, n, k, false, false,
+                                        ComputedRoot<T>{n});
   }
 }
 

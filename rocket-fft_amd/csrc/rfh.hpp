@@ -86,6 +86,7 @@ struct Direct {
   FftDesc desc{};
   DevBuf tw;   // stage twiddles (complex, plan precision)
   DevBuf gen;  // roots for radices 7, 11, 13 and generic odd primes
+  int pbo[kMaxStages] = {};  // LDS pitch of the blocks each stage writes
 };
 
 enum PlanKind {
@@ -127,6 +128,15 @@ struct RealPlan {
   DevBuf rtw;
 };
 
+// Real-to-real line of n in one LDS pass through a complex FFT of m points:
+// the FFT and the table e^{i pi q / 4n}, q <= 2n, of the DCT / DST factors.
+struct R2RPlan {
+  uint64_t n = 0, m = 0;
+  bool dbl = false;
+  Direct d;
+  DevBuf roots;
+};
+
 // process-wide switch of the specialised power-of-two kernels (fast.hip)
 extern bool g_fast_enabled;
 // whether the specialised kernel has a form for n (power of two) with
@@ -141,6 +151,9 @@ bool fast_interleaved_ok(uint64_t n, bool dbl);
 std::shared_ptr<C2CPlan> get_c2c_plan(uint64_t n, bool dbl, size_t lds_budget = 0,
                                       bool interleaved = false);
 std::shared_ptr<RealPlan> get_real_plan(uint64_t n, bool dbl, size_t lds_budget = 0);
+// ... of a real-to-real line, or null when a complex FFT of m points does not
+// run in one LDS pass (or runs as Bluestein).
+std::shared_ptr<R2RPlan> get_r2r_plan(uint64_t n, uint64_t m, bool dbl);
 // The cached plan of get_c2c_plan's arguments on the current device, or
 // null when none was built yet (never allocates).
 std::shared_ptr<C2CPlan> find_c2c_plan(uint64_t n, bool dbl, size_t lds_budget = 0,
@@ -265,9 +278,8 @@ struct RealPrePost {
   bool conj = false;  // pre: conjugate input spectrum; post: conjugate output
   bool flip = false;  // negate entries 2, 4, 6, ... (FFTPACK sign rule)
 };
-// pre -> FFT of length rr.m -> post in one LDS pass; needs p.kind == kDirect
-// with p.n == rr.m.
-void launch_r2r_fused(const C2CPlan &p, const LineSet &g, PreMode pre, PostMode post,
+// pre -> FFT of length rr.m -> post in one LDS pass (p of rr.n and rr.m).
+void launch_r2r_fused(const R2RPlan &p, const LineSet &g, PreMode pre, PostMode post,
                       const RealPrePost &rr, bool fft_forward, double fct, hipStream_t s);
 void launch_pre(PreMode mode, const RealPrePost &rp, const LineSet &g, bool dbl,
                 void *tmp_complex, hipStream_t s);

@@ -14,7 +14,8 @@ PKG_ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(PKG_ROOT, "csrc")
 BUILD = os.path.join(PKG_ROOT, "_build")
 LIB = os.path.join(HERE, "librocketfft_hip.so")
-SOURCES = ["plan.hip", "kernels.hip", "fast.hip", "mfma.hip", "pass1024.hip", "pipe4096.hip", "ragged.hip",
+SOURCES = ["fast.hip", "fast64.hip", "lines_c2c.hip", "lines_blue.hip", "lines_real.hip", "lines_r2r.hip",
+           "ragged.hip", "plan.hip", "kernels.hip", "mfma.hip", "pass1024.hip", "pipe4096.hip",
            "engine.hip", "lineops.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -22,11 +23,16 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function",
 ]
+# The general line kernel holds every radix in one loop over the stages;
+# hoisting their constants and strides out of it costs hundreds of spilled
+# scalar registers.
+FILE_FLAGS = {s: ["-mllvm", "-disable-machine-licm"]
+              for s in ("lines_c2c.hip", "lines_blue.hip", "lines_real.hip", "lines_r2r.hip")}
 
 
 def _compile(src):
     obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [HIPCC, *FLAGS, *FILE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")
