@@ -222,6 +222,21 @@ struct AxisPlan {
   std::shared_ptr<C2CPlan> plan;
 };
 
+// Contiguous lines beyond the ordinary one-pass limit (two buffers in LDS)
+// whose one buffer still fits run in one pass, one line per workgroup, instead
+// of two or three passes over HBM.  With few of them a workgroup's chain of
+// stages takes as long as the passes, which spread a line over many CUs: us in
+// passes -> in one pass, 3 / 16 / 64 / 256 lines of 4099 complex128 (Bluestein
+// over 8232) 32.9 -> 32.3 / 32.2 -> 32.8 / 42.8 -> 34.1 / 86.9 -> 42.5; 8 /
+// 1000 lines of 6000 complex128 11.9 -> 12.7 / 93 -> 75; 4 / 64 / 4096 lines of
+// 16384 complex64 16.2 -> 16.2 / 18.5 -> 17.6 / 492 -> 354.
+constexpr int64_t kWholeLines = 32;
+
+// LDS budget of the plan for a line set (0: the ordinary one).
+size_t axis_budget(uint64_t n, bool dbl, bool inter, int64_t nlines) {
+  return !inter && nlines >= kWholeLines && whole_line_only(n, dbl) ? whole_line_budget() : 0;
+}
+
 AxisPlan c2c_axis_plan(Ctx &c, const int64_t *shape, int nd, int ax, const int64_t *si,
                        const int64_t *so, const void *in, void *out) {
   const uint64_t n = uint64_t(shape[ax]);
@@ -233,7 +248,7 @@ AxisPlan c2c_axis_plan(Ctx &c, const int64_t *shape, int nd, int ax, const int64
   for (int d = 0; d < r.g.nb; ++d)
     inter = inter || std::llabs(r.g.bsi[d]) < std::llabs(r.g.esi) ||
             std::llabs(r.g.bso[d]) < std::llabs(r.g.eso);
-  r.plan = get_c2c_plan(n, c.dbl, 0, inter);
+  r.plan = get_c2c_plan(n, c.dbl, axis_budget(n, c.dbl, inter, r.g.nlines), inter);
   return r;
 }
 
@@ -258,7 +273,7 @@ void *complex_work(Ctx &c, int64_t nlines, int64_t m) {
 }
 
 void c2c_work(Ctx &c, void *work, int64_t nlines, int64_t m, bool forward) {
-  auto plan = get_c2c_plan(uint64_t(m), c.dbl);
+  auto plan = get_c2c_plan(uint64_t(m), c.dbl, axis_budget(uint64_t(m), c.dbl, false, nlines));
   LineSet g = contiguous_lines(work, nlines, m);
   void *tmp = c.ws->get(kSlotTwoPass, c2c_tmp_bytes(*plan, g));
   launch_c2c(*plan, g, forward ? -1 : +1, 1.0, c.s, tmp);
@@ -806,7 +821,7 @@ void c2c_noalloc(uint64_t ndim, const arystruct_t *ain, arystruct_t *aout, aryst
       inter = inter || std::llabs(g.bsi[d]) < std::llabs(g.esi) ||
               std::llabs(g.bso[d]) < std::llabs(g.eso);
     const uint64_t n = uint64_t(in.shape[a]);
-    auto plan = find_c2c_plan(n, dbl, 0, inter);
+    auto plan = find_c2c_plan(n, dbl, axis_budget(n, dbl, inter, g.nlines), inter);
     if (!plan)
       RFH_THROW(3, "no plan on this GPU yet for length " + std::to_string(n) +
                        (dbl ? " complex128" : " complex64") +

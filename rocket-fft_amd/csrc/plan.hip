@@ -217,6 +217,48 @@ uint64_t direct_max(bool dbl, int lines, size_t budget) {
   return (budget ? budget : lds_dynamic_budget()) / (2 * elem * size_t(lines));
 }
 
+size_t whole_line_budget() { return 2 * lds_limit(); }
+
+// Whether contiguous lines of N run in one LDS pass under a budget: always
+// when two buffers of the line would fit in it, and under whole_line_budget
+// also when the line's one buffer fits the workgroup (its pitches and threads
+// included).
+static bool line_fits(uint64_t N, bool dbl, size_t budget) {
+  const uint64_t lim = direct_max(dbl, 1, budget);
+  if (N > lim) return false;
+  if (N <= std::min(lim, direct_max(dbl, 1))) return true;
+  FftDesc f{};
+  int pbo[kMaxStages] = {};
+  int ns = 1, gen = 0;
+  const std::vector<int> rad = gpu_radices(N);
+  if (rad.size() > size_t(kMixStages)) return false;
+  f.n = int(N);
+  f.nst = int(rad.size());
+  for (int s = 0; s < f.nst; ++s) {
+    if (rad[size_t(s)] > 17) return false;
+    f.st[s] = Stage{rad[size_t(s)], ns, 0, gen};
+    pbo[s] = block_pitch(ns * rad[size_t(s)], ns, dbl);
+    ns *= rad[size_t(s)];
+  }
+  return mix_geometry(f, pbo, dbl, int64_t(1) << 20, false, 0, lds_limit()).L > 0;
+}
+
+bool whole_line_only(uint64_t n, bool dbl) {
+  const uint64_t two = direct_max(dbl, 1);
+  if (2 * n <= two || n > direct_max(dbl, 1, whole_line_budget())) return false;
+  static std::mutex mu;
+  static std::map<std::pair<uint64_t, bool>, bool> known;
+  std::lock_guard<std::mutex> lk(mu);
+  const auto key = std::make_pair(n, dbl);
+  auto it = known.find(key);
+  if (it != known.end()) return it->second;
+  uint64_t N = 0;
+  if (!plan_bluestein(n, false, &N)) N = n;
+  const bool yes = N > two && line_fits(N, dbl, whole_line_budget());
+  known.emplace(key, yes);
+  return yes;
+}
+
 // --------------------------------------------------------------- twiddles
 
 // e^{-2 pi i e / m} in FP64 with exact integer octant reduction.
@@ -382,9 +424,18 @@ static void make_bluestein(PlanRec &p, uint64_t n, uint64_t n2) {
   p.bn2 = n2;
 }
 
+// LDS the groups of adjacent lines of a split may take: a plan under a budget
+// of its own (the batch executor's) keeps its groups small, so that several
+// share a CU, unless only a larger one has a split.
+constexpr size_t kSplitBudget = 65536;
+
 // Two-pass split N = n1 * n2 with both passes in LDS at `lines` lines per
 // group; the most balanced split wins.  0 when none exists.
 static uint64_t pick_split(uint64_t N, bool dbl, int lines, size_t budget) {
+  if (budget > kSplitBudget && budget != lds_dynamic_budget()) {
+    const uint64_t n1 = pick_split(N, dbl, lines, kSplitBudget);
+    if (n1) return n1;
+  }
   const uint64_t lim = direct_max(dbl, lines, budget);
   uint64_t best = 0;
   double bestd = 1e300;
@@ -480,7 +531,9 @@ static void make_multi(PlanRec &p, uint64_t N, uint64_t n1) {
 // Returns n1 (0: keep the reference length).
 static uint64_t pick_blue_pow2(uint64_t n, uint64_t ref_n2, bool dbl, size_t budget,
                                uint64_t *gpu_n2) {
-  const uint64_t lim = direct_max(dbl, two_pass_lines(dbl), budget);
+  const uint64_t lim = direct_max(dbl, two_pass_lines(dbl),
+                                  budget == lds_dynamic_budget() ? budget
+                                                                 : std::min(budget, kSplitBudget));
   const uint64_t need = 2 * n - 2;
   uint64_t best_n1 = 0, best = 0;
   for (uint64_t n1 : {uint64_t(1024), uint64_t(512), uint64_t(256)}) {
@@ -508,7 +561,7 @@ static PlanRec build_c2c_rec(uint64_t n, bool dbl, size_t budget, bool inter) {
   // interleaved lines, a group of adjacent lines wide enough for full row
   // segments (the specialised power-of-two kernel, or `lines` lines)
   auto direct_ok = [&](uint64_t N) {
-    if (!inter) return N <= direct_max(dbl, 1, budget);
+    if (!inter) return line_fits(N, dbl, budget);
     return fast_interleaved_ok(N, dbl) || N <= direct_max(dbl, lines, budget);
   };
   uint64_t bn2 = 0;
@@ -568,7 +621,7 @@ static RealRec build_real_rec(uint64_t n, bool dbl, size_t budget) {
   // complex plan of n/2 with the split twiddle in the pre/post kernels, and
   // odd lengths the complex plan of n.
   const bool blue = m > 1 && plan_bluestein(m, false, &bn2);
-  if (n >= 2 && !blue && m <= direct_max(dbl, 1, budget)) {
+  if (n >= 2 && !blue && line_fits(m, dbl, budget)) {
     p.fused = true;
     make_direct(p.d, m);
     if (n % 2 == 0) {

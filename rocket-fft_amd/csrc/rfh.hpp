@@ -173,6 +173,11 @@ std::vector<int> gpu_radices(uint64_t n);
 // Largest line length that fits the LDS budget (0 = device) with `lines`
 // lines per group.
 uint64_t direct_max(bool dbl, int lines, size_t budget = 0);
+// Budget of plans whose contiguous lines may take a workgroup's whole LDS with
+// their one buffer, and whether lines of n (or their Bluestein length) run in
+// one pass only under it.
+size_t whole_line_budget();
+bool whole_line_only(uint64_t n, bool dbl);
 size_t lds_limit();
 
 // Reference plan facts restated (bit-exact).
