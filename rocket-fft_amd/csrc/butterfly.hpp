@@ -287,18 +287,5 @@ struct Bfly<14> : BflyPfa<7, 2> {};
 template <>
 struct Bfly<15> : BflyPfa<5, 3> {};
 
-template <int R, typename T>
-__device__ __forceinline__ void dft_pfa(C2<T> *v, T dir) {
-  if (dir > T(0)) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = C2<T>{v[r].y, v[r].x};
-  }
-  bfly<R>(v);
-  if (dir > T(0)) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = C2<T>{v[r].y, v[r].x};
-  }
-}
-
 }  // namespace dev
 }  // namespace rfh

@@ -1,6 +1,6 @@
 // device.hpp -- device-side building blocks shared by the line kernels:
-// complex arithmetic, radix butterflies, Stockham stages, the kernel
-// argument block and the load/store helpers.
+// complex arithmetic, power-of-two butterflies, the kernel argument
+// block and the load/store helpers.
 #pragma once
 
 #include "lines.hpp"
@@ -78,45 +78,6 @@ __device__ __forceinline__ void dft2(C2<T> *v) {
 }
 
 template <typename T>
-__device__ __forceinline__ void dft3(C2<T> *v, T dir) {
-  const T s = T(0.866025403784438646763723170752936183);
-  const C2<T> t = v[1] + v[2], d = v[1] - v[2];
-  const C2<T> a = v[0] + T(-0.5) * t;
-  v[0] = v[0] + t;
-  const C2<T> b = rot(s * d, dir);
-  v[1] = a + b;
-  v[2] = a - b;
-}
-
-// Radix 9 as 3 x 3: DFT3 over x[n2], x[n2+3], x[n2+6] for each n2, twiddle
-// W9^(n2 k1), DFT3 over n2; X[k1 + 3 k2].  W9^m = cos(2 pi m/9) + dir i sin(2 pi m/9).
-template <typename T>
-__device__ __forceinline__ void dft9(C2<T> *v, T dir) {
-  const T c1 = T(0.766044443118978035202392650555416674),
-          s1 = T(0.642787609686539326322643409907263433),
-          c2 = T(0.173648177666930348851716626769314796),
-          s2 = T(0.984807753012208059366743024589523014),
-          c4 = T(-0.93969262078590838405410927732473147),
-          s4 = T(0.342020143325668733044099614682259581);
-  C2<T> a[3] = {v[0], v[3], v[6]}, b[3] = {v[1], v[4], v[7]}, c[3] = {v[2], v[5], v[8]};
-  dft3(a, dir);
-  dft3(b, dir);
-  dft3(c, dir);
-  b[1] = cmul(b[1], C2<T>{c1, dir * s1});
-  b[2] = cmul(b[2], C2<T>{c2, dir * s2});
-  c[1] = cmul(c[1], C2<T>{c2, dir * s2});
-  c[2] = cmul(c[2], C2<T>{c4, dir * s4});
-#pragma unroll
-  for (int k1 = 0; k1 < 3; ++k1) {
-    C2<T> t[3] = {a[k1], b[k1], c[k1]};
-    dft3(t, dir);
-    v[k1] = t[0];
-    v[k1 + 3] = t[1];
-    v[k1 + 6] = t[2];
-  }
-}
-
-template <typename T>
 __device__ __forceinline__ void dft4(C2<T> *v, T dir) {
   const C2<T> t0 = v[0] + v[2], t1 = v[0] - v[2], t2 = v[1] + v[3];
   const C2<T> t3 = rot(v[1] - v[3], dir);
@@ -124,22 +85,6 @@ __device__ __forceinline__ void dft4(C2<T> *v, T dir) {
   v[2] = t0 - t2;
   v[1] = t1 + t3;
   v[3] = t1 - t3;
-}
-
-template <typename T>
-__device__ __forceinline__ void dft5(C2<T> *v, T dir) {
-  const T c1 = T(0.309016994374947424102293417182819059);
-  const T c2 = T(-0.809016994374947424102293417182819059);
-  const T s1 = T(0.951056516295153572116439333379382143);
-  const T s2 = T(0.587785252292473129168705954639072769);
-  const C2<T> t1 = v[1] + v[4], t2 = v[2] + v[3], d1 = v[1] - v[4], d2 = v[2] - v[3];
-  const C2<T> a1 = v[0] + c1 * t1 + c2 * t2, a2 = v[0] + c2 * t1 + c1 * t2;
-  const C2<T> b1 = rot(s1 * d1 + s2 * d2, dir), b2 = rot(s2 * d1 - s1 * d2, dir);
-  v[0] = v[0] + t1 + t2;
-  v[1] = a1 + b1;
-  v[4] = a1 - b1;
-  v[2] = a2 + b2;
-  v[3] = a2 - b2;
 }
 
 template <typename T>
@@ -185,146 +130,13 @@ __device__ __forceinline__ void dft16(C2<T> *v, T dir) {
   }
 }
 
-// Odd prime P through symmetric pairs; g[q] = (cos 2 pi q/P, sin 2 pi q/P).
-template <int P, typename T>
-__device__ __forceinline__ void dftp(C2<T> *v, T dir, const C2<T> *__restrict__ g) {
-  constexpr int H = (P - 1) / 2;
-  C2<T> t[H], d[H];
-  const C2<T> x0 = v[0];
-  C2<T> sum = v[0];
-#pragma unroll
-  for (int m = 1; m <= H; ++m) {
-    t[m - 1] = v[m] + v[P - m];
-    d[m - 1] = v[m] - v[P - m];
-    sum = sum + t[m - 1];
-  }
-  v[0] = sum;  // the inputs live on in x0, t and d
-#pragma unroll
-  for (int k = 1; k <= H; ++k) {
-    C2<T> a = x0, b = {T(0), T(0)};
-#pragma unroll
-    for (int m = 1; m <= H; ++m) {
-      const C2<T> w = g[(m * k) % P];
-      a = a + w.x * t[m - 1];
-      b = b + w.y * d[m - 1];
-    }
-    const C2<T> rb = rot(b, dir);
-    v[k] = a + rb;
-    v[P - k] = a - rb;
-  }
-}
-
 template <int R, typename T>
-__device__ void dft_pfa(C2<T> *v, T dir);  // butterfly.hpp
-
-template <int R, typename T>
-__device__ __forceinline__ void dft(C2<T> *v, T dir, const C2<T> *g) {
+__device__ __forceinline__ void dft(C2<T> *v, T dir) {
+  static_assert(R == 2 || R == 4 || R == 8 || R == 16, "power-of-two radices");
   if constexpr (R == 2) dft2(v);
-  else if constexpr (R == 3) dft3(v, dir);
   else if constexpr (R == 4) dft4(v, dir);
-  else if constexpr (R == 5) dft5(v, dir);
   else if constexpr (R == 8) dft8(v, dir);
-  else if constexpr (R == 9) dft9(v, dir);
-  else if constexpr (R == 16) dft16(v, dir);
-  else if constexpr (R == 6 || R == 10 || R == 12 || R == 14 || R == 15) dft_pfa<R>(v, dir);
-  else dftp<R>(v, dir, g);
-}
-
-// ------------------------------------------------------------------ stages
-// Stockham stage (radix R, ns = product of earlier radices): butterfly j of
-// N/R reads src[j + r N/R], multiplies by W_{ns R}^{(j mod ns) r}, and writes
-// dst[(j - k) R + k + r ns] with k = j mod ns.  Output is in natural order
-// after the last stage.
-
-template <int R, typename T>
-__device__ __forceinline__ void stage_fixed(const C2<T> *__restrict__ src,
-                                            C2<T> *__restrict__ dst, int L, int ld, int N,
-                                            int ns, const C2<T> *__restrict__ tw,
-                                            const C2<T> *__restrict__ g, T dir) {
-  const int NR = N / R;
-  const int total = L * NR;
-  const float invNR = 1.0f / float(NR), invns = 1.0f / float(ns);
-  for (int u = threadIdx.x; u < total; u += blockDim.x) {
-    const int l = fdiv(u, NR, invNR);
-    const int j = u - l * NR;
-    const int q = fdiv(j, ns, invns);
-    const int k = j - q * ns;
-    const C2<T> *s = src + l * ld + j;
-    C2<T> *d = dst + l * ld + q * ns * R + k;
-    C2<T> v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = s[r * NR];
-    if (ns > 1) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) v[r] = cmul(v[r], dirw(tw[(r - 1) * ns + k], dir));
-    }
-    dft<R>(v, dir, g);
-#pragma unroll
-    for (int r = 0; r < R; ++r) d[r * ns] = v[r];
-  }
-}
-
-// Any odd radix at run time: inputs are twiddled in place in src, then each
-// output pair (k, R - k) of each butterfly is accumulated straight from LDS by
-// its own thread, from the symmetric sums x_m + x_{R-m} and x_m - x_{R-m}.
-// O(R) work per element, spread over (R + 1) / 2 threads per butterfly so
-// that a line with few butterflies still fills the workgroup; used for
-// primes above 13.
-template <typename T>
-__device__ void stage_generic(C2<T> *__restrict__ src, C2<T> *__restrict__ dst, int L,
-                              int ld, int N, int R, int ns, const C2<T> *__restrict__ tw,
-                              const C2<T> *__restrict__ g, T dir) {
-  const int NR = N / R;
-  const int H = (R - 1) / 2;
-  const float invNR = 1.0f / float(NR), invns = 1.0f / float(ns);
-  if (ns > 1) {  // stage twiddles, in place, one (butterfly, input) pair per item
-    const int tot = L * NR * (R - 1);
-    const float inv = 1.0f / float(L * NR);
-    for (int u = threadIdx.x; u < tot; u += blockDim.x) {
-      const int r1 = fdiv(u, L * NR, inv);  // r - 1
-      const int lj = u - r1 * (L * NR);
-      const int l = fdiv(lj, NR, invNR);
-      const int j = lj - l * NR;
-      const int k = j - fdiv(j, ns, invns) * ns;
-      C2<T> *p = src + l * ld + j + (r1 + 1) * NR;
-      *p = cmul(*p, dirw(tw[r1 * ns + k], dir));
-    }
-    __syncthreads();
-  }
-  // one (butterfly, output pair kk / R - kk) per item, butterflies fastest so
-  // that a wave shares kk and reads the same root g[kk m mod R]
-  const int total = L * NR * (H + 1);
-  const float invH = 1.0f / float(H + 1);
-  for (int u = threadIdx.x; u < total; u += blockDim.x) {
-    const int lk = fdiv(u, NR, invNR);
-    const int j = u - lk * NR;
-    const int l = fdiv(lk, H + 1, invH);
-    const int kk = lk - l * (H + 1);
-    const int q = fdiv(j, ns, invns);
-    const int k = j - q * ns;
-    const C2<T> *s = src + l * ld + j;
-    C2<T> *d = dst + l * ld + q * ns * R + k;
-    const C2<T> x0 = s[0];
-    if (kk == 0) {
-      C2<T> sum = x0;
-      for (int r = 1; r < R; ++r) sum = sum + s[r * NR];
-      d[0] = sum;
-      continue;
-    }
-    C2<T> a = x0, b = {T(0), T(0)};
-    int idx = 0;
-    for (int m = 1; m <= H; ++m) {
-      idx += kk;
-      if (idx >= R) idx -= R;
-      const C2<T> vm = s[m * NR], vp = s[(R - m) * NR];
-      const C2<T> w = g[idx];
-      a = a + w.x * (vm + vp);
-      b = b + w.y * (vm - vp);
-    }
-    const C2<T> rb = rot(b, dir);
-    d[kk * ns] = a + rb;
-    d[(R - kk) * ns] = a - rb;
-  }
+  else dft16(v, dir);
 }
 
 // ----------------------------------------------------------- line kernel
@@ -365,7 +177,7 @@ struct LineArgs {
   int64_t esi, eso;
   const T *in;
   T *out;
-  int L, log2L, ld, nin, nout, lfast_in, lfast_out;
+  int nin, nout, lfast_in, lfast_out;
   int auxdim;    // batch dim whose index is a line's aux (four-step row / column)
   int twlds_lo, twlds_hi;  // pass A of the specialised kernel: four-step twiddle
                            // tables (t0 / t1 entries) copied to LDS; 0 = read globally
@@ -411,26 +223,6 @@ __device__ __forceinline__ void stc(T *p, C2<T> v) {
   else {
     p[0] = v.x;
     p[1] = v.y;
-  }
-}
-
-// visit (l, j) for l < nl, j < cnt; l-fastest when lines interleave in memory
-template <typename F>
-__device__ __forceinline__ void for_tile(int nl, int cnt, int lfast, int log2L, F &&f) {
-  if (lfast) {
-    const int Lm = (1 << log2L) - 1;
-    const int total = cnt << log2L;
-    for (int u = threadIdx.x; u < total; u += blockDim.x) {
-      const int l = u & Lm, j = u >> log2L;
-      if (l < nl) f(l, j);
-    }
-  } else {
-    const int total = nl * cnt;
-    const float inv = 1.0f / float(cnt);
-    for (int u = threadIdx.x; u < total; u += blockDim.x) {
-      const int l = fdiv(u, cnt, inv);
-      f(l, u - l * cnt);
-    }
   }
 }
 
@@ -689,368 +481,6 @@ __device__ __forceinline__ T post_elem(int mode, G &&get, I n, I k, bool ortho, 
       break;
   }
   return r;
-}
-
-// Stage 0 of a line group fed straight from global memory: butterfly u of
-// the group takes inputs j + r NR of line l through `load` (the op's
-// pre-processing), and writes its radix-R outputs to dst (ns = 1: no
-// twiddles, output position j R + r).  Missing lines (l >= nl) get zeros.
-template <int R, typename T, typename Ld>
-__device__ __forceinline__ void stage0_in(Ld &&load, C2<T> *__restrict__ dst, int L, int nl,
-                                          int ld, int N, int lfast, int log2L,
-                                          const C2<T> *__restrict__ g, T dir) {
-  const int NR = N / R;
-  const int total = L * NR;
-  const float invNR = 1.0f / float(NR);
-  for (int u = threadIdx.x; u < total; u += blockDim.x) {
-    int l, j;
-    if (lfast) {
-      l = u & ((1 << log2L) - 1);
-      j = u >> log2L;
-    } else {
-      l = fdiv(u, NR, invNR);
-      j = u - l * NR;
-    }
-    C2<T> v[R];
-    if (l < nl) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) v[r] = load(l, j + r * NR);
-    } else {
-#pragma unroll
-      for (int r = 0; r < R; ++r) v[r] = C2<T>{T(0), T(0)};
-    }
-    dft<R>(v, dir, g);
-    C2<T> *d = dst + l * ld + j * R;
-#pragma unroll
-    for (int r = 0; r < R; ++r) d[r] = v[r];
-  }
-}
-
-// Last stage of a line group written straight to global memory: butterfly
-// j (< ns, NR = ns) of line l reads src[j + r ns], twiddles by W^{j r},
-// and hands natural-order bin j + r ns to `store` (the op's post-processing).
-template <int R, typename T, typename St>
-__device__ __forceinline__ void stage_last_out(St &&store, const C2<T> *__restrict__ src,
-                                               int L, int nl, int ld, int ns, int lfast,
-                                               int log2L, const C2<T> *__restrict__ tw,
-                                               const C2<T> *__restrict__ g, T dir) {
-  const int total = L * ns;
-  const float invns = 1.0f / float(ns);
-  for (int u = threadIdx.x; u < total; u += blockDim.x) {
-    int l, j;
-    if (lfast) {
-      l = u & ((1 << log2L) - 1);
-      j = u >> log2L;
-    } else {
-      l = fdiv(u, ns, invns);
-      j = u - l * ns;
-    }
-    if (l >= nl) continue;
-    const C2<T> *s = src + l * ld + j;
-    C2<T> v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = s[r * ns];
-    if (ns > 1) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) v[r] = cmul(v[r], dirw(tw[(r - 1) * ns + j], dir));
-    }
-    dft<R>(v, dir, g);
-#pragma unroll
-    for (int r = 0; r < R; ++r) store(l, j + r * ns, v[r]);
-  }
-}
-
-// Radices whose first / last stage may be fused with global memory: the
-// hand-written butterflies (the symmetric-pair ones would raise the register
-// count of every line kernel)
-__device__ __forceinline__ bool fusable_radix(int r) {
-  return r == 2 || r == 3 || r == 4 || r == 5 || r == 8 || r == 9 || r == 16;
-}
-
-template <typename T, typename Ld>
-__device__ __forceinline__ void stage0_in_any(int R, Ld &&load, C2<T> *dst, int L, int nl,
-                                              int ld, int N, int lfast, int log2L,
-                                              const C2<T> *g, T dir) {
-  switch (R) {
-    case 2: stage0_in<2>(load, dst, L, nl, ld, N, lfast, log2L, g, dir); break;
-    case 3: stage0_in<3>(load, dst, L, nl, ld, N, lfast, log2L, g, dir); break;
-    case 4: stage0_in<4>(load, dst, L, nl, ld, N, lfast, log2L, g, dir); break;
-    case 5: stage0_in<5>(load, dst, L, nl, ld, N, lfast, log2L, g, dir); break;
-    case 8: stage0_in<8>(load, dst, L, nl, ld, N, lfast, log2L, g, dir); break;
-    case 9: stage0_in<9>(load, dst, L, nl, ld, N, lfast, log2L, g, dir); break;
-    default: stage0_in<16>(load, dst, L, nl, ld, N, lfast, log2L, g, dir); break;
-  }
-}
-
-template <typename T, typename St>
-__device__ __forceinline__ void stage_last_out_any(int R, St &&store, const C2<T> *src, int L,
-                                                   int nl, int ld, int ns, int lfast,
-                                                   int log2L, const C2<T> *tw,
-                                                   const C2<T> *g, T dir) {
-  switch (R) {
-    case 2: stage_last_out<2>(store, src, L, nl, ld, ns, lfast, log2L, tw, g, dir); break;
-    case 3: stage_last_out<3>(store, src, L, nl, ld, ns, lfast, log2L, tw, g, dir); break;
-    case 4: stage_last_out<4>(store, src, L, nl, ld, ns, lfast, log2L, tw, g, dir); break;
-    case 5: stage_last_out<5>(store, src, L, nl, ld, ns, lfast, log2L, tw, g, dir); break;
-    case 8: stage_last_out<8>(store, src, L, nl, ld, ns, lfast, log2L, tw, g, dir); break;
-    case 9: stage_last_out<9>(store, src, L, nl, ld, ns, lfast, log2L, tw, g, dir); break;
-    default: stage_last_out<16>(store, src, L, nl, ld, ns, lfast, log2L, tw, g, dir); break;
-  }
-}
-
-// Stages s0 .. s1-1 of f out of LDS (ping-pong a -> b); returns the buffer
-// holding the result.
-template <typename T>
-__device__ C2<T> *run_stages(const FftDesc &f, int s0, int s1, C2<T> *a, C2<T> *b, int L,
-                             int ld, const C2<T> *__restrict__ tw,
-                             const C2<T> *__restrict__ gen, T dir) {
-  for (int s = s0; s < s1; ++s) {
-    const Stage st = f.st[s];
-    const C2<T> *t = tw + st.twoff;
-    const C2<T> *g = gen + st.genoff;
-    switch (st.radix) {
-      case 2: stage_fixed<2>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 3: stage_fixed<3>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 4: stage_fixed<4>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 5: stage_fixed<5>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 7: stage_fixed<7>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 8: stage_fixed<8>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 9: stage_fixed<9>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 11: stage_fixed<11>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 13: stage_fixed<13>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 17: stage_fixed<17>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 6: stage_fixed<6>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 10: stage_fixed<10>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 12: stage_fixed<12>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 14: stage_fixed<14>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 15: stage_fixed<15>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      case 16: stage_fixed<16>(a, b, L, ld, f.n, st.ns, t, g, dir); break;
-      default: stage_generic(a, b, L, ld, f.n, st.radix, st.ns, t, g, dir); break;
-    }
-    __syncthreads();
-    C2<T> *x = a;
-    a = b;
-    b = x;
-  }
-  return a;
-}
-
-// One tile (a.L lines starting at line tile * a.L) of a line set: load with
-// the op's pre-processing, all Stockham stages out of LDS (two buffers in
-// smem_raw), store with the op's post-processing.  When the first (last)
-// stage has a fixed radix it reads (writes) global memory directly instead
-// of going through LDS; ops whose store needs two bins at once (r2c of even
-// length, the real-to-real modes) and the Bluestein ops keep the LDS store.
-// s_oi / s_oo / s_aux are a.L-entry LDS scratch for the per-line offsets.
-template <typename T, int OP, bool VIN, bool VOUT>
-__device__ __forceinline__ void line_body(const LineArgs<T> &a, int64_t tile,
-                                          unsigned char *smem_raw, int64_t *s_oi,
-                                          int64_t *s_oo, int *s_aux) {
-  C2<T> *bufA = reinterpret_cast<C2<T> *>(smem_raw);
-  C2<T> *bufB = bufA + a.L * a.ld;
-  const int64_t b0 = tile * a.L;
-  const int nl = int(min(int64_t(a.L), a.nlines - b0));
-  // offsets of the group's lines; the slots of missing lines (the last
-  // group of a line set) hold zeros and are never used to address memory
-  for (int l = threadIdx.x; l < a.L; l += blockDim.x) {
-    const LineOffsets o = group_slot(b0, l, a.L, a.nlines, a.nb, a.bdim, a.bsi, a.bso, a.auxdim);
-    s_oi[l] = o.oi;
-    s_oo[l] = o.oo;
-    s_aux[l] = o.aux;
-  }
-  __syncthreads();
-
-  const int ld = a.ld;
-  const bool conjf = (a.sub & SUB_CONJ) != 0;
-  // ---------------------------------------------------- per-element load
-  auto load = [&](int l, int j) -> C2<T> {
-    const T *base = a.in + s_oi[l];
-    C2<T> v;
-    if constexpr (OP == OP_C2C) {
-      v = ldc<VIN>(base + rot_index(j, a.rot_in, a.nin) * a.esi);
-    } else if constexpr (OP == OP_PASSB || OP == OP_BLUEROW) {
-      v = ldc<VIN>(base + j * a.esi);
-    } else if constexpr (OP == OP_PASSA) {
-      if (a.sub & SUB_CHIRP) {
-        const int64_t m = int64_t(j) * a.other + s_aux[l];
-        if (m < a.bign) {
-          const C2<T> c = a.t2[m];
-          v = cmul(ldc<VIN>(base + blue_col_offset(j, m, a.rot_in, a.bign, s_aux[l], a.esi,
-                                                   a.other)),
-                   conjf ? c : conjc(c));
-        } else {
-          v = C2<T>{T(0), T(0)};
-        }
-      } else {
-        v = ldc<VIN>(base + rot_index(j, a.rot_in, a.nin) * a.esi);
-      }
-    } else if constexpr (OP == OP_BLUE) {
-      if (j < a.bign) {  // element (j + rot_in) mod n, times the chirp at j
-        const C2<T> c = a.t0[j];
-        v = cmul(ldc<VIN>(base + rot_index(j, a.rot_in, int(a.bign)) * a.esi),
-                 conjf ? c : conjc(c));
-      } else {
-        v = C2<T>{T(0), T(0)};
-      }
-    } else if constexpr (OP == OP_R2C_EVEN) {
-      if constexpr (VIN)  // contiguous real line: one 2-wide load
-        v = ldc<true>(base + 2 * j);
-      else
-        v = C2<T>{base[2 * j * a.esi], base[(2 * j + 1) * a.esi]};
-    } else if constexpr (OP == OP_R2C_ODD) {
-      v = C2<T>{base[j * a.esi], T(0)};
-    } else if constexpr (OP == OP_C2R_EVEN) {
-      const int h = a.f.n;
-      C2<T> xj = ldc<VIN>(base + j * a.esi), xm = ldc<VIN>(base + (h - j) * a.esi);
-      if (conjf) {
-        xj.y = -xj.y;
-        xm.y = -xm.y;
-      }
-      if (j == 0) {
-        xj.y = T(0);
-        xm.y = T(0);
-      }
-      const C2<T> A = xj + conjc(xm);
-      const C2<T> B = cmul(xj - conjc(xm), conjc(a.t0[j]));
-      v = C2<T>{A.x - B.y, A.y + B.x};
-    } else if constexpr (OP == OP_R2R) {
-      v = C2<T>{T(0), T(0)};
-    } else {  // OP_C2R_ODD
-      const int n = a.f.n;
-      if (j == 0) {
-        v = C2<T>{base[0], T(0)};
-      } else if (2 * j < n) {
-        v = ldc<VIN>(base + j * a.esi);
-        if (conjf) v.y = -v.y;
-      } else {
-        v = ldc<VIN>(base + (n - j) * a.esi);
-        if (!conjf) v.y = -v.y;
-      }
-    }
-    return v;
-  };
-  // -------------------------------------- per-element store (bin k < nout)
-  constexpr bool ELEM_STORE = OP == OP_C2C || OP == OP_PASSA || OP == OP_PASSB ||
-                              OP == OP_R2C_ODD || OP == OP_C2R_EVEN || OP == OP_C2R_ODD;
-  auto store = [&](int l, int k, C2<T> v) {
-    if (k >= a.nout) return;
-    T *base = a.out + s_oo[l];
-    if constexpr (OP == OP_C2C) {
-      stc<VOUT>(base + rot_index(k, a.rot_out, a.nout) * a.eso, a.fct * v);
-    } else if constexpr (OP == OP_PASSA) {
-      if (a.sub & SUB_FINAL) {  // Bluestein columns, last pass: chirp and fct, m < n
-        const int64_t m = s_aux[l] + int64_t(k) * a.other;
-        if (m < a.bign) {
-          const C2<T> c = a.t0[m];
-          stc<VOUT>(base + blue_col_offset(k, m, a.rot_out, a.bign, s_aux[l], a.eso, a.other),
-                    a.fct * cmul(v, conjf ? c : conjc(c)));
-        }
-      } else {
-        const C2<T> w = dirw(big_twiddle(a, int64_t(k) * s_aux[l]), a.dir);
-        stc<VOUT>(base + k * a.eso, cmul(v, w));
-      }
-    } else if constexpr (OP == OP_BLUEROW) {
-      const C2<T> w = dirw(big_twiddle(a, int64_t(k) * s_aux[l]), T(1));
-      stc<VOUT>(base + k * a.eso, cmul(v, w));
-    } else if constexpr (OP == OP_PASSB) {
-      const int64_t m = s_aux[l] + int64_t(k) * a.other;
-      if (a.sub & SUB_KERNEL) {
-        const C2<T> w = a.t1[m];
-        stc<VOUT>(base + k * a.eso, cmul(v, conjf ? conjc(w) : w));
-      } else if (a.sub & SUB_FINAL) {
-        if (m < a.bign) {
-          const C2<T> c = a.t0[m];
-          stc<VOUT>(base + k * a.eso, a.fct * cmul(v, conjf ? c : conjc(c)));
-        }
-      } else {
-        stc<VOUT>(base + rot_index(k, a.rot_out, a.nout) * a.eso, a.fct * v);
-      }
-    } else if constexpr (OP == OP_BLUE) {  // bin k to (k + rot_out) mod n
-      const C2<T> c = a.t0[k];
-      stc<VOUT>(base + rot_index(k, a.rot_out, a.nout) * a.eso,
-                a.fct * cmul(v, conjf ? c : conjc(c)));
-    } else if constexpr (OP == OP_R2C_ODD) {
-      if (conjf) v.y = -v.y;
-      stc<VOUT>(base + k * a.eso, a.fct * v);
-    } else if constexpr (OP == OP_C2R_EVEN) {
-      const C2<T> z = a.fct * v;
-      if constexpr (VOUT) {  // contiguous real line: one 2-wide store
-        stc<true>(base + 2 * k, z);
-      } else {
-        base[2 * k * a.eso] = z.x;
-        base[(2 * k + 1) * a.eso] = z.y;
-      }
-    } else if constexpr (OP == OP_C2R_ODD) {
-      base[k * a.eso] = a.fct * v.x;
-    }
-  };
-
-  // ---------------------------------------------------------- load + FFT
-  const FftDesc &f = a.f;
-  const bool two_ffts = OP == OP_BLUE || OP == OP_BLUEROW;
-  // the real-to-real modes keep their (heavier) loads out of the fused stage
-  const bool fuse_in = OP != OP_R2R && f.nst >= 1 && fusable_radix(f.st[0].radix);
-  // the last stage writes global memory itself when it is not also the
-  // fused first stage and the op stores bin by bin
-  const bool fuse_out = ELEM_STORE && !two_ffts && f.nst >= 2 &&
-                        fusable_radix(f.st[f.nst - 1].radix);
-  C2<T> *res;
-  if (fuse_in) {
-    stage0_in_any(f.st[0].radix, load, bufA, a.L, nl, ld, f.n, a.lfast_in, a.log2L,
-                  a.gen + f.st[0].genoff, a.dir);
-    __syncthreads();
-    res = run_stages<T>(f, 1, fuse_out ? f.nst - 1 : f.nst, bufA, bufB, a.L, ld, a.tw, a.gen,
-                        a.dir);
-  } else {
-    for_tile(nl, a.nin, a.lfast_in, a.log2L,
-             [&](int l, int j) { bufA[l * ld + j] = load(l, j); });
-    __syncthreads();
-    res = run_stages<T>(f, 0, fuse_out ? f.nst - 1 : f.nst, bufA, bufB, a.L, ld, a.tw, a.gen,
-                        a.dir);
-  }
-  if (fuse_out) {
-    const Stage st = f.st[f.nst - 1];
-    stage_last_out_any(st.radix, store, res, a.L, nl, ld, st.ns, a.lfast_out, a.log2L,
-                       a.tw + st.twoff, a.gen + st.genoff, a.dir);
-    return;
-  }
-  if constexpr (OP == OP_BLUE || OP == OP_BLUEROW) {
-    const int n2 = a.f.n;
-    for_tile(nl, n2, 0, a.log2L, [&](int l, int k) {
-      const C2<T> w = OP == OP_BLUE ? a.t1[k] : a.t2[s_aux[l] + int64_t(k) * a.other];
-      res[l * ld + k] = cmul(res[l * ld + k], conjf ? conjc(w) : w);
-    });
-    __syncthreads();
-    res = run_stages<T>(f, 0, f.nst, res, res == bufA ? bufB : bufA, a.L, ld, a.tw, a.gen,
-                        -a.dir);
-  }
-
-  // --------------------------------------------------------------- store
-  for_tile(nl, a.nout, a.lfast_out, a.log2L, [&](int l, int k) {
-    const C2<T> *r = res + l * ld;
-    if constexpr (OP == OP_R2C_EVEN) {
-      T *base = a.out + s_oo[l];
-      const int h = a.f.n;
-      C2<T> X;
-      if (k == 0 || k == h) {
-        const C2<T> z = r[0];
-        X = C2<T>{k == 0 ? z.x + z.y : z.x - z.y, T(0)};
-      } else {
-        const C2<T> zk = r[k], zm = conjc(r[h - k]);
-        const C2<T> fe = T(0.5) * (zk + zm);
-        const C2<T> dd = zk - zm;
-        const C2<T> fo = C2<T>{T(0.5) * dd.y, T(-0.5) * dd.x};  // (zk - zm) / 2i
-        X = fe + cmul(a.t0[k], fo);
-      }
-      if (conjf) X.y = -X.y;
-      stc<VOUT>(base + k * a.eso, a.fct * X);
-    } else if constexpr (OP == OP_R2R) {
-      T *base = a.out + s_oo[l];
-      (void)base;
-    } else {
-      store(l, k, r[k]);
-    }
-  });
 }
 
 }  // namespace dev

@@ -293,7 +293,7 @@ __device__ __forceinline__ void fstage(const FCtx<T> &c) {
 #pragma unroll
         for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], dirw(tw[(r - 1) * NS + k], dir));
       }
-      dft<R>(v[q], dir, a.gen);
+      dft<R>(v[q], dir);
     }
   }
   if constexpr (LAST && DIRECT_OUT && OP == OP_R2C_EVEN) {
@@ -401,7 +401,7 @@ __device__ __forceinline__ void fstage_split(
 #pragma unroll
         for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], dirw(tw[(r - 1) * NS + k], dir));
       }
-      dft<R>(v[q], dir, a.gen);
+      dft<R>(v[q], dir);
     }
   }
   if constexpr (LAST && DIRECT_OUT) {

@@ -36,36 +36,6 @@ thread_local const char *t_last_family = "k_lines";  // kernel family of the las
 
 // ----------------------------------------------------------- host launch
 
-int pow2floor(int64_t v) {
-  int p = 1;
-  while (int64_t(p) * 2 <= v) p *= 2;
-  return p;
-}
-
-int ilog2(int v) {
-  int l = 0;
-  while ((1 << l) < v) ++l;
-  return l;
-}
-
-// lines per group: the largest power of two whose two LDS buffers fit
-// `budget` (and are not wasted on missing lines)
-int choose_lines(int ld, size_t elem, int64_t nlines, bool interleaved) {
-  // interleaved lines want as many adjacent lines as LDS holds (row
-  // segments); contiguous lines leave room for several groups per CU
-  const size_t budget = interleaved ? lds_limit() - kLineStaticLds
-                                    : std::min<size_t>(48 * 1024, lds_limit() - kLineStaticLds);
-  int L = 1;
-  while (L * 2 <= kMaxLinesPerGroup && size_t(2) * (L * 2) * ld * elem <= budget &&
-         int64_t(L) < nlines)
-    L *= 2;
-  // fewer lines per group when the groups would leave CUs idle (down to one
-  // line for contiguous lines, two adjacent lines for interleaved ones)
-  const int floor_l = interleaved ? 2 : 1;
-  while (L > floor_l && nlines < int64_t(L) * 512) L /= 2;
-  return L;
-}
-
 bool lfast_for(int64_t es, const LineSet &g, bool input) {
   if (g.nb == 0) return false;
   const int64_t bs = input ? g.bsi[g.nb - 1] : g.bso[g.nb - 1];
@@ -99,15 +69,10 @@ LineArgs<T> make_line_args(const PassSpec &ps, const LineSet &g) {
   a.in = static_cast<const T *>(g.in);
   a.out = static_cast<T *>(g.out);
   a.f = ps.d->desc;
-  a.ld = a.f.n;
   a.nin = ps.nin;
   a.nout = ps.nout;
   a.lfast_in = lfast_for(g.esi, g, true);
   a.lfast_out = lfast_for(g.eso, g, false);
-  const size_t elem = 2 * sizeof(T);
-  a.L = ps.lines ? ps.lines
-                 : choose_lines(a.ld, elem, g.nlines, a.lfast_in || a.lfast_out);
-  a.log2L = ilog2(a.L);
   a.tw = static_cast<const C2<T> *>(ps.d->tw.p);
   a.gen = static_cast<const C2<T> *>(ps.d->gen.p);
   a.dir = T(ps.dir);

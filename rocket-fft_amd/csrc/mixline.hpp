@@ -42,7 +42,11 @@ template <typename T>
 constexpr int kMixThreads = mix_max_threads(sizeof(T) == 8);
 
 // OP of a kernel that runs every operation but the real-to-real ones, by
-// LineArgs::op (the batch executor's)
+// LineArgs::op (the batch executor's).  Lines are loaded to LDS and stored from
+// LDS by one loop per operation, and the stages exist once per radix: with each
+// operation's loads and stores unrolled into each radix, as in k_lines, the
+// kernel took 1.9 MB of code and 400 s to compile, at the same speed (1447 and
+// 1452 us on the 4096-job batch; 188 KB and 19 s this way).
 constexpr int OP_ANY = -1;
 template <int OP, typename T>
 __device__ __forceinline__ int op_of(const LineArgs<T> &a) {
@@ -91,59 +95,72 @@ __device__ __forceinline__ C2<T> step_twiddle(const LineArgs<T> &a, int k, int a
   return cmul(a.t0[unsigned(e) & mask], a.t1[e >> a.shift]);
 }
 
-// Inputs j + r NR (r < R) of a line, with the op's pre-processing.
-template <typename T, int OP, int R>
+// Inputs j + r NR (r < R) of a line, with the op's pre-processing.  CLAMP:
+// beyond the line its last element instead.
+template <typename T, int OP, int R, bool CLAMP = false>
 __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c, int j, int NR,
                                         C2<T> *v) {
   const bool cj = (a.sub & SUB_CONJ) != 0;
   const int64_t es = a.esi;
   const int op = op_of<OP>(a);
+  auto at = [&](int r) { return CLAMP ? min(j + r * NR, a.f.n - 1) : j + r * NR; };
   if (op == OP_C2C || op == OP_PASSB || op == OP_BLUEROW || op == OP_PASSA) {
     if (op == OP_PASSA && (a.sub & SUB_CHIRP)) {  // x[m] conj(chirp[m]), zero from m = n on
+      // (loads without a condition around them, so that all are in flight)
+      C2<T> w[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int jj = j + r * NR;
-        const int64_t m = int64_t(jj) * a.other + c.aux;
-        v[r] = C2<T>{T(0), T(0)};
-        if (m < a.bign) {
-          const C2<T> w = a.t2[m];
-          v[r] = cmul(gload(c.in + blue_col_offset(jj, m, a.rot_in, a.bign, c.aux, es, a.other)),
-                      cj ? w : conjc(w));
-        }
+        const int64_t m = int64_t(at(r)) * a.other + c.aux;
+        const int jj = m < a.bign ? at(r) : 0;
+        const int64_t mc = m < a.bign ? m : c.aux;
+        w[r] = a.t2[mc];
+        v[r] = gload(c.in + blue_col_offset(jj, mc, a.rot_in, a.bign, c.aux, es, a.other));
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const bool on = int64_t(at(r)) * a.other + c.aux < a.bign;
+        const C2<T> y = cmul(v[r], cj ? w[r] : conjc(w[r]));
+        v[r] = on ? y : C2<T>{T(0), T(0)};
       }
     } else if ((op == OP_C2C || op == OP_PASSA) && a.rot_in) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[r] = gload(c.in + rot_index(j + r * NR, a.rot_in, a.nin) * es);
+      for (int r = 0; r < R; ++r) v[r] = gload(c.in + rot_index(at(r), a.rot_in, a.nin) * es);
     } else {
       const T *p = c.in + j * es;
       const int64_t step = NR * es;
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[r] = gload(p + r * step);
+      for (int r = 0; r < R; ++r) v[r] = gload(CLAMP ? c.in + at(r) * es : p + r * step);
     }
   } else if (op == OP_BLUE) {
     const int n = int(a.bign);
+    C2<T> w[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {  // element (j + rot_in) mod n, times the chirp at j
+      const int jj = at(r) < n ? at(r) : 0;
+      w[r] = a.t0[jj];
+      v[r] = gload(c.in + rot_index(jj, a.rot_in, n) * es);
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int jj = j + r * NR;
-      v[r] = C2<T>{T(0), T(0)};
-      if (jj < n) {  // element (j + rot_in) mod n, times the chirp at j
-        const C2<T> w = a.t0[jj];
-        v[r] = cmul(gload(c.in + rot_index(jj, a.rot_in, n) * es), cj ? w : conjc(w));
-      }
+      const C2<T> y = cmul(v[r], cj ? w[r] : conjc(w[r]));
+      v[r] = at(r) < n ? y : C2<T>{T(0), T(0)};
     }
   } else if (op == OP_R2C_EVEN) {
     const T *p = c.in + 2 * j * es;
     const int64_t step = 2 * NR * es;
     if (es == 1) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[r] = gload(p + r * step);
+      for (int r = 0; r < R; ++r) v[r] = gload(CLAMP ? c.in + 2 * at(r) * es : p + r * step);
     } else {
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[r] = C2<T>{p[r * step], p[r * step + es]};
+      for (int r = 0; r < R; ++r) {
+        const T *q = CLAMP ? c.in + 2 * at(r) * es : p + r * step;
+        v[r] = C2<T>{q[0], q[es]};
+      }
     }
   } else if (op == OP_R2C_ODD) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = C2<T>{c.in[(j + r * NR) * es], T(0)};
+    for (int r = 0; r < R; ++r) v[r] = C2<T>{c.in[at(r) * es], T(0)};
   } else if (op == OP_C2R_EVEN) {
     const int h = a.f.n;
     const T *p = c.in + j * es, *pm = c.in + (h - j) * es;
@@ -151,13 +168,13 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
     C2<T> xm[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      v[r] = gload(p + r * step);
-      xm[r] = gload(pm - r * step);
+      v[r] = gload(CLAMP ? c.in + at(r) * es : p + r * step);
+      xm[r] = gload(CLAMP ? c.in + (h - at(r)) * es : pm - r * step);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       C2<T> x = v[r], y = xm[r];
-      const int jj = j + r * NR;
+      const int jj = at(r);
       if (!cj) y.y = -y.y;  // conj of the mirrored bin (of the conjugated input)
       else x.y = -x.y;
       if (jj == 0) x.y = y.y = T(0);
@@ -168,14 +185,14 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
   } else if constexpr (OP == OP_R2R) {
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      v[r] = pre_elem<T, int>(a.sub & 0xff, c.in, es, int(a.bign), a.f.n, j + r * NR,
+      v[r] = pre_elem<T, int>(a.sub & 0xff, c.in, es, int(a.bign), a.f.n, at(r),
                               (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_CONJ) != 0,
                               (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0});
   } else {  // OP_C2R_ODD
     const int n = a.f.n;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int jj = j + r * NR;
+      const int jj = at(r);
       if (jj == 0) {
         v[r] = C2<T>{c.in[0], T(0)};
       } else if (2 * jj < n) {
@@ -195,13 +212,15 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
   }
 }
 
-// Bins j + r ns (r < R), with the op's post-processing.
-template <typename T, int OP, int R>
+// Bins j + r ns (r < R), with the op's post-processing.  CLAMP: those beyond
+// the line are left out.
+template <typename T, int OP, int R, bool CLAMP = false>
 __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &c, int j, int ns,
                                          C2<T> *v) {
   const bool cj = (a.sub & SUB_CONJ) != 0;
   const int64_t es = a.eso;
   const int op = op_of<OP>(a);
+  auto in_line = [&](int r) { return !CLAMP || j + r * ns < a.f.n; };
   if (is_blue(op) || (op != OP_R2C_ODD && a.dir > T(0))) {  // the inverse transform ran on exchanged parts
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = C2<T>{v[r].y, v[r].x};
@@ -212,45 +231,61 @@ __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &
     if (a.rot_out) {
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        gstore(c.out + rot_index(j + r * ns, a.rot_out, a.nout) * es, a.fct * v[r]);
+        if (in_line(r))
+          gstore(c.out + rot_index(j + r * ns, a.rot_out, a.nout) * es, a.fct * v[r]);
     } else {
 #pragma unroll
-      for (int r = 0; r < R; ++r) gstore(p + r * step, a.fct * v[r]);
+      for (int r = 0; r < R; ++r)
+        if (in_line(r)) gstore(p + r * step, a.fct * v[r]);
     }
   } else if (op == OP_PASSA) {
+    // the factors of all bins first, without a condition around their loads
+    C2<T> w[R];
     if (a.sub & SUB_FINAL) {  // Bluestein columns, last pass: chirp and fct, m < n
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int64_t m = c.aux + int64_t(j + r * ns) * a.other;
+        w[r] = a.t0[m < a.bign ? m : c.aux];
+      }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int k = j + r * ns;
         const int64_t m = c.aux + int64_t(k) * a.other;
-        if (m < a.bign) {
-          const C2<T> w = a.t0[m];
+        if (in_line(r) && m < a.bign)
           gstore(c.out + blue_col_offset(k, m, a.rot_out, a.bign, c.aux, es, a.other),
-                 a.fct * cmul(v[r], cj ? w : conjc(w)));
-        }
+                 a.fct * cmul(v[r], cj ? w[r] : conjc(w[r])));
       }
     } else {
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        gstore(p + r * step, cmul(v[r], dirw(step_twiddle(a, j + r * ns, c.aux), a.dir)));
+        w[r] = step_twiddle(a, CLAMP ? min(j + r * ns, a.f.n - 1) : j + r * ns, c.aux);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (in_line(r)) gstore(p + r * step, cmul(v[r], dirw(w[r], a.dir)));
     }
   } else if (op == OP_BLUEROW) {
+    C2<T> w[R];
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      gstore(p + r * step, cmul(v[r], conjc(step_twiddle(a, j + r * ns, c.aux))));
+      w[r] = step_twiddle(a, CLAMP ? min(j + r * ns, a.f.n - 1) : j + r * ns, c.aux);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (in_line(r)) gstore(p + r * step, cmul(v[r], conjc(w[r])));
   } else if (op == OP_BLUE) {  // bin k < n, chirped, to (k + rot_out) mod n
+    C2<T> w[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[r] = a.t0[j + r * ns < a.nout ? j + r * ns : 0];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int k = j + r * ns;
-      if (k < a.nout) {
-        const C2<T> w = a.t0[k];
-        gstore(c.out + rot_index(k, a.rot_out, a.nout) * es, a.fct * cmul(v[r], cj ? w : conjc(w)));
-      }
+      if (in_line(r) && k < a.nout)
+        gstore(c.out + rot_index(k, a.rot_out, a.nout) * es,
+               a.fct * cmul(v[r], cj ? w[r] : conjc(w[r])));
     }
   } else if (op == OP_R2C_ODD) {
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      if (j + r * ns < a.nout) {
+      if (in_line(r) && j + r * ns < a.nout) {
         if (cj) v[r].y = -v[r].y;
         gstore(p + r * step, a.fct * v[r]);
       }
@@ -258,17 +293,20 @@ __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &
     T *q = c.out + 2 * j * es;
     if (es == 1) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) gstore(q + 2 * r * step, a.fct * v[r]);
+      for (int r = 0; r < R; ++r)
+        if (in_line(r)) gstore(q + 2 * r * step, a.fct * v[r]);
     } else {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        q[2 * r * step] = a.fct * v[r].x;
-        q[2 * r * step + es] = a.fct * v[r].y;
-      }
+      for (int r = 0; r < R; ++r)
+        if (in_line(r)) {
+          q[2 * r * step] = a.fct * v[r].x;
+          q[2 * r * step + es] = a.fct * v[r].y;
+        }
     }
   } else if (op == OP_C2R_ODD) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) p[r * step] = a.fct * v[r].x;
+    for (int r = 0; r < R; ++r)
+      if (in_line(r)) p[r * step] = a.fct * v[r].x;
   }
 }
 
@@ -277,13 +315,15 @@ __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &
 template <typename T, int OP, int R>
 __device__ __forceinline__ void kernel_product(const LineArgs<T> &a, const MixCtx<T> &c, int j,
                                                int ns, C2<T> *v) {
-  const bool cj = (a.sub & SUB_CONJ) != 0;
-  const int op = op_of<OP>(a);
+  const T cs = (a.sub & SUB_CONJ) != 0 ? T(-1) : T(1);
+  const bool row = op_of<OP>(a) == OP_BLUEROW;
+  const C2<T> *kp = row ? a.t2 + c.aux : a.t1;
+  const int64_t ks = row ? a.other : 1;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int k = j + r * ns;
-    const C2<T> w = op == OP_BLUE ? a.t1[k] : a.t2[c.aux + int64_t(k) * a.other];
-    const C2<T> y = cmul(v[r], cj ? conjc(w) : w);
+    C2<T> w = kp[(j + r * ns) * ks];
+    w.y *= cs;
+    const C2<T> y = cmul(v[r], w);
     v[r] = C2<T>{y.y, y.x};
   }
 }
@@ -298,16 +338,20 @@ __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m
   constexpr int QM = kMaxElems<T> / R > 0 ? kMaxElems<T> / R : 1;
   const int op = op_of<OP>(a);
   const int NR = st.nr, ns = st.ns;
-  const bool from_lds = !first || OP == OP_R2R || m.flat;
+  const bool from_lds = !first || OP == OP_R2R || OP == OP_ANY || m.flat;
   const C2<T> *tw = a.tw + st.twoff;
   C2<T> v[QM][R];
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
     const int j = c.j + q * m.T;
     if (q < st.q && c.ok && j < NR) {
-      if (!from_lds) {
-        op_load<T, OP, R>(a, c, j, NR, v[q]);
-      } else {
+      bool loaded = false;
+      if constexpr (OP != OP_ANY)
+        if (!from_lds) {
+          op_load<T, OP, R>(a, c, j, NR, v[q]);
+          loaded = true;
+        }
+      if (!loaded) {
         const int b = fdiv(j, ns, st.invns), k = j - b * ns;
         const C2<T> *s = c.ln + b * st.pbi + k;
 #pragma unroll
@@ -320,13 +364,15 @@ __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m
       bfly<R>(v[q]);
     }
   }
-  if (elem_store(op) && !is_blue(op) && last && !m.flat) {
+  if constexpr (OP != OP_ANY) {
+    if (elem_store(op) && !is_blue(op) && last && !m.flat) {
 #pragma unroll
-    for (int q = 0; q < QM; ++q) {
-      const int j = c.j + q * m.T;
-      if (q < st.q && c.ok && j < NR) op_store<T, OP, R>(a, c, j, ns, v[q]);
+      for (int q = 0; q < QM; ++q) {
+        const int j = c.j + q * m.T;
+        if (q < st.q && c.ok && j < NR) op_store<T, OP, R>(a, c, j, ns, v[q]);
+      }
+      return;
     }
-    return;
   }
   if (is_blue(op)) {
     if (last) {  // ns == NR: k == j
@@ -336,15 +382,15 @@ __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m
         if (q < st.q && c.ok && j < NR) {
           kernel_product<T, OP, R>(a, c, j, ns, v[q]);
           bfly<R>(v[q]);
-          if (first) {
-            op_store<T, OP, R>(a, c, j, NR, v[q]);
-          } else {
+          if (!first) {
 #pragma unroll
             for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], tw[(r - 1) * ns + j]);
+          } else if constexpr (OP != OP_ANY) {
+            op_store<T, OP, R>(a, c, j, NR, v[q]);
           }
         }
       }
-      if (first) return;
+      if (first && OP != OP_ANY) return;
       __syncthreads();
 #pragma unroll
       for (int q = 0; q < QM; ++q) {
@@ -393,15 +439,15 @@ __device__ __forceinline__ void mix_unstage(const LineArgs<T> &a, const MixGeom 
 #pragma unroll
       for (int r = 0; r < R; ++r) v[q][r] = d[r * ns];
       bfly<R>(v[q]);
-      if (first) {
-        op_store<T, OP, R>(a, c, j, NR, v[q]);
-      } else {
+      if (!first) {
 #pragma unroll
         for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], tw[(r - 1) * ns + k]);
+      } else if constexpr (OP != OP_ANY) {
+        op_store<T, OP, R>(a, c, j, NR, v[q]);
       }
     }
   }
-  if (first) return;
+  if (first && OP != OP_ANY) return;
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
@@ -416,17 +462,35 @@ __device__ __forceinline__ void mix_unstage(const LineArgs<T> &a, const MixGeom 
   __syncthreads();
 }
 
-// The whole line to LDS, in order.
+// The whole line to LDS, in order (with the batch executor's operations
+// kLineBatch loads of a thread in flight).
+constexpr int kLineBatch = 8;
 template <typename T, int OP>
 __device__ __forceinline__ void load_line(const LineArgs<T> &a, const MixGeom &m,
                                           const MixCtx<T> &c) {
+  constexpr int U = OP == OP_ANY ? kLineBatch : 1;
   if (c.ok)
-    for (int e = c.j; e < a.f.n; e += m.T) {
-      C2<T> v[1];
-      op_load<T, OP, 1>(a, c, e, 0, v);
-      c.ln[e] = v[0];
+    for (int e = c.j; e < a.f.n; e += U * m.T) {
+      C2<T> v[U];
+      op_load<T, OP, U, (U > 1)>(a, c, e, m.T, v);
+#pragma unroll
+      for (int r = 0; r < U; ++r)
+        if (e + r * m.T < a.f.n) c.ln[e + r * m.T] = v[r];
     }
   __syncthreads();
+}
+
+// ... and from LDS.
+template <typename T, int OP>
+__device__ __forceinline__ void store_line(const LineArgs<T> &a, const MixGeom &m,
+                                           const MixCtx<T> &c) {
+  if (c.ok)
+    for (int e = c.j; e < a.f.n; e += kLineBatch * m.T) {
+      C2<T> v[kLineBatch];
+#pragma unroll
+      for (int r = 0; r < kLineBatch; ++r) v[r] = c.ln[min(e + r * m.T, a.f.n - 1)];
+      op_store<T, OP, kLineBatch, true>(a, c, e, m.T, v);
+    }
 }
 
 // A stage of a prime radix R above 17: st.q output pairs (kk, R - kk) of one
@@ -440,7 +504,7 @@ __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixG
   constexpr int PM = kMaxElems<T> / 2;
   const int R = st.radix, NR = st.nr, ns = st.ns, H = (R - 1) / 2;
   const C2<T> *tw = a.tw + st.twoff;
-  if (first && OP != OP_R2R && !m.flat) load_line<T, OP>(a, m, c);  // an input serves several threads
+  if (first && OP != OP_R2R && OP != OP_ANY && !m.flat) load_line<T, OP>(a, m, c);  // an input serves several threads
   const int ch = fdiv(c.j, NR, 1.0f / float(NR)), j = c.j - ch * NR;
   const int k0 = ch * st.q;  // first pair of the chunk
   const bool on = c.ok && k0 <= H;
@@ -478,7 +542,7 @@ __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixG
     }
   }
   // outputs: bin kk and bin R - kk of the butterfly
-  const bool lds = !(elem_store(op_of<OP>(a)) && last && !m.flat);
+  const bool lds = OP == OP_ANY || !(elem_store(op_of<OP>(a)) && last && !m.flat);
   const bool sw = lds && last && OP == OP_R2R && a.dir > T(0);
   if (lds) __syncthreads();
   if (on) {
@@ -492,7 +556,7 @@ __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixG
           C2<T> *d = c.ln + b * st.pbo + k;
           d[kk * ns] = swapri(lo, sw);
           if (kk) d[(R - kk) * ns] = swapri(hi, sw);
-        } else {  // last stage: ns == NR, bins j + kk ns
+        } else if constexpr (OP != OP_ANY) {  // last stage: ns == NR, bins j + kk ns
           op_store<T, OP, 1>(a, c, j + kk * ns, 0, &lo);
           if (kk) op_store<T, OP, 1>(a, c, j + (R - kk) * ns, 0, &hi);
         }
@@ -568,7 +632,7 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
     __syncthreads();
   }
   // the real-to-real modes' heavier loads stay out of the unrolled stages
-  if (OP == OP_R2R && m.nst) load_line<T, OP>(a, m, c);
+  if ((OP == OP_R2R || OP == OP_ANY) && m.nst) load_line<T, OP>(a, m, c);
   for (int s = 0; s < m.nst; ++s) {
     const MixStage &st = m.st[s];
     const bool first = s == 0, last = s == m.nst - 1;
@@ -608,6 +672,8 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
       gstore(out + l * bs + 2 * p, a.fct * swapri(lds[l * m.ld + p], a.dir > T(0)));
     }
   }
+  if constexpr (OP == OP_ANY)
+    if (m.nst && elem_store(op)) store_line<T, OP>(a, m, c);
   if (op == OP_R2C_EVEN) {  // bins k and h - k of the half-length spectrum
     if (c.ok) {
       const int h = a.f.n;

@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(1024, 1)
     // 64 (i0 / 4): stage 1's input i0 / 4 of its butterfly 16 (i0 mod 4) + r,
     // whose twiddle W_256^((i0 / 4) r) is applied here, while no prefetch
     // holds registers
-    dft<16>(v, dir, static_cast<const C2<float> *>(nullptr));
+    dft<16>(v, dir);
     {
       C2<float> *ln = lds + l0 * kP;
       const C2<float> *tw = st1l + (i0 >> 2) * 16 + z;  // row 0: ones
@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(1024, 1)
       C2<float> *ln = lds + l0 * kP;
 #pragma unroll
       for (int r = 0; r < 16; ++r) w[r] = ln[pad(i0 + 64 * r)];  // twiddled in stage 0
-      dft<16>(w, dir, static_cast<const C2<float> *>(nullptr));
+      dft<16>(w, dir);
 #pragma unroll
       for (int r = 0; r < 16; ++r) ln[pad(i0 + 64 * r)] = w[r];
     }

@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(1024, 1)
     // butterfly i lands at 16 i + r = (16 (i mod 16) + r) + 256 (i / 16):
     // stage 1's input i / 16 of its butterfly 16 (i mod 16) + r, whose
     // twiddle W_256^((i / 16) r) is applied here
-    dft<16>(v, dir, static_cast<const C2<float> *>(nullptr));
+    dft<16>(v, dir);
     {
       const C2<float> *tw = st1l + (i >> 4) * 16 + z;  // row 0: ones
       ln[pad(i * 16)] = v[0];
@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(1024, 1)
       C2<float> w[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) w[r] = ln[pad(i + kT * r)];  // twiddled in stage 0
-      dft<16>(w, dir, static_cast<const C2<float> *>(nullptr));
+      dft<16>(w, dir);
       const C2<float> *tw = st1l + (i >> 4) * 16 + z;  // row 0: ones
       ln[pad(i)] = cmul(w[0], aj);
 #pragma unroll
@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(1024, 1)
       C2<float> u[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) u[r] = ln[pad(16 * r + (i & 15) + kT * (i >> 4))];
-      dft<16>(u, dir, static_cast<const C2<float> *>(nullptr));
+      dft<16>(u, dir);
       const uint32_t vo = uint32_t(s_oo[s][l]) * 4u;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {

@@ -209,7 +209,6 @@ size_t lds_limit() {
   return lim;
 }
 
-// Static LDS of the line kernels (per-line offsets) is reserved first.
 static size_t lds_dynamic_budget() { return lds_limit() - kLineStaticLds; }
 
 uint64_t direct_max(bool dbl, int lines, size_t budget) {
@@ -302,10 +301,6 @@ static void upload_any(DevBuf &b, const std::vector<std::complex<double>> &v, bo
     upload_cplx<float>(b, v);
 }
 
-static bool has_fixed_kernel(int r) {
-  return r <= 16 && r != 7 && r != 11 && r != 13;
-}
-
 // ---------------------------------------------------------- plan records
 // A plan is decided and its tables generated on the host (FP64) into a
 // record; the device plan is built from the record.  Records are what the
@@ -357,7 +352,7 @@ static void make_direct(DirectRec &d, uint64_t n, const std::vector<int> &rad) {
     if (ns > 1)
       for (int r = 1; r < R; ++r)
         for (int k = 0; k < ns; ++k) d.tw.push_back(wfwd(uint64_t(k) * r, uint64_t(ns) * R));
-    if (!has_fixed_kernel(R))
+    if (R > 17)  // the smaller ones are compile-time butterflies
       for (int q = 0; q < R; ++q) d.gen.push_back(std::conj(wfwd(q, R)));  // (cos, +sin)
     ns *= R;
   }

@@ -1,20 +1,20 @@
 // ragged.hip -- many independent transforms of uneven lengths and kinds
-// (complex c2c, real r2c / c2r) in persistent launches.
+// (complex c2c, real r2c / c2r) in a few launches.
 //
 // A batch is planned once (rfh_batch_create): every job gets the passes the
 // per-call engine would run for it (direct LDS line, Bluestein in LDS, the
 // four-step passes, or pre -> c2c -> post for real lengths without a fused
 // plan), all sized to one LDS budget, with its temporaries carved out of one
-// arena.  The passes are cut into work units (a run of tiles of one pass)
-// and grouped by level: level k holds the k-th pass of every job that has
-// one, so a unit depends only on units of earlier levels.  Execution is one
-// fill kernel that zeroes the levels' unit counters, then one persistent
-// launch per level (a job has at most a handful of passes): resident
-// workgroups pull units from that level's counter, largest job first, and
-// run their tiles.  Kernel boundaries order the levels, so no workgroup ever
-// waits on another and a large job's tiles spread over many CUs.  The LDS
-// budget and the grid size are picked by a small autotuner that times the
-// candidates on scratch copies of the batch's buffers.
+// arena.  The passes are cut into tiles (a group of lines each), one workgroup
+// per tile on the general line body (mixline.hpp), and grouped by level: level
+// k holds the k-th pass of every job that has one, so a tile depends only on
+// tiles of earlier levels.  A level runs as one launch per workgroup size (64
+// to 1024 threads), the largest passes first: the hardware hands the next tile
+// to whichever CU has room, a long line takes a whole CU's LDS and a short one
+// a wave.  Kernel boundaries order the levels, so no workgroup ever waits on
+// another and a large job's tiles spread over many CUs.  The LDS budget is
+// picked by a small autotuner that times the candidates on scratch copies of
+// the batch's buffers.
 //
 // Execution allocates nothing and calls no host synchronisation, so it can
 // be captured in a HIP graph.
@@ -35,7 +35,6 @@
 #include <tuple>
 
 #include "../../include/rocket_fft_hip.h"
-#include "butterfly.hpp"
 #include "passes.hpp"
 
 namespace rfh {
@@ -44,21 +43,38 @@ using namespace dev;
 
 constexpr int OP_PRE = 9;   // one line: real / half-complex input -> complex work line
 constexpr int OP_POST = 10; // one line: complex work line -> real / half-complex output
-// elements of work a unit gathers from consecutive tiles of one pass
-constexpr int64_t kUnitElems = 4096;
 // elements of a pre / post line per tile: the elementwise real-transform
 // steps are cut into tiles like the line passes, so that a long line's
 // pre / post step spreads over many workgroups instead of one
 constexpr int64_t kPrePostChunk = 2048;
 
-struct PassDev {
-  int op;
-  int tiles;
+// Workgroup sizes, and the LDS a tile may take in them: a launch reserves for
+// every workgroup what its largest tile needs, and with these limits the CU's
+// 160 KB hold the waves its registers do (four per SIMD).
+struct TileClass {
+  int threads;
+  size_t lds;
 };
-struct UnitDev {  // tiles tile0 .. tile0 + ntiles - 1 of pass `pass`
+constexpr TileClass kClass[] = {{64, 10240}, {256, 40960}, {512, 81920}, {1024, 163840}};
+constexpr int kClasses = 4;
+// A class with fewer threads than this in a level joins the next larger one
+// there: half a round of the chip's waves costs less than a launch of its own.
+constexpr int64_t kMergeThreads = 256 * 512;
+constexpr int kXcds = 8;  // workgroup i of a launch runs on XCD i mod 8
+
+template <typename T>
+struct BatchPass {
+  int op;
+  LineArgs<T> a;
+  MixGeom m;
+};
+struct UnitDev {  // tile `tile` of pass `pass`
   int pass;
-  int tile0;
-  int ntiles;
+  int tile;
+};
+struct Launch {  // units [first, first + count) in workgroups of `threads`
+  int threads, first, count;
+  size_t lds;
 };
 
 // elements [tile C, (tile + 1) C) of a pre / post line (C = kPrePostChunk)
@@ -98,65 +114,40 @@ __device__ void post_line(const LineArgs<T> &a, int tile) {
   }
 }
 
+// One tile per workgroup.  Bound by a tile's latency (about 20 us for 4096
+// elements of a column pass: arguments, loads, two twiddled exchanges, stores,
+// each waiting for the one before) times the 16 waves per CU that 128
+// registers allow: 4096 jobs 1857 -> 947 us, 2.4 GB of traffic at 2.5 TB/s,
+// against 256-thread workgroups that pulled units from a queue and ran every
+// tile, long or short, with two line buffers.
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_ragged(const UnitDev *__restrict__ units,
-                                                    int nunits,
-                                                    const PassDev *__restrict__ passes,
-                                                    const LineArgs<T> *__restrict__ args,
-                                                    unsigned *queue) {
+__global__ void __launch_bounds__(kMixThreads<T>)
+    k_ragged(const UnitDev *__restrict__ units, const BatchPass<T> *__restrict__ passes) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ int64_t s_oi[kMaxLinesPerGroup], s_oo[kMaxLinesPerGroup];
-  __shared__ int s_aux[kMaxLinesPerGroup];
-  __shared__ int s_unit;
-  for (;;) {
-    if (threadIdx.x == 0) s_unit = int(atomicAdd(queue, 1u));
-    __syncthreads();
-    const int q = __builtin_amdgcn_readfirstlane(s_unit);
-    __syncthreads();  // every lane has read s_unit before the next grab
-    if (q >= nunits) break;
-    const UnitDev u = units[q];
-    const PassDev pd = passes[u.pass];
-    const LineArgs<T> &a = args[u.pass];
-    for (int t = u.tile0; t < u.tile0 + u.ntiles; ++t) {
-      switch (pd.op) {
-        case OP_C2C: line_body<T, OP_C2C, true, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_PASSA: line_body<T, OP_PASSA, true, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_PASSB: line_body<T, OP_PASSB, true, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_BLUE: line_body<T, OP_BLUE, true, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_BLUEROW: line_body<T, OP_BLUEROW, true, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_R2C_EVEN: line_body<T, OP_R2C_EVEN, true, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_R2C_ODD: line_body<T, OP_R2C_ODD, false, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_C2R_EVEN: line_body<T, OP_C2R_EVEN, true, true>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_C2R_ODD: line_body<T, OP_C2R_ODD, true, false>(a, t, smem_raw, s_oi, s_oo, s_aux); break;
-        case OP_PRE: pre_line<T>(a, t); break;
-        default: post_line<T>(a, t); break;
-      }
-      __syncthreads();  // tile boundary: LDS and per-line slots are reused
-    }
-  }
-}
-
-__global__ void k_zero(unsigned *p, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0u;
+  const UnitDev u = units[blockIdx.x];
+  const BatchPass<T> &p = passes[u.pass];
+  if (p.op == OP_PRE) pre_line<T>(p.a, u.tile);
+  else if (p.op == OP_POST) post_line<T>(p.a, u.tile);
+  else mix_body<T, OP_ANY>(p.a, p.m, u.tile, smem_raw);
 }
 
 // ------------------------------------------------------------------ host
 
 struct Built {
-  size_t budget = 0;          // dynamic LDS per workgroup
-  DevBuf units, passes, args, queue, arena;
-  std::vector<int> level_off;  // units of level k: [level_off[k], level_off[k + 1])
+  size_t budget = 0;
+  DevBuf units, passes, arena;
+  std::vector<Launch> launches;  // in order
   std::vector<std::shared_ptr<C2CPlan>> c2c_keep;
   std::vector<std::shared_ptr<RealPlan>> real_keep;
   int njobs = 0;
-  int lds_need = 0;
+  int lds_need = 0;  // of the launch that takes most
+  int grid = 0;      // workgroups of the largest launch
 };
 
 struct Batch {
   bool dbl = false;
   std::vector<rfh_job_t> jobs;
   std::unique_ptr<Built> b;
-  int grid = 0;
   int autotuned = 0;
   double tuned_ms = 0;
 };
@@ -174,11 +165,26 @@ LineSet one_line(const void *in, void *out, int64_t esi, int64_t eso) {
   return g;
 }
 
-// cost estimate for largest-first ordering: bytes moved by all passes
-double job_cost(const std::vector<PassLaunch> &pl) {
-  double c = 0;
-  for (const auto &p : pl) c += double(p.g.nlines) * double(p.ps.nin + p.ps.nout);
-  return c;
+// Geometry of a pass's tiles: 16 elements per thread whatever the number of
+// lines (other jobs fill the CUs), short interleaved lines gathered to about
+// 256 threads, and no more lines than there are.
+template <typename T>
+MixGeom batch_geom(const PassSpec &ps, const LineArgs<T> &a) {
+  const bool inter = a.lfast_in || a.lfast_out;
+  int want = ps.lines;
+  if (inter) {
+    want = std::max(want, sizeof(T) == 8 ? 4 : 8);
+    while (want < 64 && want * 2 * ((a.f.n + 15) / 16) <= 256) want *= 2;
+    while (want > 1 && want / 2 >= a.nlines) want /= 2;
+  }
+  // a prime stage's long sums are spread over as many threads as there are
+  bool prime = false;
+  for (int s = 0; s < a.f.nst; ++s) prime = prime || a.f.st[s].radix > 17;
+  MixGeom m = mix_geometry(a.f, ps.d->pbo, sizeof(T) == 8,
+                           prime && !inter ? 1 : int64_t(1) << 30, inter, want, lds_limit());
+  if (m.L == 0) RFH_THROW(3, "ragged batch: a line does not fit in LDS");
+  if (!inter) m.L = int(std::min<int64_t>(m.L, a.nlines));
+  return m;
 }
 
 template <typename T>
@@ -236,94 +242,182 @@ std::unique_ptr<Built> build(const std::vector<rfh_job_t> &jobs, bool dbl, size_
                                            r2c ? !j.forward : j.forward, j.fct));
       continue;
     }
+    // Real lengths without a fused plan: pre -> c2c -> post through the work
+    // line.  Of an even length the pairs of reals are the complex line: r2c
+    // transforms the input as it lies, c2r into the output.
     void *work = ar + work_off[i];
-    PassSpec pre{};
-    pre.d = &cplan[i]->main;  // only desc.n (= m) is read
-    pre.op = OP_PRE;
-    pre.bign = int64_t(j.n);
     const bool half = rplan[i]->half;
-    const int pre_mode = r2c ? (half ? kPreRealPairs : kPreRealAsComplex)
-                             : (half ? kPreHalfSpectrum : kPreHermitian);
-    const int post_mode = r2c ? (half ? kPostHalfSpectrum : kPostComplexHalf)
-                              : (half ? kPostRealPairs : kPostReal);
-    pre.sub = pre_mode | (!r2c && j.forward ? R2R_CONJ : 0);
-    per[i].push_back(PassLaunch{pre, one_line(j.in, work, r2c ? 1 : 2, 2)});
-    const auto cp = describe_c2c(*cplan[i], one_line(work, work, 2, 2), r2c ? -1 : +1, 1.0,
+    const void *cin = work;
+    void *cout = work;
+    double cfct = 1.0;
+    if (r2c && half) {
+      cin = j.in;
+    } else {
+      PassSpec pre{};
+      pre.d = &cplan[i]->main;  // only desc.n (= m) is read
+      pre.op = OP_PRE;
+      pre.bign = int64_t(j.n);
+      const int mode = r2c ? kPreRealAsComplex : (half ? kPreHalfSpectrum : kPreHermitian);
+      pre.sub = mode | (!r2c && j.forward ? R2R_CONJ : 0);
+      per[i].push_back(PassLaunch{pre, one_line(j.in, work, r2c ? 1 : 2, 2)});
+    }
+    if (!r2c && half) {
+      cout = j.out;
+      cfct = j.fct;
+    }
+    const auto cp = describe_c2c(*cplan[i], one_line(cin, cout, 2, 2), r2c ? -1 : +1, cfct,
                                  ar + tmp_off[i]);
     check_tmp_spans(cp, ar + tmp_off[i],
                     c2c_tmp_bytes(*cplan[i], one_line(nullptr, nullptr, 2, 2)), dbl ? 8 : 4);
     for (const auto &pl : cp) per[i].push_back(pl);
-    PassSpec post{};
-    post.d = &cplan[i]->main;
-    post.op = OP_POST;
-    post.bign = int64_t(j.n);
-    post.fct = j.fct;
-    post.sub = (post_mode << 8) | (r2c && !j.forward ? R2R_CONJ : 0);
-    per[i].push_back(PassLaunch{post, one_line(work, j.out, 2, r2c ? 2 : 1)});
+    if (cout == work) {
+      PassSpec post{};
+      post.d = &cplan[i]->main;
+      post.op = OP_POST;
+      post.bign = int64_t(j.n);
+      post.fct = j.fct;
+      const int mode = r2c ? (half ? kPostHalfSpectrum : kPostComplexHalf) : kPostReal;
+      post.sub = (mode << 8) | (r2c && !j.forward ? R2R_CONJ : 0);
+      per[i].push_back(PassLaunch{post, one_line(work, j.out, 2, r2c ? 2 : 1)});
+    }
   }
-  // pass 3: device tables; units by level, the jobs of a level largest first
-  std::vector<PassDev> pd;
-  std::vector<LineArgs<T>> la;
-  std::vector<std::pair<double, int>> cost;
-  std::vector<int> first(jobs.size());
-  int lds_need = 0, levels = 0;
+  // pass 3: device tables; tiles by level and workgroup size
+  struct Item {  // one pass
+    double cost;  // of all its tiles: elements x stages, a prime stage by its sums
+  double time;  // of one tile, in the same units over its threads
+    int pass, tiles, level, cls;
+    size_t lds;
+  };
+  std::vector<BatchPass<T>> pd;
+  std::vector<std::vector<Item>> job_items(jobs.size());
+  int levels = 0;
+  auto class_of = [](int threads, size_t lds) {
+    int c = 0;
+    while (c < kClasses - 1 && (kClass[c].threads < threads || kClass[c].lds < lds)) ++c;
+    return c;
+  };
   for (size_t i = 0; i < jobs.size(); ++i) {
-    first[i] = int(pd.size());
     levels = std::max(levels, int(per[i].size()));
     for (const PassLaunch &pl : per[i]) {
       if (pl.ps.op == OP_BLUE_IN || pl.ps.op == OP_BLUE_MUL || pl.ps.op == OP_BLUE_OUT)
         RFH_THROW(3, "ragged batch: length " + std::to_string(jobs[i].n) +
-                         " needs the multi-pass Bluestein form, which the persistent kernel "
+                         " needs the multi-pass Bluestein form, which the batch kernel "
                          "does not run");
-      LineArgs<T> a = make_line_args<T>(pl.ps, pl.g);
-      int tiles = int((pl.g.nlines + a.L - 1) / a.L);
-      if (pl.ps.op == OP_PRE || pl.ps.op == OP_POST) {
-        a.f.n = int(cplan[i]->n);  // work-line length m
-        a.L = 1;
+      BatchPass<T> p{};
+      p.op = pl.ps.op;
+      p.a = make_line_args<T>(pl.ps, pl.g);
+      Item it{};
+      if (p.op == OP_PRE || p.op == OP_POST) {
+        p.a.f.n = int(cplan[i]->n);  // work-line length m
         // outputs of the step: the work line, or the half spectrum / real line
-        const int post_mode = (a.sub >> 8) & 0xff;
+        const int post_mode = (p.a.sub >> 8) & 0xff;
         const int64_t count =
-            pl.ps.op == OP_PRE ? int64_t(a.f.n)
-            : (post_mode == kPostComplexHalf || post_mode == kPostHalfSpectrum) ? a.bign / 2 + 1
-                                                                                 : a.bign;
-        tiles = int((count + kPrePostChunk - 1) / kPrePostChunk);
+            p.op == OP_PRE ? int64_t(p.a.f.n)
+            : (post_mode == kPostComplexHalf || post_mode == kPostHalfSpectrum) ? p.a.bign / 2 + 1
+                                                                                : p.a.bign;
+        it.tiles = int((count + kPrePostChunk - 1) / kPrePostChunk);
+        it.cost = double(count);
+        it.time = double(kPrePostChunk) / kThreads;
+        it.cls = class_of(kThreads, 0);
       } else {
-        lds_need = std::max<int>(lds_need, int(2 * a.L * a.ld * ce));
+        p.m = batch_geom<T>(pl.ps, p.a);
+        it.tiles = int((pl.g.nlines + p.m.L - 1) / p.m.L);
+        double stages = 0;
+        for (int s = 0; s < p.m.nst; ++s)
+          stages += p.m.st[s].radix > 17 ? 0.3 * p.m.st[s].radix : 1.0;
+        if (p.op == OP_BLUE || p.op == OP_BLUEROW) stages *= 2;
+        it.cost = double(pl.g.nlines) * p.a.f.n * stages;
+        it.time = double(p.a.f.n) * (stages + 4) / p.m.T;
+        it.lds = size_t(p.m.L * p.m.ld + p.m.ngen) * ce;
+        it.cls = class_of(p.m.L * p.m.T, it.lds);
+        if (it.lds > lds_limit() || p.m.L * p.m.T > kMixThreads<T>)
+          RFH_THROW(3, "ragged batch: a pass exceeds the workgroup");
       }
-      pd.push_back(PassDev{pl.ps.op, tiles});
-      la.push_back(a);
+      it.pass = int(pd.size());
+      pd.push_back(p);
+      job_items[i].push_back(it);
     }
-    cost.push_back({job_cost(per[i]), int(i)});
   }
-  if (size_t(lds_need) > budget) RFH_THROW(3, "ragged batch: a pass exceeds the LDS budget");
-  B->lds_need = lds_need;
-  std::stable_sort(cost.begin(), cost.end(),
-                   [](const std::pair<double, int> &x, const std::pair<double, int> &y) {
-                     return x.first > y.first;
-                   });
-  std::vector<UnitDev> units;
-  B->level_off.assign(1, 0);
-  for (int lv = 0; lv < levels; ++lv) {
-    for (const auto &c : cost) {
-      const size_t i = size_t(c.second);
-      if (int(per[i].size()) <= lv) continue;
-      const int pid = first[i] + lv;
-      const LineArgs<T> &a = la[size_t(pid)];
-      // a unit holds enough tiles for about kUnitElems elements of work
-      const bool pp = pd[size_t(pid)].op == OP_PRE || pd[size_t(pid)].op == OP_POST;
-      const int64_t per_tile =
-          pp ? kPrePostChunk : int64_t(std::max(1, a.L)) * std::max(1, a.f.n);
-      const int tpu = int(std::max<int64_t>(1, kUnitElems / per_tile));
-      for (int t0 = 0; t0 < pd[size_t(pid)].tiles; t0 += tpu)
-        units.push_back(UnitDev{pid, t0, std::min(tpu, pd[size_t(pid)].tiles - t0)});
+  // Levels: a job of fewer passes than the longest starts where the least work
+  // is, so that the one-pass jobs fill the levels that few long ones reach.
+  std::vector<double> load(size_t(levels), 0.0);
+  std::vector<size_t> order(jobs.size());
+  for (size_t i = 0; i < jobs.size(); ++i) order[i] = i;
+  auto job_cost = [&](size_t i) {
+    double c = 0;
+    for (const Item &it : job_items[i]) c += it.cost;
+    return c;
+  };
+  std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) {
+    const auto key = [&](size_t i) { return std::make_pair(job_items[i].size(), job_cost(i)); };
+    return key(x) > key(y);
+  });
+  std::vector<std::vector<Item>> by_level(size_t(levels) * kClasses);
+  for (size_t i : order) {
+    const size_t np = job_items[i].size();
+    size_t at = 0;
+    double best = 1e300;
+    for (size_t o = 0; o + np <= size_t(levels); ++o) {
+      double most = 0;
+      for (size_t k = 0; k < np; ++k) most = std::max(most, load[o + k] + job_items[i][k].cost);
+      if (most < best) {
+        best = most;
+        at = o;
+      }
     }
-    B->level_off.push_back(int(units.size()));
+    for (size_t k = 0; k < np; ++k) {
+      Item &it = job_items[i][k];
+      load[at + k] += it.cost;
+      by_level[(at + k) * kClasses + size_t(it.cls)].push_back(it);
+    }
+  }
+  std::vector<UnitDev> units;
+  for (int lv = 0; lv < levels; ++lv) {
+    std::vector<Item> *cl = &by_level[size_t(lv) * kClasses];
+    for (int c = 0; c < kClasses - 1; ++c) {
+      int64_t threads = 0;
+      for (const Item &it : cl[c]) threads += int64_t(it.tiles) * kClass[c].threads;
+      int up = c + 1;
+      while (up < kClasses && cl[up].empty()) ++up;
+      if (threads && threads < kMergeThreads && up < kClasses) {
+        cl[up].insert(cl[up].end(), cl[c].begin(), cl[c].end());
+        cl[c].clear();
+      }
+    }
+    for (int c = kClasses - 1; c >= 0; --c) {
+      if (cl[c].empty()) continue;
+      Launch L{std::min(kClass[c].threads, kMixThreads<T>), int(units.size()), 0, 0};
+      // the longest tiles first; all tiles of a pass on one XCD, whose L2
+      // then holds the pass's tables once
+      std::stable_sort(cl[c].begin(), cl[c].end(), [](const Item &x, const Item &y) {
+        return x.time > y.time;
+      });
+      std::vector<UnitDev> q[kXcds];
+      for (const Item &it : cl[c]) {
+        int x = 0;
+        for (int k = 1; k < kXcds; ++k)
+          if (q[k].size() < q[x].size()) x = k;
+        for (int t = 0; t < it.tiles; ++t) q[x].push_back(UnitDev{it.pass, t});
+        L.count += it.tiles;
+        L.lds = std::max(L.lds, it.lds);
+      }
+      size_t head[kXcds] = {};
+      for (int i = 0; i < L.count; ++i) {
+        int x = i % kXcds;
+        if (head[x] == q[x].size())  // this one is empty: the fullest gives a tile
+          for (int k = 0; k < kXcds; ++k)
+            if (q[k].size() - head[k] > q[x].size() - head[x]) x = k;
+        units.push_back(q[x][head[x]++]);
+      }
+      B->launches.push_back(L);
+    }
+  }
+  for (const Launch &L : B->launches) {
+    B->lds_need = std::max(B->lds_need, int(L.lds));
+    B->grid = std::max(B->grid, L.count);
   }
   B->units.upload(units.data(), units.size() * sizeof(UnitDev));
-  B->passes.upload(pd.data(), pd.size() * sizeof(PassDev));
-  B->args.upload(la.data(), la.size() * sizeof(LineArgs<T>));
-  std::vector<unsigned> zeros(size_t(std::max(levels, 1)), 0u);
-  B->queue.upload(zeros.data(), zeros.size() * sizeof(unsigned));
+  B->passes.upload(pd.data(), pd.size() * sizeof(BatchPass<T>));
   for (auto &p : cplan)
     if (p) B->c2c_keep.push_back(p);
   for (auto &p : rplan)
@@ -335,7 +429,7 @@ std::mutex g_attr_mu;
 std::set<std::pair<int, int>> g_attr_set;  // (device, double precision)
 
 template <typename T>
-void launch_batch(const Built &B, int grid, hipStream_t s) {
+void launch_batch(const Built &B, hipStream_t s) {
   if (B.njobs == 0) return;
   const void *fn = reinterpret_cast<const void *>(&k_ragged<T>);
   {
@@ -350,17 +444,10 @@ void launch_batch(const Built &B, int grid, hipStream_t s) {
       g_attr_set.insert({dev, int(sizeof(T) == 8)});
     }
   }
-  const int levels = int(B.level_off.size()) - 1;
-  unsigned *queue = static_cast<unsigned *>(B.queue.p);
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, s, queue, levels);
-  for (int lv = 0; lv < levels; ++lv) {
-    const int n = B.level_off[size_t(lv) + 1] - B.level_off[size_t(lv)];
-    if (n == 0) continue;
-    hipLaunchKernelGGL(k_ragged<T>, dim3(unsigned(std::min(grid, n))), dim3(kThreads),
-                       size_t(B.lds_need), s,
-                       static_cast<const UnitDev *>(B.units.p) + B.level_off[size_t(lv)], n,
-                       static_cast<const PassDev *>(B.passes.p),
-                       static_cast<const LineArgs<T> *>(B.args.p), queue + lv);
+  for (const Launch &L : B.launches) {
+    hipLaunchKernelGGL(k_ragged<T>, dim3(unsigned(L.count)), dim3(unsigned(L.threads)), L.lds, s,
+                       static_cast<const UnitDev *>(B.units.p) + L.first,
+                       static_cast<const BatchPass<T> *>(B.passes.p));
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) RFH_THROW(2, std::string("ragged launch: ") + hipGetErrorString(e));
   }
@@ -377,20 +464,20 @@ int cu_count() {
   return n;
 }
 
-void run(Batch &bt, int grid, hipStream_t s) {
+void run(Batch &bt, hipStream_t s) {
   if (bt.dbl)
-    launch_batch<double>(*bt.b, grid, s);
+    launch_batch<double>(*bt.b, s);
   else
-    launch_batch<float>(*bt.b, grid, s);
+    launch_batch<float>(*bt.b, s);
 }
 
-double time_ms(Batch &bt, int grid, hipStream_t s, int reps) {
+double time_ms(Batch &bt, hipStream_t s, int reps) {
   hipEvent_t e0, e1;
   HIP_CHECK(hipEventCreate(&e0));
   HIP_CHECK(hipEventCreate(&e1));
-  run(bt, grid, s);  // warm
+  run(bt, s);  // warm
   HIP_CHECK(hipEventRecord(e0, s));
-  for (int r = 0; r < reps; ++r) run(bt, grid, s);
+  for (int r = 0; r < reps; ++r) run(bt, s);
   HIP_CHECK(hipEventRecord(e1, s));
   HIP_CHECK(hipEventSynchronize(e1));
   float ms = 0;
@@ -404,13 +491,13 @@ std::unique_ptr<Built> build_any(const Batch &bt, size_t budget) {
   return bt.dbl ? build<double>(bt.jobs, true, budget) : build<float>(bt.jobs, false, budget);
 }
 
-// Autotuner: LDS budget (which sets the four-step splits and how many
-// workgroups share a CU) x grid size; each candidate is timed on the batch.
+// Autotuner: the LDS budget, which sets how long a line runs in one pass
+// (a long one has a CU to itself); each candidate is timed on the batch.
 // Results are kept per batch signature (precision, then kind and length of
 // every job) for the process and, when a cache directory is set, in a text
 // file per GPU architecture and CU count that later processes read:
 //   <dir>/ragged_tune_<arch>_<cus>cu.txt, one line per signature:
-//   "rfh1 <fnv-1a hash> <second hash> <jobs> <lds budget> <grid>"
+//   "rfh1 <fnv-1a hash> <second hash> <jobs> <lds budget> <largest grid>"
 // Lines are appended with one write each; unreadable lines are ignored.
 std::mutex g_tune_mu;
 std::map<std::vector<uint64_t>, std::pair<size_t, int>> g_tuned;
@@ -442,13 +529,9 @@ DiskKey disk_key(const std::vector<uint64_t> &sig) {
   return DiskKey{h1, h2, uint64_t(sig.size())};
 }
 
-// LDS budgets the autotuner tries (the device limit less the kernel's static
-// LDS caps the larger two)
-std::vector<size_t> tune_budgets() {
-  const size_t cap = lds_limit() - 8192;
-  return {size_t(32768), size_t(65536), std::min<size_t>(98304, cap),
-          std::min<size_t>(147456, cap)};
-}
+// LDS budgets the autotuner tries: lines of up to 4096 / 8192 complex64
+// elements in one pass, or all that fit a CU
+std::vector<size_t> tune_budgets() { return {size_t(65536), size_t(131072), whole_line_budget()}; }
 
 bool budget_ok(size_t b) {
   for (size_t c : tune_budgets())
@@ -484,7 +567,7 @@ void load_disk(const std::string &path) {
     size_t budget = 0;
     int grid = 0;
     if (!(is >> tag >> std::hex >> k.h1 >> k.h2 >> std::dec >> k.n >> budget >> grid)) continue;
-    if (tag != "rfh1" || !budget_ok(budget) || grid <= 0 || grid > 64 * cu_count()) continue;
+    if (tag != "rfh1" || !budget_ok(budget) || grid <= 0) continue;
     g_disk[k] = {budget, grid};
   }
 }
@@ -510,7 +593,6 @@ void autotune(Batch &bt, hipStream_t s) {
     auto it = g_tuned.find(sig);
     if (it != g_tuned.end()) {
       bt.b = build_any(bt, it->second.first);
-      bt.grid = it->second.second;
       bt.autotuned = 2;
       return;
     }
@@ -527,7 +609,6 @@ void autotune(Batch &bt, hipStream_t s) {
         }
         if (b) {
           bt.b = std::move(b);
-          bt.grid = d->second.second;
           bt.autotuned = 3;
           g_tuned[sig] = d->second;
           return;
@@ -569,37 +650,29 @@ void autotune(Batch &bt, hipStream_t s) {
   }
   double best = 1e300;
   size_t best_budget = 0;
-  int best_grid = 0;
   for (size_t budget : tune_budgets()) {
     try {
       tb.b = build_any(tb, budget);
     } catch (const Error &) {
       continue;
     }
-    const int per_cu = std::max(1, int((lds_limit() - 8192) / std::max<size_t>(tb.b->lds_need, 1)));
-    for (int wpc : {1, 2, 4}) {
-      if (wpc > per_cu) continue;
-      const int grid = cu_count() * wpc;
-      const double ms = time_ms(tb, grid, s, 3);
-      if (ms < best) {
-        best = ms;
-        best_budget = budget;
-        best_grid = grid;
-      }
+    const double ms = time_ms(tb, s, 3);
+    if (ms < best) {
+      best = ms;
+      best_budget = budget;
     }
   }
   HIP_CHECK(hipStreamSynchronize(s));  // the timing runs are done with the scratch copies
   tb.b.reset();
   if (!best_budget) RFH_THROW(3, "ragged batch: no LDS budget fits every job");
   bt.b = build_any(bt, best_budget);
-  bt.grid = best_grid;
   bt.autotuned = 1;
   bt.tuned_ms = best;
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tuned[sig] = {best_budget, best_grid};
+  g_tuned[sig] = {best_budget, bt.b->grid};
   if (!path.empty() && path == cache_file()) {
-    append_disk(path, dk, best_budget, best_grid);
-    g_disk[dk] = {best_budget, best_grid};
+    append_disk(path, dk, best_budget, bt.b->grid);
+    g_disk[dk] = {best_budget, bt.b->grid};
   }
 }
 
@@ -665,7 +738,6 @@ int rfh_batch_create(const rfh_job_t *jobs, int64_t njobs, bool double_precision
         autotune(*bt, s);
       } else {
         bt->b = build_any(*bt, 65536);
-        bt->grid = cu_count() * 2;
       }
     } catch (...) {
       delete bt;
@@ -678,7 +750,7 @@ int rfh_batch_create(const rfh_job_t *jobs, int64_t njobs, bool double_precision
 int rfh_batch_execute(void *handle, void *stream) {
   return guarded_int([&] {
     Batch *bt = static_cast<Batch *>(handle);
-    run(*bt, bt->grid, static_cast<hipStream_t>(stream));
+    run(*bt, static_cast<hipStream_t>(stream));
   });
 }
 
@@ -742,7 +814,7 @@ int rfh_tune_cache(const char *dir, bool clear_memory) {
 
 int rfh_batch_info(void *handle, int *grid, int *lds_bytes, int *autotuned, double *tuned_ms) {
   Batch *bt = static_cast<Batch *>(handle);
-  *grid = bt->grid;
+  *grid = bt->b ? bt->b->grid : 0;
   *lds_bytes = bt->b ? bt->b->lds_need : 0;
   *autotuned = bt->autotuned;
   *tuned_ms = bt->tuned_ms;

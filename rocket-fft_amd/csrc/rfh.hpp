@@ -22,12 +22,9 @@ constexpr int kMaxBatchDims = 10;
 constexpr int kMaxDims = 32;
 constexpr int kMaxLinesPerGroup = 256;
 constexpr int kThreads = 256;
-// LDS kept back from the line kernels' dynamic buffers for their static
-// arrays: the per-line offset slots, 8 + 8 + 4 bytes for each of up to
-// kMaxLinesPerGroup lines (5120 B), rounded up.  The launch checks the
-// kernel's actual static size against the device limit.
+// Ordinary plans run lines in one pass up to the length of which two buffers fit
+// the LDS less this (4928 complex128, 9856 complex64 elements).
 constexpr size_t kLineStaticLds = 6144;
-static_assert(kLineStaticLds >= kMaxLinesPerGroup * (8 + 8 + 4), "line kernel static LDS");
 
 // ------------------------------------------------------------------ errors
 
@@ -55,7 +52,7 @@ void fork_guard();
 
 // One Stockham stage of an LDS-resident FFT: radix, ns = product of the
 // radices before it, offsets of its twiddles W_{ns*radix}^{k*r} (r = 1..radix-1,
-// k < ns, laid out [(r-1)*ns + k]) and, for odd radices above 5, of its
+// k < ns, laid out [(r-1)*ns + k]) and, for primes above 17, of its
 // table of roots W_radix^q (q < radix) stored as (cos, sin).
 struct Stage {
   int radix;
@@ -85,7 +82,7 @@ struct DevBuf {
 struct Direct {
   FftDesc desc{};
   DevBuf tw;   // stage twiddles (complex, plan precision)
-  DevBuf gen;  // roots for radices 7, 11, 13 and generic odd primes
+  DevBuf gen;  // roots of primes above 17
   int pbo[kMaxStages] = {};  // LDS pitch of the blocks each stage writes
 };
 

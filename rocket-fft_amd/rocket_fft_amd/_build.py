@@ -27,7 +27,8 @@ FLAGS = [
 # hoisting their constants and strides out of it costs hundreds of spilled
 # scalar registers.
 FILE_FLAGS = {s: ["-mllvm", "-disable-machine-licm"]
-              for s in ("lines_c2c.hip", "lines_blue.hip", "lines_real.hip", "lines_r2r.hip")}
+              for s in ("lines_c2c.hip", "lines_blue.hip", "lines_real.hip", "lines_r2r.hip",
+                        "ragged.hip")}
 
 
 def _compile(src):
