@@ -106,6 +106,12 @@ void rfh_clear_error(void);
  * arrays always block).  Returns 0 on success. */
 int rfh_set_stream(void *stream, bool blocking);
 
+/* One call on a stream: rfh_begin(stream) is rfh_set_stream(stream, false) and
+ * rfh_clear_error(); rfh_end() is rfh_set_stream(NULL, true) and returns the
+ * code of the calls in between (0: none failed). */
+void rfh_begin(void *stream);
+int rfh_end(void);
+
 /* Enables (default) or disables the compile-time specialised line kernels
  * for power-of-two lengths; disabled, every transform runs the generic
  * kernels.  Process-wide; meant for tests that compare the two paths. */

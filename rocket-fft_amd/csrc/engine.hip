@@ -382,12 +382,30 @@ void span_of(const Arr &a, size_t scalar, size_t elem_scalars, int64_t *lo, int6
   *hi = (h + int64_t(elem_scalars)) * int64_t(scalar);
 }
 
+// Whether the elements of `a` lie without gaps or overlaps in their span.
+bool dense(const Arr &a, size_t elem_scalars) {
+  int dims[kMaxDims], nd = 0;
+  for (int d = 0; d < a.ndim; ++d)
+    if (a.shape[d] > 1) dims[nd++] = d;
+  std::sort(dims, dims + nd,
+            [&](int x, int y) { return std::llabs(a.str[x]) < std::llabs(a.str[y]); });
+  int64_t st = int64_t(elem_scalars);
+  for (int k = 0; k < nd; ++k) {
+    if (std::llabs(a.str[dims[k]]) != st) return false;
+    st *= a.shape[dims[k]];
+  }
+  return true;
+}
+
 // Runs `body` with device-visible data pointers; host arrays are staged
-// through device buffers (input span copied in, output span copied in
-// first so untouched gaps survive, then copied back).
+// through device buffers: the input span is copied in, the output span copied
+// back.  The output is copied in first only where the transform leaves
+// something of it alone: gaps between its elements, elements beyond the ones
+// it writes (whole_out false), or an input inside its span (256 x 1000
+// complex128: 558 -> 406 us a call).
 template <typename F>
 void with_device_arrays(Arr &in, size_t in_elem, Arr &out, size_t out_elem, size_t scalar,
-                        F &&body) {
+                        F &&body, bool whole_out = true) {
   int dev_in = -1, dev_out = -1;
   const bool din = is_device_ptr(in.data, &dev_in);
   const bool dout = is_device_ptr(out.data, &dev_out);
@@ -410,16 +428,19 @@ void with_device_arrays(Arr &in, size_t in_elem, Arr &out, size_t out_elem, size
   char *in_host = in.data, *out_host = out.data;
   int64_t ilo = 0, ihi = 0, olo = 0, ohi = 0;
   char *out_dev_base = nullptr;
+  bool inside = false;  // the input lies in the output's span
+  if (!din) span_of(in, scalar, in_elem, &ilo, &ihi);
   if (!dout) {
     span_of(out, scalar, out_elem, &olo, &ohi);
+    inside = !din && in_host + ilo >= out_host + olo && in_host + ihi <= out_host + ohi;
     out_dev_base = static_cast<char *>(ws.get(kSlotHostOut, size_t(ohi - olo)));
-    HIP_CHECK(hipMemcpyAsync(out_dev_base, out_host + olo, size_t(ohi - olo),
-                             hipMemcpyHostToDevice, s));
+    if (inside || !whole_out || !dense(out, out_elem))
+      HIP_CHECK(hipMemcpyAsync(out_dev_base, out_host + olo, size_t(ohi - olo),
+                               hipMemcpyHostToDevice, s));
     out.data = out_dev_base - olo;
   }
   if (!din) {
-    span_of(in, scalar, in_elem, &ilo, &ihi);
-    if (!dout && in_host + ilo >= out_host + olo && in_host + ihi <= out_host + ohi) {
+    if (inside) {
       in.data = out.data + (in_host - out_host);  // inside the output span
     } else {
       char *b = static_cast<char *>(ws.get(kSlotHostIn, size_t(ihi - ilo)));
@@ -582,12 +603,16 @@ void r2c(uint64_t ndim, const arystruct_t *ain, arystruct_t *aout, arystruct_t *
   std::copy(shape, shape + ndim, need);
   if (!sym) need[ax.back()] = shape[ax.back()] / 2 + 1;
   check_fits(out, need, "output");  // out keeps its own extent for host staging
-  with_device_arrays(in, 1, out, 2, sc, [&](Ctx &c) {
-    c.dbl = dbl;
-    r2c_nd(c, in.shape, in.ndim, in.str, out.str, ax.data(), int(ax.size()), in.data,
-           out.data, forward, fct);
-    if (sym) launch_sym_fill(mirror_geom(in.shape, out.str, int(ndim), ax), dbl, out.data, c.s);
-  });
+  with_device_arrays(
+      in, 1, out, 2, sc,
+      [&](Ctx &c) {
+        c.dbl = dbl;
+        r2c_nd(c, in.shape, in.ndim, in.str, out.str, ax.data(), int(ax.size()), in.data,
+               out.data, forward, fct);
+        if (sym)
+          launch_sym_fill(mirror_geom(in.shape, out.str, int(ndim), ax), dbl, out.data, c.s);
+      },
+      std::equal(need, need + ndim, out.shape));
 }
 
 void c2r(uint64_t ndim, const arystruct_t *ain, arystruct_t *aout, arystruct_t *axes,
@@ -915,6 +940,19 @@ int rfh_last_error(char *buf, size_t len) {
 void rfh_clear_error(void) {
   t_err = 0;
   t_msg.clear();
+}
+
+void rfh_begin(void *stream) {
+  t_stream = static_cast<hipStream_t>(stream);
+  t_blocking = false;
+  t_err = 0;
+  t_msg.clear();
+}
+
+int rfh_end(void) {
+  t_stream = nullptr;
+  t_blocking = true;
+  return t_err;
 }
 
 int rfh_set_stream(void *stream, bool blocking) {

@@ -24,6 +24,7 @@ stream, asynchronously like any torch op).  There is no CPU fallback: the
 functions raise if the HIP library is missing.
 """
 import ctypes
+import math
 import numbers
 import os
 
@@ -71,6 +72,10 @@ def _load():
     L.rfh_last_error.restype = ctypes.c_int
     L.rfh_clear_error.argtypes = []
     L.rfh_clear_error.restype = None
+    L.rfh_begin.argtypes = [vp]
+    L.rfh_begin.restype = None
+    L.rfh_end.argtypes = []
+    L.rfh_end.restype = ctypes.c_int
     L.rfh_set_stream.argtypes = [vp, b]
     L.rfh_set_stream.restype = ctypes.c_int
     for name in ("rfh_cfftp_factors", "rfh_rfftp_factors"):
@@ -100,13 +105,14 @@ _struct_cache = {}
 
 
 def _arystruct_type(ndim):
+    """(structure, shape-and-strides array) types of an ndim-dimensional array."""
     t = _struct_cache.get(ndim)
     if t is None:
-        t = type(f"arystruct_{ndim}", (ctypes.Structure,), {"_fields_": [
+        dims = ctypes.c_int64 * (2 * max(ndim, 1))
+        t = (type(f"arystruct_{ndim}", (ctypes.Structure,), {"_fields_": [
             ("meminfo", ctypes.c_void_p), ("parent", ctypes.c_void_p),
             ("nitems", ctypes.c_int64), ("itemsize", ctypes.c_int64),
-            ("data", ctypes.c_void_p),
-            ("shape_and_strides", ctypes.c_int64 * (2 * max(ndim, 1)))]})
+            ("data", ctypes.c_void_p), ("shape_and_strides", dims)]}), dims)
         _struct_cache[ndim] = t
     return t
 
@@ -115,20 +121,28 @@ def _is_torch(a):
     return type(a).__module__.startswith("torch")
 
 
-_TORCH_ITEMSIZE = {"torch.float32": 4, "torch.float64": 8, "torch.complex64": 8,
-                   "torch.complex128": 16}
+_TORCH_ITEM = {}  # dtype -> (item size, kind)
+
+
+def _torch_item(dtype):
+    item = _TORCH_ITEM.get(dtype)
+    if item is None:
+        import torch
+        _TORCH_ITEM.update({torch.float32: (4, "f"), torch.float64: (8, "f"),
+                            torch.complex64: (8, "c"), torch.complex128: (16, "c")})
+        item = _TORCH_ITEM.get(dtype)
+        if item is None:
+            raise TypeError(f"unsupported tensor dtype {dtype}")
+    return item
 
 
 def _describe(a):
     """(ndim, shape, byte strides, itemsize, data pointer, kind, is_cuda)."""
     if _is_torch(a):
-        key = str(a.dtype)
-        if key not in _TORCH_ITEMSIZE:
-            raise TypeError(f"unsupported tensor dtype {a.dtype}")
-        isz = _TORCH_ITEMSIZE[key]
-        kind = "c" if a.is_complex() else "f"
-        return (a.dim(), tuple(a.shape), tuple(s * isz for s in a.stride()), isz,
-                a.data_ptr(), kind, a.is_cuda)
+        isz, kind = _torch_item(a.dtype)
+        shape = a.shape
+        return (len(shape), shape, [s * isz for s in a.stride()], isz, a.data_ptr(), kind,
+                a.is_cuda)
     if not isinstance(a, np.ndarray):
         raise TypeError("arrays must be numpy arrays or torch tensors")
     if a.dtype.kind not in "fc" or a.dtype.itemsize not in (4, 8, 16):
@@ -138,17 +152,29 @@ def _describe(a):
 
 def _struct(a):
     nd, shape, strides, isz, ptr, kind, cuda = _describe(a)
-    S = _arystruct_type(nd)()
-    S.nitems = int(np.prod(shape)) if nd else 1
-    S.itemsize = isz
-    S.data = ptr
-    for i in range(nd):
-        S.shape_and_strides[i] = shape[i]
-        S.shape_and_strides[nd + i] = strides[i]
-    return S, nd, kind, cuda
+    S, dims = _arystruct_type(nd)
+    return (S(None, None, math.prod(shape), isz, ptr, dims(*shape, *strides)), nd, kind, cuda)
+
+
+def _raw_stream(device):
+    """The handle of torch's current stream on a device."""
+    import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # 0.1 us, a Stream object 1.8
+    if raw is not None and device.index is not None:
+        return raw(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def _axes_struct(axes, ndim):
+    S, dims = _arystruct_type(1)
+    if type(axes) is np.ndarray and axes.ndim == 1 and axes.dtype == np.int64:
+        axes = axes.tolist()
+    if type(axes) is list and all(type(a) is int for a in axes):  # the usual forms
+        if any(a < 0 or a >= ndim for a in axes):
+            raise ValueError("axis out of range")
+        n = len(axes)
+        keep = (ctypes.c_uint64 * max(n, 1))(*axes)
+        return S(None, None, n, 8, ctypes.addressof(keep), dims(n, 8)), keep
     ax = np.asarray(axes)
     if ax.ndim != 1:
         raise TypeError("Axes must be a one-dimensional array")
@@ -157,21 +183,19 @@ def _axes_struct(axes, ndim):
     if ax.size and (ax.min() < 0 or ax.max() >= ndim):
         raise ValueError("axis out of range")
     ax = ax.astype(np.uint64)
-    S = _arystruct_type(1)()
-    S.nitems = ax.size
-    S.itemsize = 8
-    S.data = ax.ctypes.data
-    S.shape_and_strides[0] = ax.size
-    S.shape_and_strides[1] = 8
-    return S, ax
+    return S(None, None, ax.size, 8, ax.ctypes.data, dims(ax.size, 8)), ax
 
 
 def _check_bool(name, v):
+    if v is True or v is False:
+        return
     if not isinstance(v, (bool, np.bool_)):
         raise TypeError(f"'{name}' must be a boolean")
 
 
 def _check_int(name, v):
+    if type(v) is int:
+        return
     if isinstance(v, (bool, np.bool_)) or not isinstance(v, (numbers.Integral, np.integer)):
         raise TypeError(f"'{name}' must be an integer")
 
@@ -179,6 +203,8 @@ def _check_int(name, v):
 def _check_float(name, v):
     # rocket_fft/pocketfft.py widens float arguments only; integer fct fails
     # typing there (tests/test_low_level_interface.py:218-225)
+    if type(v) is float:
+        return
     if isinstance(v, (bool, np.bool_, numbers.Integral, np.integer)) or not isinstance(
             v, (numbers.Real, np.floating)):
         raise TypeError(f"'{name}' must be a floating-point number")
@@ -191,21 +217,21 @@ def _call(fname, ain, aout, axes, *mid):
         raise TypeError("Input and output array must have the same number of dimensions")
     S_ax, keep = _axes_struct(axes, nd)
     L = _load()
-    stream = None
+    run = getattr(L, fname)
+    args = (nd, ctypes.byref(S_in), ctypes.byref(S_out), ctypes.byref(S_ax), *mid)
     if cin or cout:
-        import torch
-        stream = torch.cuda.current_stream(aout.device if cout else ain.device).cuda_stream
-        L.rfh_set_stream(ctypes.c_void_p(stream), False)
-    try:
+        L.rfh_begin(_raw_stream(aout.device if cout else ain.device))
+        try:
+            run(*args)
+        finally:
+            code = L.rfh_end()
+    else:
         L.rfh_clear_error()
-        getattr(L, fname)(nd, ctypes.byref(S_in), ctypes.byref(S_out), ctypes.byref(S_ax), *mid)
-        code, msg = last_error()
-    finally:
-        if stream is not None:
-            L.rfh_set_stream(None, True)
+        run(*args)
+        code = L.rfh_last_error(None, 0)
     del keep
     if code:
-        raise RuntimeError(f"{fname}: {msg}")
+        raise RuntimeError(f"{fname}: {last_error()[1]}")
     return aout
 
 

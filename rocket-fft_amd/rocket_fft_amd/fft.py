@@ -45,11 +45,18 @@ def _is_torch(a):
     return type(a).__module__.startswith("torch")
 
 
+_PAIRS = {}  # dtype -> _dtype_pair
+
+
 def _dtype_pair(a):
     """(real dtype, complex dtype) names for the transform of a."""
-    name = str(a.dtype).replace("torch.", "")
-    single = name in ("float32", "complex64")
-    return ("float32", "complex64") if single else ("float64", "complex128")
+    pair = _PAIRS.get(a.dtype)
+    if pair is None:
+        single = str(a.dtype).replace("torch.", "") in ("float32", "complex64")
+        pair = ("float32", "complex64") if single else ("float64", "complex128")
+        if len(_PAIRS) < 64:
+            _PAIRS[a.dtype] = pair
+    return pair
 
 
 def _is_complex(a):
@@ -97,7 +104,7 @@ def _shape_and_axes(a, s, axes):
     nd = a.ndim
     if s is not None and isinstance(s, numbers.Integral):
         s = [s]
-    if axes is not None and isinstance(axes, numbers.Integral):
+    if axes is not None and type(axes) not in (list, tuple) and isinstance(axes, numbers.Integral):
         axes = [axes]
     if s is not None:
         s = [int(v) for v in s]
@@ -152,7 +159,7 @@ def _fct(shape, axes, norm, forward, delta=None):
 
 
 def _ax(axes):
-    return np.asarray(axes, dtype=np.int64)
+    return [int(a) for a in axes]
 
 
 # ------------------------------------------------------------- drivers
