@@ -156,8 +156,8 @@ enum LineOp {
   OP_BLUE_MUL = 12,  // work[m] *= kernel[m]
   OP_BLUE_OUT = 13,  // y[m] = fct * work[m] * conj(chirp[m]) for m < n
   // Bluestein rows of the three-pass form: forward FFT of the row, times the
-  // kernel t2 at m = aux + k * other, inverse FFT, times the inverse four-step
-  // twiddle (tables t0 / t1); written back in place
+  // kernel (t2, laid out by rows: bin k of row aux at aux * n + k), inverse FFT,
+  // times the inverse four-step twiddle (tables t0 / t1); written back in place
   OP_BLUEROW = 14,
 };
 // OP_R2R packs its modes into LineArgs::sub

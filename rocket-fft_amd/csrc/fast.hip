@@ -104,16 +104,62 @@ __device__ __forceinline__ C2<T> fload(const FCtx<T> &c, int p) {
     const int h = a.f.n;
     return c2r_pre(a, c.rtw, ldc<VIN>(c.gin + p * a.esi), ldc<VIN>(c.gin + (h - p) * a.esi), p);
   } else if constexpr (OP == OP_PASSA) {
-    if (a.sub & SUB_CHIRP) {  // Bluestein columns: x[m] times the chirp, zero from m = n on
-      const int64_t m = int64_t(p) * a.other + c.aux;
-      if (m >= a.bign) return C2<T>{T(0), T(0)};
-      const C2<T> ch = a.t2[m];
-      const int64_t off = blue_col_offset(p, m, a.rot_in, a.bign, c.aux, a.esi, a.other);
-      return cmul(ldc<VIN>(c.gin + off), (a.sub & SUB_CONJ) ? ch : conjc(ch));
-    }
     return ldc<VIN>(c.gin + ((p + a.rot_in) & (a.f.n - 1)) * a.esi);
   } else {  // OP_C2C (power-of-two lengths: the rotation is a mask)
     return ldc<VIN>(c.gin + ((p + a.rot_in) & (a.f.n - 1)) * a.esi);
+  }
+}
+
+// Bluestein columns: inputs p = j + r NR (r < R) times the chirp, zero from
+// m = n on.  Every load comes before the first product, under conditions the
+// whole wave shares only (the lanes past n read element aux): with a branch on
+// m around each load a thread's loads waited for one another.
+template <typename T, int R, int NR, bool VIN>
+__device__ __forceinline__ void chirp_load(const FCtx<T> &c, int j, C2<T> (&v)[R]) {
+  const LineArgs<T> &a = *c.a;
+  C2<T> ch[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    v[r] = ch[r] = C2<T>{T(0), T(0)};
+    if (int64_t(r * NR) * a.other < a.bign) {
+      const int p = j + r * NR;
+      const int64_t m = int64_t(p) * a.other + c.aux;
+      const bool on = m < a.bign;
+      const int64_t mc = on ? m : c.aux;
+      ch[r] = a.t2[mc];
+      v[r] = ldc<VIN>(c.gin + blue_col_offset(on ? p : 0, mc, a.rot_in, a.bign, c.aux, a.esi,
+                                              a.other));
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool on = int64_t(j + r * NR) * a.other + c.aux < a.bign;
+    const C2<T> y = cmul(v[r], (a.sub & SUB_CONJ) ? ch[r] : conjc(ch[r]));
+    v[r] = on ? y : C2<T>{T(0), T(0)};
+  }
+}
+
+// Bluestein columns, last pass: bins p = j + r NS (r < R) times the chirp and
+// fct, those below n stored; the chirps are loaded as above.
+template <typename T, int R, int NS, bool VOUT>
+__device__ __forceinline__ void chirp_store(const FCtx<T> &c, int j, const C2<T> (&v)[R]) {
+  const LineArgs<T> &a = *c.a;
+  C2<T> ch[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    ch[r] = C2<T>{T(0), T(0)};
+    if (int64_t(r * NS) * a.other < a.bign) {
+      const int64_t m = c.aux + int64_t(j + r * NS) * a.other;
+      ch[r] = a.t0[m < a.bign ? m : c.aux];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int p = j + r * NS;
+    const int64_t m = c.aux + int64_t(p) * a.other;
+    if (m < a.bign)
+      stc<VOUT>(c.gout + blue_col_offset(p, m, a.rot_out, a.bign, c.aux, a.eso, a.other),
+                a.fct * cmul(v[r], (a.sub & SUB_CONJ) ? ch[r] : conjc(ch[r])));
   }
 }
 
@@ -256,6 +302,50 @@ __device__ __forceinline__ void c2r_load_shuffled(const FCtx<T> &c, C2<T> (&v)[R
   }
 }
 
+// Bluestein rows, inverse transform (65537 = 256 x 512, 128 lines c64: 101 -> 82
+// us for the rows against both transforms in order through LDS, 12 passes over
+// it instead of 8): stage S undone (butterfly with the other
+// sign, conjugate twiddles), reading where the forward stage had written and
+// writing where it had read; stage 0 stores.
+template <typename T, int N, int TPL, int OP, bool VOUT, typename SC, int S>
+__device__ __forceinline__ void funstage(const FCtx<T> &c) {
+  constexpr int R = SC::at(S), NS = SC::ns(S), NR = N / R, Q = (NR + TPL - 1) / TPL;
+  const LineArgs<T> &a = *c.a;
+  C2<T> v[Q][R];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int j = c.i + q * TPL;
+    if (Q * TPL == NR || j < NR) {
+      const int k = j % NS;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q][r] = c.line[padi<T>((j - k) * R + k + r * NS)];
+      dft<R>(v[q], -c.dir);
+      if constexpr (S > 0) {
+        const C2<T> *tw = a.tw + a.f.st[S].twoff;
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], dirw(tw[(r - 1) * NS + k], -c.dir));
+      } else if (c.valid) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          fstore<T, OP, VOUT>(a, c.twl, c.gout, c.aux, j + r * NR, v[q][r]);
+      }
+    }
+  }
+  if constexpr (S > 0) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int j = c.i + q * TPL;
+      if (Q * TPL == NR || j < NR) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) c.line[padi<T>(j + r * NR)] = v[q][r];
+      }
+    }
+    __syncthreads();
+    funstage<T, N, TPL, OP, VOUT, SC, S - 1>(c);
+  }
+}
+
 template <typename T, int N, int TPL, int OP, bool VIN, bool VOUT, bool DIRECT_OUT,
           typename SC, int S, bool FLAT, bool SHUF = false>
 __device__ __forceinline__ void fstage(const FCtx<T> &c) {
@@ -275,6 +365,8 @@ __device__ __forceinline__ void fstage(const FCtx<T> &c) {
     if (Q * TPL == NR || j < NR) {
       if constexpr (SHUF) {
         c2r_load_shuffled<T, N, TPL, R, VIN>(c, v[q]);
+      } else if (FIRST && !FLAT && OP == OP_PASSA && c.valid && (a.sub & SUB_CHIRP)) {
+        chirp_load<T, R, NR, VIN>(c, j, v[q]);
       } else {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -296,7 +388,50 @@ __device__ __forceinline__ void fstage(const FCtx<T> &c) {
       dft<R>(v[q], dir);
     }
   }
-  if constexpr (LAST && DIRECT_OUT && OP == OP_R2C_EVEN) {
+  if constexpr (LAST && OP == OP_BLUEROW) {
+    // bins j + r NS are in registers, the inputs of the inverse transform's
+    // first butterflies when its stages run backwards: the kernel product
+    // needs no exchange, and both transforms together take 2 (S - 1)
+    static_assert(NR == NS || N == R, "the last stage's bins");
+    const bool cj = (a.sub & SUB_CONJ) != 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int j = c.i + q * TPL;
+      if (Q * TPL == NR || j < NR) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const C2<T> w = a.t2[int64_t(c.aux) * N + j + r * NS];
+          v[q][r] = cmul(v[q][r], cj ? conjc(w) : w);
+        }
+        dft<R>(v[q], -dir);
+        if constexpr (FIRST) {
+          if (c.valid) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+              fstore<T, OP, VOUT>(a, c.twl, c.gout, c.aux, j + r * NR, v[q][r]);
+          }
+        } else {
+          const C2<T> *tw = a.tw + a.f.st[S].twoff;
+#pragma unroll
+          for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], dirw(tw[(r - 1) * NS + j], -dir));
+        }
+      }
+    }
+    if constexpr (!FIRST) {
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int j = c.i + q * TPL;
+        if (Q * TPL == NR || j < NR) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) c.line[padi<T>(j + r * NR)] = v[q][r];
+        }
+      }
+      __syncthreads();
+      funstage<T, N, TPL, OP, VOUT, SC, S - 1>(c);
+    }
+    return;
+  } else if constexpr (LAST && DIRECT_OUT && OP == OP_R2C_EVEN) {
     static_assert(Q * TPL == NR && NR == NS, "r2c from registers needs full butterflies");
     r2c_store_shuffled<T, N, TPL, Q, R, VOUT>(c, v);
     return;
@@ -306,9 +441,13 @@ __device__ __forceinline__ void fstage(const FCtx<T> &c) {
       for (int q = 0; q < Q; ++q) {
         const int j = c.i + q * TPL;
         if (Q * TPL == NR || j < NR) {
+          if (OP == OP_PASSA && (a.sub & SUB_FINAL)) {
+            chirp_store<T, R, NS, VOUT>(c, j, v[q]);
+          } else {
 #pragma unroll
-          for (int r = 0; r < R; ++r)
-            fstore<T, OP, VOUT>(a, c.twl, c.gout, c.aux, j + r * NS, v[q][r]);
+            for (int r = 0; r < R; ++r)
+              fstore<T, OP, VOUT>(a, c.twl, c.gout, c.aux, j + r * NS, v[q][r]);
+          }
         }
       }
     }
@@ -390,7 +529,9 @@ __device__ __forceinline__ void fstage_split(
   for (int q = 0; q < Q; ++q) {
     const int j = c.i + q * TPL;
     if (Q * TPL == NR || j < NR) {
-      if constexpr (FIRST) {
+      if (FIRST && OP == OP_PASSA && c.valid && (a.sub & SUB_CHIRP)) {
+        chirp_load<T, R, NR, VIN>(c, j, v[q]);
+      } else if constexpr (FIRST) {
 #pragma unroll
         for (int r = 0; r < R; ++r)
           v[q][r] = c.valid ? fload<T, OP, VIN>(c, j + r * NR) : C2<T>{T(0), T(0)};
@@ -410,9 +551,13 @@ __device__ __forceinline__ void fstage_split(
       for (int q = 0; q < Q; ++q) {
         const int j = c.i + q * TPL;
         if (Q * TPL == NR || j < NR) {
+          if (OP == OP_PASSA && (a.sub & SUB_FINAL)) {
+            chirp_store<T, R, NS, VOUT>(c, j, v[q]);
+          } else {
 #pragma unroll
-          for (int r = 0; r < R; ++r)
-            fstore<T, OP, VOUT>(a, c.twl, c.gout, c.aux, j + r * NS, v[q][r]);
+            for (int r = 0; r < R; ++r)
+              fstore<T, OP, VOUT>(a, c.twl, c.gout, c.aux, j + r * NS, v[q][r]);
+          }
         }
       }
     }
@@ -539,21 +684,10 @@ __global__ void __launch_bounds__(TPL *LPB, SPLIT ? 4 : 1) k_fast(const LineArgs
     }
   }
   if constexpr (OP == OP_BLUEROW) {
-    // Bluestein rows: forward FFT (global -> natural order in LDS), times
-    // the kernel t2 at m = aux + k other, inverse FFT out of LDS, stored in
+    // Bluestein rows: forward FFT, times the kernel, inverse FFT, stored in
     // place with the inverse four-step twiddle; every load of a line comes
     // before the barriers that precede its stores
-    fstage<T, N, TPL, OP, VIN, VOUT, false, SC, 0, false>(c);
-    if (c.valid) {
-      const bool cj = (a.sub & SUB_CONJ) != 0;
-      for (int k = i; k < N; k += TPL) {
-        const C2<T> w = a.t2[aux + int64_t(k) * a.other];
-        c.line[padi<T>(k)] = cmul(c.line[padi<T>(k)], cj ? conjc(w) : w);
-      }
-    }
-    __syncthreads();
-    c.dir = -a.dir;
-    fstage<T, N, TPL, OP, VIN, VOUT, true, SC, 0, true>(c);
+    fstage<T, N, TPL, OP, VIN, VOUT, true, SC, 0, false>(c);
     return;
   }
   if constexpr (FLAT) {

@@ -317,11 +317,10 @@ __device__ __forceinline__ void kernel_product(const LineArgs<T> &a, const MixCt
                                                int ns, C2<T> *v) {
   const T cs = (a.sub & SUB_CONJ) != 0 ? T(-1) : T(1);
   const bool row = op_of<OP>(a) == OP_BLUEROW;
-  const C2<T> *kp = row ? a.t2 + c.aux : a.t1;
-  const int64_t ks = row ? a.other : 1;
+  const C2<T> *kp = row ? a.t2 + int64_t(c.aux) * a.f.n : a.t1;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    C2<T> w = kp[(j + r * ns) * ks];
+    C2<T> w = kp[j + r * ns];
     w.y *= cs;
     const C2<T> y = cmul(v[r], w);
     v[r] = C2<T>{y.y, y.x};

@@ -521,8 +521,13 @@ static void make_multi(PlanRec &p, uint64_t N, uint64_t n1) {
 // So when the padded length needs two passes the GPU uses n1 * m with n1 a
 // power of two (the column passes on the specialised kernel) and
 // m = good_size(ceil((2n - 2) / n1)), if that is at most 6% longer than the
-// reference's length; among equal lengths the larger n1 wins (shorter rows on
-// the generic kernel).  For n = 2^k + 1 (65537) this is exactly 2^(k+1).
+// reference's length; among equal lengths the smallest n1 wins: a tile of 16
+// columns of 256 takes 35 KB of LDS, four to a CU, one of 1024 the whole CU,
+// whose loads, stages and stores then take turns, and rows shorter than a wave
+// idle lanes (us with columns of 1024 / 512 / 256 first: 256 x 65537 c64 431 / 431
+// / 416, 92 x 10037 c64 55 / 49 / 43, 100 x 32749 c64 101 / 99 / 87, 100 x 12289
+// c128 98 / 84 / 77; 64 x 50021 c64 110 / 106 / 111).  For n = 2^k + 1 (65537)
+// the length is exactly 2^(k+1).
 // Returns n1 (0: keep the reference length).
 static uint64_t pick_blue_pow2(uint64_t n, uint64_t ref_n2, bool dbl, size_t budget,
                                uint64_t *gpu_n2) {
@@ -531,7 +536,7 @@ static uint64_t pick_blue_pow2(uint64_t n, uint64_t ref_n2, bool dbl, size_t bud
                                                                  : std::min(budget, kSplitBudget));
   const uint64_t need = 2 * n - 2;
   uint64_t best_n1 = 0, best = 0;
-  for (uint64_t n1 : {uint64_t(1024), uint64_t(512), uint64_t(256)}) {
+  for (uint64_t n1 : {uint64_t(256), uint64_t(512), uint64_t(1024)}) {
     if (n1 > lim || !fast_interleaved_ok(n1, dbl)) continue;
     const uint64_t m = good_size_cmplx((need + n1 - 1) / n1);
     if (m < 2 || m > lim) continue;
@@ -648,7 +653,14 @@ static std::shared_ptr<C2CPlan> materialize(const PlanRec &r) {
   }
   if (r.bn2) {
     upload_any(p->bk, r.bk, r.dbl);
-    upload_any(p->bkf, r.bkf, r.dbl);
+    if (r.kind == kBlueTwoPass) {  // by rows, as the row pass reads it: bin k1 + n1 k2 at k1 n2 + k2
+      std::vector<std::complex<double>> rows(r.bkf.size());
+      for (uint64_t k1 = 0; k1 < r.n1; ++k1)
+        for (uint64_t k2 = 0; k2 < r.n2; ++k2) rows[k1 * r.n2 + k2] = r.bkf[k1 + r.n1 * k2];
+      upload_any(p->bkf, rows, r.dbl);
+    } else {
+      upload_any(p->bkf, r.bkf, r.dbl);
+    }
     p->bn2 = r.bn2;
   }
   if (r.sub_n) p->sub = get_c2c_plan_any(r.sub_n, r.dbl, r.budget, r.sub_inter);

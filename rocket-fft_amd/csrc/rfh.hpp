@@ -107,7 +107,7 @@ struct C2CPlan {
   DevBuf big_lo, big_hi; // W_N^e = lo[e & mask] * hi[e >> shift]  (forward sign)
   int shift = 0;
   uint64_t bn2 = 0;      // Bluestein length (0 = none)
-  DevBuf bk, bkf;        // chirp e^{+i pi m^2/n} (n) and DFT(chirp)/bn2 (bn2)
+  DevBuf bk, bkf;        // chirp e^{+i pi m^2/n} (n) and DFT(chirp)/bn2 (bn2; two passes: by rows)
   std::shared_ptr<const C2CPlan> sub;  // kMultiPass: rows of M = n2; kBlueMulti: length bn2
   size_t budget = 0;     // dynamic LDS the plan's passes may use per workgroup
 };
