@@ -210,11 +210,14 @@ MixGeom mix_geometry(const Desc &f, const int *pbo, bool dbl, int64_t nlines, bo
     if (L > 1) ld += ((slot - ld) % G + G) % G;
   } else if (m.T <= 128) {
     // groups of about 256 threads; among the sizes up to 512 threads the
-    // first that leaves under a tenth of its last wave's lanes idle
+    // first that leaves under a tenth of its last wave's lanes idle.  Groups
+    // of 5 to 7 waves fill the four SIMDs unevenly: lines of 1000 (100
+    // threads) in threes / fives, 65536 of them c64 263 / 240 us, 32000 c128
+    // 297 / 250; of 600 (40 threads) in eights / sixes 16000 c64 41.6 / 36.5
     double best = 0;
     for (int l = std::max(1, 192 / m.T); l * m.T <= 512 && l <= kMixLines; ++l) {
-      const int t = l * m.T;
-      const double use = double(t) / double((t + 63) / 64 * 64);
+      const int t = l * m.T, waves = (t + 63) / 64;
+      const double use = double(t) / double(64 * waves) * (waves > 4 && waves < 8 ? 0.9 : 1.0);
       if (use > best + 0.02) {
         best = use;
         L = l;
