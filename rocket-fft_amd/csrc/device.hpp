@@ -362,12 +362,11 @@ __device__ __forceinline__ C2<T> pre_elem(int mode, const T *x, int64_t es, I n,
       // a = x (DCT-III) or x reversed (DST-III), a_n = 0, ortho scales x_0 by
       // sqrt 2; V_j = (a_j - i a_{n-j}) e^{i pi j/2n} and the inverse FFT of
       // length n holds the even outputs up and the odd outputs down
-      auto at = [&](I q) -> T {
-        if (q >= n) return T(0);
-        const I src = mode == kPreDct3N ? q : n - 1 - q;
+      auto at = [&](I q) -> T {  // (the load has no condition around it)
+        const I qc = q < n ? q : n - 1, src = mode == kPreDct3N ? qc : n - 1 - qc;
         T xv = x[src * es];
         if (ortho && src == 0) xv *= sqrt2;
-        return xv;
+        return q < n ? xv : T(0);
       };
       v = cmul(C2<T>{at(j), -at(n - j)}, root(2 * j));
       break;

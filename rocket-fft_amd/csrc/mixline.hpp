@@ -29,6 +29,8 @@
 // inverse transform needs no tables of its own: S - 1 exchanges each way.
 #pragma once
 
+#include <type_traits>
+
 #include "butterfly.hpp"
 #include "mixgeom.hpp"
 
@@ -64,6 +66,17 @@ struct MixCtx {
   int aux;      // index along the line set's auxdim (four-step row / column)
   int j;        // place in the line
   bool ok;      // the line exists and the thread has a place in it
+  bool line;    // ... the line exists (a line alone in its group: for every thread)
+};
+
+// How the threads walk a line element by element: a line alone in its group
+// takes all of the group's threads, also those without a place in the stages.
+template <typename T>
+struct Walk {
+  int step;
+  bool on;
+  __device__ __forceinline__ Walk(const MixGeom &m, const MixCtx<T> &c)
+      : step(m.L == 1 ? int(blockDim.x) : m.T), on(m.L == 1 ? c.line : c.ok) {}
 };
 
 template <typename T>
@@ -461,21 +474,63 @@ __device__ __forceinline__ void mix_unstage(const LineArgs<T> &a, const MixGeom 
   __syncthreads();
 }
 
+// Real-to-real modes: f(mode) with the mode a compile-time constant for the
+// DCT / DST types, so that the elements of a batch are in one stretch of code
+// and their loads in flight together.
+template <typename F>
+__device__ __forceinline__ void with_pre_mode(int mode, F &&f) {
+  switch (mode) {
+#define RFH_MODE(M) \
+  case M: f(std::integral_constant<int, M>{}); break;
+    RFH_MODE(kPreDct1) RFH_MODE(kPreDst1) RFH_MODE(kPreType4) RFH_MODE(kPreDct2N)
+    RFH_MODE(kPreDst2N) RFH_MODE(kPreDct3N) RFH_MODE(kPreDst3N)
+    default: f(mode);
+  }
+}
+template <typename F>
+__device__ __forceinline__ void with_post_mode(int mode, F &&f) {
+  switch (mode) {
+    RFH_MODE(kPostDct1) RFH_MODE(kPostDst1) RFH_MODE(kPostDct4) RFH_MODE(kPostDst4)
+    RFH_MODE(kPostDct2N) RFH_MODE(kPostDst2N) RFH_MODE(kPostDct3N) RFH_MODE(kPostDst3N)
+#undef RFH_MODE
+    default: f(mode);
+  }
+}
+
 // The whole line to LDS, in order (with the batch executor's operations
-// kLineBatch loads of a thread in flight).
+// and the real-to-real ones kLineBatch loads of a thread in flight).
 constexpr int kLineBatch = 8;
 template <typename T, int OP>
 __device__ __forceinline__ void load_line(const LineArgs<T> &a, const MixGeom &m,
                                           const MixCtx<T> &c) {
-  constexpr int U = OP == OP_ANY ? kLineBatch : 1;
-  if (c.ok)
-    for (int e = c.j; e < a.f.n; e += U * m.T) {
-      C2<T> v[U];
-      op_load<T, OP, U, (U > 1)>(a, c, e, m.T, v);
+  const Walk<T> w(m, c);
+  if constexpr (OP == OP_R2R) {
+    if (w.on)
+      with_pre_mode(a.sub & 0xff, [&](auto mode) {
+        for (int e = c.j; e < a.f.n; e += kLineBatch * w.step) {
+          C2<T> v[kLineBatch];
 #pragma unroll
-      for (int r = 0; r < U; ++r)
-        if (e + r * m.T < a.f.n) c.ln[e + r * m.T] = v[r];
-    }
+          for (int r = 0; r < kLineBatch; ++r)
+            v[r] = pre_elem<T, int>(mode, c.in, a.esi, int(a.bign), a.f.n,
+                                    min(e + r * w.step, a.f.n - 1), (a.sub & R2R_ORTHO) != 0,
+                                    (a.sub & R2R_CONJ) != 0, (a.sub & R2R_FLIP) != 0,
+                                    TableRoot<T>{a.t0});
+#pragma unroll
+          for (int r = 0; r < kLineBatch; ++r)
+            if (e + r * w.step < a.f.n) c.ln[e + r * w.step] = swapri(v[r], a.dir > T(0));
+        }
+      });
+  } else {
+    constexpr int U = OP == OP_ANY ? kLineBatch : 1;
+    if (w.on)
+      for (int e = c.j; e < a.f.n; e += U * w.step) {
+        C2<T> v[U];
+        op_load<T, OP, U, (U > 1)>(a, c, e, w.step, v);
+#pragma unroll
+        for (int r = 0; r < U; ++r)
+          if (e + r * w.step < a.f.n) c.ln[e + r * w.step] = v[r];
+      }
+  }
   __syncthreads();
 }
 
@@ -483,12 +538,13 @@ __device__ __forceinline__ void load_line(const LineArgs<T> &a, const MixGeom &m
 template <typename T, int OP>
 __device__ __forceinline__ void store_line(const LineArgs<T> &a, const MixGeom &m,
                                            const MixCtx<T> &c) {
-  if (c.ok)
-    for (int e = c.j; e < a.f.n; e += kLineBatch * m.T) {
+  const Walk<T> w(m, c);
+  if (w.on)
+    for (int e = c.j; e < a.f.n; e += kLineBatch * w.step) {
       C2<T> v[kLineBatch];
 #pragma unroll
-      for (int r = 0; r < kLineBatch; ++r) v[r] = c.ln[min(e + r * m.T, a.f.n - 1)];
-      op_store<T, OP, kLineBatch, true>(a, c, e, m.T, v);
+      for (int r = 0; r < kLineBatch; ++r) v[r] = c.ln[min(e + r * w.step, a.f.n - 1)];
+      op_store<T, OP, kLineBatch, true>(a, c, e, w.step, v);
     }
 }
 
@@ -580,19 +636,20 @@ __device__ __forceinline__ MixCtx<T> mix_place(const LineArgs<T> &a, const MixGe
     l = t & (m.L - 1);
     j = t >> m.log2L;
   } else {
-    l = fdiv(t, m.T, m.invT);
+    l = m.L == 1 ? 0 : fdiv(t, m.T, m.invT);
     j = t - l * m.T;
   }
   MixCtx<T> c;
   const int64_t b = tile * m.L + l;
-  c.ok = l < m.L && j < m.T && b < a.nlines;
-  const LineOffsets o = c.ok ? line_offsets(b, a.nb, a.bdim, a.bsi, a.bso, a.auxdim)
+  c.line = l < m.L && b < a.nlines;
+  c.ok = c.line && j < m.T;
+  const LineOffsets o = c.line ? line_offsets(b, a.nb, a.bdim, a.bsi, a.bso, a.auxdim)
                              : LineOffsets{0, 0, 0};
   c.in = a.in + o.oi;
   c.out = a.out + o.oo;
   c.aux = o.aux;
   c.j = j;
-  c.ln = lds + (c.ok ? l : 0) * m.ld;
+  c.ln = lds + (c.line ? l : 0) * m.ld;
   return c;
 }
 
@@ -674,10 +731,11 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
   if constexpr (OP == OP_ANY)
     if (m.nst && elem_store(op)) store_line<T, OP>(a, m, c);
   if (op == OP_R2C_EVEN) {  // bins k and h - k of the half-length spectrum
-    if (c.ok) {
+    const Walk<T> w(m, c);
+    if (w.on) {
       const int h = a.f.n;
       const bool cj = (a.sub & SUB_CONJ) != 0;
-      for (int k = c.j; k <= h; k += m.T) {
+      for (int k = c.j; k <= h; k += w.step) {
         C2<T> X;
         if (k == 0 || k == h) {
           const C2<T> z = c.ln[0];
@@ -694,13 +752,23 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
     }
   }
   if constexpr (OP == OP_R2R) {
-    if (c.ok) {
+    const Walk<T> w(m, c);
+    if (w.on) {
       const C2<T> *ln = c.ln;
-      for (int k = c.j; k < a.nout; k += m.T)
-        c.out[k * a.eso] =
-            a.fct * post_elem<T, int>((a.sub >> 8) & 0xff, [&](int q) { return ln[q]; },
-                                      int(a.bign), k, (a.sub & R2R_ORTHO) != 0,
-                                      (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0});
+      with_post_mode((a.sub >> 8) & 0xff, [&](auto mode) {
+        for (int k = c.j; k < a.nout; k += kLineBatch * w.step) {
+          T y[kLineBatch];
+#pragma unroll
+          for (int r = 0; r < kLineBatch; ++r)
+            y[r] = a.fct * post_elem<T, int>(mode, [&](int q) { return ln[q]; }, int(a.bign),
+                                             min(k + r * w.step, a.nout - 1),
+                                             (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_FLIP) != 0,
+                                             TableRoot<T>{a.t0});
+#pragma unroll
+          for (int r = 0; r < kLineBatch; ++r)
+            if (k + r * w.step < a.nout) c.out[(k + r * w.step) * a.eso] = y[r];
+        }
+      });
     }
   }
 }
