@@ -232,9 +232,22 @@ struct AxisPlan {
 // 16384 complex64 16.2 -> 16.2 / 18.5 -> 17.6 / 492 -> 354.
 constexpr int64_t kWholeLines = 32;
 
-// LDS budget of the plan for a line set (0: the ordinary one).
-size_t axis_budget(uint64_t n, bool dbl, bool inter, int64_t nlines) {
-  return !inter && nlines >= kWholeLines && whole_line_only(n, dbl) ? whole_line_budget() : 0;
+// The cached plan for a line set, or null: the one for its number of lines,
+// else the other of the two.
+std::shared_ptr<C2CPlan> find_lines_plan(uint64_t n, bool dbl, bool inter, int64_t nlines) {
+  if (inter || !whole_line_only(n, dbl)) return find_c2c_plan(n, dbl, 0, inter);
+  const bool whole = nlines >= kWholeLines;
+  auto p = find_c2c_plan(n, dbl, whole ? whole_line_budget() : 0, false);
+  return p ? p : find_c2c_plan(n, dbl, whole ? 0 : whole_line_budget(), false);
+}
+
+// ... built when missing; a call that is being captured, which cannot build
+// one, takes whichever of the two there is.
+std::shared_ptr<C2CPlan> lines_plan(const Ctx &c, uint64_t n, bool inter, int64_t nlines) {
+  if (c.ws->capturing)
+    if (auto p = find_lines_plan(n, c.dbl, inter, nlines)) return p;
+  const bool whole = !inter && nlines >= kWholeLines && whole_line_only(n, c.dbl);
+  return get_c2c_plan(n, c.dbl, whole ? whole_line_budget() : 0, inter);
 }
 
 AxisPlan c2c_axis_plan(Ctx &c, const int64_t *shape, int nd, int ax, const int64_t *si,
@@ -248,7 +261,7 @@ AxisPlan c2c_axis_plan(Ctx &c, const int64_t *shape, int nd, int ax, const int64
   for (int d = 0; d < r.g.nb; ++d)
     inter = inter || std::llabs(r.g.bsi[d]) < std::llabs(r.g.esi) ||
             std::llabs(r.g.bso[d]) < std::llabs(r.g.eso);
-  r.plan = get_c2c_plan(n, c.dbl, axis_budget(n, c.dbl, inter, r.g.nlines), inter);
+  r.plan = lines_plan(c, n, inter, r.g.nlines);
   return r;
 }
 
@@ -273,7 +286,7 @@ void *complex_work(Ctx &c, int64_t nlines, int64_t m) {
 }
 
 void c2c_work(Ctx &c, void *work, int64_t nlines, int64_t m, bool forward) {
-  auto plan = get_c2c_plan(uint64_t(m), c.dbl, axis_budget(uint64_t(m), c.dbl, false, nlines));
+  auto plan = lines_plan(c, uint64_t(m), false, nlines);
   LineSet g = contiguous_lines(work, nlines, m);
   void *tmp = c.ws->get(kSlotTwoPass, c2c_tmp_bytes(*plan, g));
   launch_c2c(*plan, g, forward ? -1 : +1, 1.0, c.s, tmp);
@@ -846,7 +859,7 @@ void c2c_noalloc(uint64_t ndim, const arystruct_t *ain, arystruct_t *aout, aryst
       inter = inter || std::llabs(g.bsi[d]) < std::llabs(g.esi) ||
               std::llabs(g.bso[d]) < std::llabs(g.eso);
     const uint64_t n = uint64_t(in.shape[a]);
-    auto plan = find_c2c_plan(n, dbl, axis_budget(n, dbl, inter, g.nlines), inter);
+    auto plan = find_lines_plan(n, dbl, inter, g.nlines);
     if (!plan)
       RFH_THROW(3, "no plan on this GPU yet for length " + std::to_string(n) +
                        (dbl ? " complex128" : " complex64") +

@@ -70,3 +70,36 @@ def test_whole_lines_rolled(n, dtype):
         assert R.c2c_shifted(t, got, np.array([1]), True, 1.0, [si], [so])
         R.c2c(torch.roll(t, si, 1), plain, np.array([1]), True, 1.0)
         assert torch.equal(got, torch.roll(plain, so, 1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first,then", [(33, 3), (3, 33)])
+def test_whole_lines_captured_with_the_other_plan(first, then):
+    """A length warmed with few lines is captured with many, and the other way
+    round: a capture builds no plan, it takes the one there is."""
+    import torch
+    n = {33: 12000, 3: 12500}[first]  # lengths of its own: no plan of either kind yet
+    g = torch.Generator(device="cuda").manual_seed(n)
+    big = torch.randn((64, 1 << 16), dtype=torch.complex64, device="cuda", generator=g)
+    x = torch.randn((then, n), dtype=torch.complex64, device="cuda", generator=g)
+    y = torch.zeros_like(x)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        R.c2c(big, big, np.array([1]), True, 1.0)  # the stream's workspace
+        w = torch.randn((first, n), dtype=torch.complex64, device="cuda")
+        R.c2c(w, w, np.array([1]), True, 1.0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        R.c2c(x, y, np.array([1]), True, 1.0)
+    want = np.fft.fft(x.cpu().numpy().astype(np.complex128), axis=1)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(y.cpu().numpy(), want) <= 1e-6
+    z = torch.zeros_like(x)
+    R.c2c_noalloc(x, z, np.array([1]), True, 1.0)
+    torch.cuda.synchronize()
+    assert torch.equal(z, y)
