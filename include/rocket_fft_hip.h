@@ -216,15 +216,15 @@ int rfh_mfma_probe(int bf16, const float *a, const float *b, float *d, void *str
 
 /* ---- ragged batches ---------------------------------------------------------
  * Many independent transforms of uneven lengths and kinds (complex c2c, real
- * r2c / c2r), planned once and executed in one persistent launch (a job
- * queue drained by resident workgroups, largest job first).  No reference
+ * r2c / c2r), planned once and executed in a few launches (one
+ * workgroup per group of lines, the longest first).  No reference
  * counterpart: rocket-fft calls its engine once per array.  Each job is one
  * contiguous line in device memory; fct, forward and the r2c/c2r
  * conjugation rules mean what they mean in numba_c2c / numba_r2c /
  * numba_c2r.  Execution allocates nothing and can be captured in a HIP
  * graph; the buffers named at creation are the ones every execution uses.
- * autotune = true times LDS budgets and grid sizes on the batch and keeps
- * the fastest (remembered per batch signature for the process). */
+ * autotune = true times LDS budgets on the batch and keeps the fastest
+ * (remembered per batch signature for the process). */
 enum { RFH_JOB_C2C = 0, RFH_JOB_R2C = 1, RFH_JOB_C2R = 2 };
 typedef struct {
     int32_t kind;     /* RFH_JOB_* */
@@ -238,7 +238,7 @@ int rfh_batch_create(const rfh_job_t *jobs, int64_t njobs, bool double_precision
                      bool autotune, void *stream, void **handle);
 int rfh_batch_execute(void *handle, void *stream);
 /* The same jobs launched one transform at a time through the per-call
- * engine (the comparison point of the persistent launch). */
+ * engine (the comparison point of the batched launches). */
 int rfh_batch_execute_serial(void *handle, void *stream);
 /* autotuned: 0 = not tuned, 1 = timed by this call, 2 = result remembered by
  * this process, 3 = read from the cache directory. */

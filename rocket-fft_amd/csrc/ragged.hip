@@ -676,7 +676,7 @@ void autotune(Batch &bt, hipStream_t s) {
   }
 }
 
-// device or managed memory (the persistent kernel dereferences job pointers
+// device or managed memory (the kernel dereferences job pointers
 // directly; host memory would fault)
 bool device_memory(const void *p) {
   if (!p) return false;

@@ -601,7 +601,8 @@ JOB_KINDS = {"c2c": 0, "r2c": 1, "c2r": 2}
 
 class RaggedBatch:
     """Many independent transforms of uneven lengths and kinds, planned once
-    and run in one persistent launch (``rfh_batch_*`` in the C ABI).
+    and run in a few launches, one per level of passes and workgroup size
+    (``rfh_batch_*`` in the C ABI).
 
     jobs: iterable of (kind, forward, n, inp, out, fct) with kind in
     {"c2c", "r2c", "c2r"}, n the transform length (the real length for
@@ -673,7 +674,7 @@ class RaggedBatch:
             raise RuntimeError(f"{fname}: " + last_error()[1])
 
     def execute(self):
-        """One persistent launch over all jobs, on torch's current stream."""
+        """All jobs in the batch's few launches, on torch's current stream."""
         self._run("rfh_batch_execute")
 
     def execute_serial(self):
