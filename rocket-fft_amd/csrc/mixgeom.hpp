@@ -18,6 +18,15 @@ constexpr int kMixLines = 256;  // lines per group, at most
 // one wave on every SIMD (256 CUs of four)
 constexpr int64_t kFillThreads = 256 * 4 * 64;
 
+// A launch's threads are counted in 31 bits: line sets of more groups run in
+// several launches.  f(first group, groups) for each.
+constexpr int64_t kLaunchThreads = 0x7fffffff;
+template <typename F>
+void for_launches(int64_t groups, int threads, F &&f) {
+  const int64_t most = kLaunchThreads / threads;
+  for (int64_t g = 0; g < groups; g += most) f(g, std::min(most, groups - g));
+}
+
 constexpr int kMixStages = 10;
 
 struct MixStage {

@@ -14,9 +14,9 @@ namespace rfh {
 
 template <typename T, int OP>
 __global__ void __launch_bounds__(dev::kMixThreads<T>)
-    k_lines(const dev::LineArgs<T> a, const MixGeom m) {
+    k_lines(const dev::LineArgs<T> a, const MixGeom m, int64_t tile0) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  dev::mix_body<T, OP>(a, m, int64_t(dev::xcd_tile()), smem_raw);
+  dev::mix_body<T, OP>(a, m, tile0 + int64_t(dev::xcd_tile()), smem_raw);
 }
 
 template <typename T, int OP>
@@ -24,7 +24,6 @@ void launch_mix_op(const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s) {
   const size_t lds = size_t(m.L * m.ld + m.ngen) * 2 * sizeof(T);
   const int64_t groups = (a.nlines + m.L - 1) / m.L;
   const int threads = (m.L * m.T + 63) / 64 * 64;
-  if (groups > 0x7fffffff / dev::kMixThreads<T>) RFH_THROW(3, "batch too large for one launch");
   if (threads > dev::kMixThreads<T> || lds > lds_limit())
     RFH_THROW(3, "line group of " + std::to_string(a.f.n) + " needs " + std::to_string(threads) +
                      " threads and " + std::to_string(lds) + " B of LDS");
@@ -41,13 +40,15 @@ void launch_mix_op(const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s) {
       done.insert(dev);
     }
   }
-  hipLaunchKernelGGL((k_lines<T, OP>), dim3(unsigned(groups)), dim3(unsigned(threads)), lds, s, a,
-                     m);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess)
-    RFH_THROW(2, std::string("line kernel launch (") + std::to_string(groups) + " groups, " +
-                     std::to_string(lds) + " B LDS, op " + std::to_string(OP) +
-                     "): " + hipGetErrorString(e));
+  for_launches(groups, threads, [&](int64_t first, int64_t count) {
+    hipLaunchKernelGGL((k_lines<T, OP>), dim3(unsigned(count)), dim3(unsigned(threads)), lds, s,
+                       a, m, first);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+      RFH_THROW(2, std::string("line kernel launch (") + std::to_string(count) + " groups, " +
+                       std::to_string(lds) + " B LDS, op " + std::to_string(OP) +
+                       "): " + hipGetErrorString(e));
+  });
 }
 
 }  // namespace rfh
