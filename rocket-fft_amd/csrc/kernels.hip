@@ -92,8 +92,8 @@ LineArgs<T> make_line_args(const PassSpec &ps, const LineSet &g) {
 
 template <typename T>
 MixGeom make_mix_geom(const PassSpec &ps, const LineArgs<T> &a) {
-  MixGeom m = mix_geometry(a.f, ps.d->pbo, sizeof(T) == 8, a.nlines, a.lfast_in || a.lfast_out,
-                           ps.lines, lds_limit());
+  MixGeom m = line_geometry(a.f, ps.d->pbo, sizeof(T) == 8, a.nlines, a.lfast_in || a.lfast_out,
+                            ps.lines, lds_limit());
   if (m.L == 0) RFH_THROW(3, "line does not fit in LDS");
   // A line of at most 8 threads: its loads and stores by place would touch one
   // cache line per 8 lanes or fewer, so the group's lines move as one run of

@@ -242,4 +242,22 @@ MixGeom mix_geometry(const Desc &f, const int *pbo, bool dbl, int64_t nlines, bo
   return m;
 }
 
+// ... of a call's lines.  Interleaved lines of few threads: adjacent lines
+// until they fill a wave; 128-byte rows alone leave a wave of 16 (complex128:
+// 8) lines of up to 17 elements with as many live lanes.  us for 4M complex64
+// / 2M complex128 elements along axis 0, 128-byte rows / one wave / four: n = 3
+// 46.8 / 26.6 / 28.9 and 64.3 / 17.4 / 19.1, n = 12 21.6 / 16.7 / 17.6 and 29.0
+// / 15.2 / 15.8, n = 24 21.8 / 18.4 / 19.1 and 24.8 / 18.4 / 18.6, n = 61 39.0
+// / 38.6 / 54.3 and 60.4 / 38.0 / 57.9.
+template <typename Desc>
+MixGeom line_geometry(const Desc &f, const int *pbo, bool dbl, int64_t nlines, bool inter, int want,
+                      size_t lds_bytes) {
+  MixGeom m = mix_geometry(f, pbo, dbl, nlines, inter, want, lds_bytes);
+  if (!inter || !m.L) return m;
+  const int base = want ? want : (dbl ? 8 : 16);
+  want = base;
+  while (want * 2 * m.T <= 64) want *= 2;
+  return want == base ? m : mix_geometry(f, pbo, dbl, nlines, inter, want, lds_bytes);
+}
+
 }  // namespace rfh

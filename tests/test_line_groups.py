@@ -1,0 +1,85 @@
+"""Groups of short lines.  Host: an interleaved group of short lines fills more
+than half of its waves' lanes and stays inside the workgroup and its LDS, at
+every length to 100.  GPU: short lengths along axis 0 with enough lines for
+whole waves, the last group a part of one, against numpy in FP64, forward and
+inverse, complex, real and back.  Bar: rel-L2 <= 1e-6 / 1e-13."""
+import subprocess
+import textwrap
+
+import numpy as np
+import pytest
+
+import rocket_fft_amd as R
+from helpers import RTYPE, rel_l2, tol_of
+from test_mix_geometry import CSRC
+
+DRIVER = textwrap.dedent(r"""
+    #include <cstdio>
+    #include "mixgeom.hpp"
+    using namespace rfh;
+    struct St { int radix, ns, twoff, genoff; };
+    struct Desc { int n, nst; St st[24]; };
+
+    int main() {
+      for (int dbl = 0; dbl < 2; ++dbl)
+        for (int n = 1; n <= 100; ++n)
+          for (int want : {0, 4, 16})
+            for (int64_t lines : {int64_t(5), int64_t(3000), int64_t(1) << 20}) {
+              const std::vector<int> rad = mix_radices(uint64_t(n));
+              Desc f{};
+              f.n = n;
+              int pbo[24] = {}, ns = 1, gen = 0;
+              for (int R : rad) {
+                f.st[f.nst] = St{R, ns, 0, gen};
+                if (R > 17) gen += R;
+                pbo[f.nst++] = block_pitch(ns * R, ns, dbl);
+                ns *= R;
+              }
+              const MixGeom m = line_geometry(f, pbo, dbl, lines, true, want, 160 * 1024);
+              const int t = m.L * m.T, lanes = (t + 63) / 64 * 64;
+              bool ok = m.L >= 2 && m.L == 1 << m.log2L && m.L <= kMixLines && t <= mix_max_threads(dbl);
+              ok = ok && size_t(m.L * m.ld + m.ngen) * (dbl ? 16 : 8) <= 160 * 1024;
+              if (lines == 1 << 20) ok = ok && 2 * t > lanes;
+              if (!ok) {
+                std::printf("FAIL n=%d dbl=%d want=%d: %d lines of %d threads\n", n, dbl, want, m.L, m.T);
+                return 1;
+              }
+            }
+      std::printf("OK\n");
+      return 0;
+    }
+""")
+
+
+def test_short_groups_fill_their_waves(tmp_path):
+    src, exe = tmp_path / "groups.cpp", tmp_path / "groups"
+    src.write_text(DRIVER)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", f"-I{CSRC}", str(src), "-o", str(exe)],
+                   check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.strip() == "OK", r.stdout + r.stderr
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n", [2, 3, 5, 6, 9, 12, 17, 19, 24, 31, 34, 61])
+def test_short_axis_groups(n, dtype):
+    import torch
+    lines = 64 * 512 + 37
+    print(f"case axis 0 of ({n}, {lines}) {dtype.__name__}", flush=True)
+    rs = np.random.RandomState(n)
+    z = (rs.standard_normal((n, lines)) + 1j * rs.standard_normal((n, lines))).astype(dtype)
+    r = rs.standard_normal((n, lines)).astype(RTYPE[dtype])
+    t, y = torch.from_numpy(z).cuda(), torch.empty((n, lines), dtype=getattr(torch, dtype.__name__), device="cuda")
+    ax = np.array([0])
+    for fwd, f in ((True, np.fft.fft), (False, np.fft.ifft)):
+        R.c2c(t, y, ax, fwd, 1.0 if fwd else 1.0 / n)
+        assert rel_l2(y.cpu().numpy(), f(z.astype(np.complex128), axis=0)) <= tol_of(dtype)
+    half = torch.empty((n // 2 + 1, lines), dtype=y.dtype, device="cuda")
+    back = torch.from_numpy(np.zeros_like(r)).cuda()
+    R.r2c(torch.from_numpy(r).cuda(), half, ax, True, 1.0)
+    assert rel_l2(half.cpu().numpy(), np.fft.rfft(r.astype(np.float64), axis=0)) <= tol_of(dtype)
+    R.c2r(half, back, ax, False, 1.0 / n)
+    assert rel_l2(back.cpu().numpy(), r) <= 2 * tol_of(dtype)
+    R.c2c(t, t, ax, False, 1.0 / n)  # in place
+    assert torch.equal(t, y)
