@@ -54,6 +54,11 @@ struct MixGeom {
   MixStage st[kMixStages];
 };
 
+// Lines of at most one butterfly of a radix up to 9, a thread each.
+inline bool short_lines(const MixGeom &m) {
+  return m.nst == 0 || (m.nst == 1 && m.st[0].radix <= 9 && m.st[0].q == 1);
+}
+
 // Threads a line of n needs when each may hold 16 elements of a stage's
 // butterflies, and how evenly the stages use them: the sum over the stages of
 // (elements held by all threads, idle places included) / n; among equals the

@@ -343,11 +343,11 @@ __device__ __forceinline__ void kernel_product(const LineArgs<T> &a, const MixCt
 // One forward stage of radix R (first: inputs from global memory; last:
 // outputs to global memory, or for Bluestein on through the kernel product
 // into the first backward stage).
-template <typename T, int OP, int R>
+template <typename T, int OP, int R, bool SHORT = false>
 __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m,
                                           const MixStage &st, const MixCtx<T> &c, bool first,
                                           bool last) {
-  constexpr int QM = kMaxElems<T> / R > 0 ? kMaxElems<T> / R : 1;
+  constexpr int QM = !SHORT && kMaxElems<T> / R > 0 ? kMaxElems<T> / R : 1;
   const int op = op_of<OP>(a);
   const int NR = st.nr, ns = st.ns;
   const bool from_lds = !first || OP == OP_R2R || OP == OP_ANY || m.flat;
@@ -621,6 +621,7 @@ __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixG
   if (lds) __syncthreads();
 }
 
+#define RFH_SHORT_RADICES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9)
 #define RFH_MIX_RADICES(X) \
   X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17)
 
@@ -654,8 +655,9 @@ __device__ __forceinline__ MixCtx<T> mix_place(const LineArgs<T> &a, const MixGe
 }
 
 // One tile (m.L lines from line tile m.L on) of a line set.  Ends without a
-// barrier: a caller that runs several tiles puts one between them.
-template <typename T, int OP>
+// barrier: a caller that runs several tiles puts one between them.  SHORT: the
+// form for short_lines(m), without the other radices' registers.
+template <typename T, int OP, bool SHORT = false>
 __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m, int64_t tile,
                                          unsigned char *smem) {
   const int op = op_of<OP>(a);
@@ -692,9 +694,16 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
   for (int s = 0; s < m.nst; ++s) {
     const MixStage &st = m.st[s];
     const bool first = s == 0, last = s == m.nst - 1;
-    switch (st.radix) {
 #define RFH_CASE(R) \
-  case R: mix_stage<T, OP, R>(a, m, st, c, first, last); break;
+  case R: mix_stage<T, OP, R, SHORT>(a, m, st, c, first, last); break;
+    if constexpr (SHORT) {
+      switch (st.radix) {
+        RFH_SHORT_RADICES(RFH_CASE)
+        default: break;
+      }
+      break;  // a single stage
+    }
+    switch (st.radix) {
       RFH_MIX_RADICES(RFH_CASE)
 #undef RFH_CASE
       default:

@@ -83,3 +83,43 @@ def test_short_axis_groups(n, dtype):
     assert rel_l2(back.cpu().numpy(), r) <= 2 * tol_of(dtype)
     R.c2c(t, t, ax, False, 1.0 / n)  # in place
     assert torch.equal(t, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 9, 10, 12, 17, 18, 19, 24, 30, 48, 62, 96])
+def test_short_rows(n, dtype):
+    """Contiguous rows, the last group a part of one; a padded output keeps its gaps."""
+    import scipy.fft
+    import torch
+    lines, ax = 257 * 9 + 1, np.array([1])
+    print(f"case rows ({lines}, {n}) {dtype.__name__}", flush=True)
+    rs = np.random.RandomState(100 + n)
+    z = (rs.standard_normal((lines, n)) + 1j * rs.standard_normal((lines, n))).astype(dtype)
+    r = rs.standard_normal((lines, n)).astype(RTYPE[dtype])
+    t, x = torch.from_numpy(z).cuda(), torch.from_numpy(r).cuda()
+    tol = tol_of(dtype)
+    for fwd, f in ((True, np.fft.fft), (False, np.fft.ifft)):
+        wide = torch.full((lines, n + 1), 7, dtype=t.dtype, device="cuda")
+        R.c2c(t, wide[:, :n], ax, fwd, 1.0 if fwd else 1.0 / n)
+        assert rel_l2(wide[:, :n].cpu().numpy(), f(z.astype(np.complex128), axis=1)) <= tol
+        assert bool((wide[:, n] == 7).all())
+    u = t.clone()
+    R.c2c(u, u, ax, False, 1.0 / n)  # in place
+    assert torch.equal(u, wide[:, :n])
+    half = torch.full((lines, n // 2 + 2), 7, dtype=t.dtype, device="cuda")
+    R.r2c(x, half[:, :-1], ax, True, 1.0)
+    assert rel_l2(half[:, :-1].cpu().numpy(), np.fft.rfft(r.astype(np.float64), axis=1)) <= tol
+    assert bool((half[:, -1] == 7).all())
+    back = torch.full((lines, n + 1), 7, dtype=x.dtype, device="cuda")
+    R.c2r(half[:, :-1], back[:, :n], ax, False, 1.0 / n)
+    assert rel_l2(back[:, :n].cpu().numpy(), r) <= 2 * tol and bool((back[:, n] == 7).all())
+    y = torch.empty_like(x)
+    for kind in (1, 2, 3, 4):
+        if kind == 1 and n < 2:
+            continue
+        R.dct(x, y, ax, kind, 1.0, False)
+        assert rel_l2(y.cpu().numpy(), scipy.fft.dct(r.astype(np.float64), kind, axis=1)) <= tol
+    R.r2r_separable_hartley(x, y, ax, 1.0)
+    f = np.fft.fft(r.astype(np.float64), axis=1)
+    assert rel_l2(y.cpu().numpy(), f.real + f.imag) <= tol
