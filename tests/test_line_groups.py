@@ -40,6 +40,9 @@ DRIVER = textwrap.dedent(r"""
               bool ok = m.L >= 2 && m.L == 1 << m.log2L && m.L <= kMixLines && t <= mix_max_threads(dbl);
               ok = ok && size_t(m.L * m.ld + m.ngen) * (dbl ? 16 : 8) <= 160 * 1024;
               if (lines == 1 << 20) ok = ok && 2 * t > lanes;
+              // one stage: a line takes its elements and a pitch that spreads the banks
+              const int G = dbl ? 16 : 32, slot = m.L < G ? G / m.L : 1;
+              if (m.nst < 2) ok = ok && m.ld < n + 2 * slot && m.ld % (2 * slot) == slot % (2 * slot);
               if (!ok) {
                 std::printf("FAIL n=%d dbl=%d want=%d: %d lines of %d threads\n", n, dbl, want, m.L, m.T);
                 return 1;
