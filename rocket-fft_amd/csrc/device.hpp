@@ -62,7 +62,7 @@ __device__ __forceinline__ unsigned xcd_tile() {
 // q = u / d for 0 <= u < 2^22 via a float reciprocal and one correction.
 __device__ __forceinline__ int fdiv(int u, int d, float inv) {
   int q = int(float(u) * inv);
-  const int r = u - q * d;
+  const int r = u - __mul24(q, d);
   q += (r >= d) - (r < 0);
   return q;
 }

@@ -90,16 +90,42 @@ LineArgs<T> make_line_args(const PassSpec &ps, const LineSet &g) {
   return a;
 }
 
+// Whether a group's short contiguous lines move flat, one after another through
+// LDS, instead of by the places of their butterflies, which touch a cache line
+// for every few lanes.  us for 4M complex64 (2M complex128) elements, by place /
+// flat.  One thread a line: n = 12 32.4 / 20.9, 15 34.6 / 19.9 (24.6 / 18.4); a
+// lone butterfly of an odd real line is as well off by place to n = 5 (c2r 20.8
+// / 26).  Two threads: 24 25.8 / 24.9, 30 30.0 / 22.6, r2c of 48 38.4 / 27.0, of
+// 24 60.2 / 24.1.  More: a prime of 37 48.5 / 33.4, 61 49.7 / 40.6, r2c of 96
+// 36.4 / 26.9, but 48 20.6 / 24.0 (16.6 / 20.0), 77 20.4 / 24.4: such lines of
+// complex64 move flat only where they are beyond the 256 MB of the last cache
+// (64M elements of 36 302 / 255, of 60 310 / 242).
+template <typename T>
+bool flat_lines(int op, const LineArgs<T> &a, const MixGeom &m) {
+  const int64_t bi = a.nb ? a.bsi[0] : 0, bo = a.nb ? a.bso[0] : 0;
+  if (!is_flat_op(op) || a.lfast_in || a.lfast_out || a.nb > 1 || m.L < 2 || m.nst == 0 ||
+      a.esi != (real_in(op) ? 1 : 2) || a.eso != (real_out(op) ? 1 : 2) || a.rot_in || a.rot_out ||
+      std::min(bi, bo) < 0 || std::max(bi, bo) >= (1 << 20))  // (places are 24-bit products)
+    return false;
+  if (m.T == 1)
+    return a.f.n > (op == OP_R2C_ODD || op == OP_C2R_ODD || op == OP_C2R_EVEN ? 5 : 2);
+  if (m.T == 2) return true;
+  if (m.ngen) return m.T <= 8;
+  return m.T <= 4 &&
+         (op == OP_R2C_EVEN ||
+          (op == OP_C2C && sizeof(T) == 4 && a.nlines * a.f.n > (int64_t(1) << 28) / 16));
+}
+
 template <typename T>
 MixGeom make_mix_geom(const PassSpec &ps, const LineArgs<T> &a) {
   MixGeom m = line_geometry(a.f, ps.d->pbo, sizeof(T) == 8, a.nlines, a.lfast_in || a.lfast_out,
                             ps.lines, lds_limit());
   if (m.L == 0) RFH_THROW(3, "line does not fit in LDS");
-  // A line of at most 8 threads: its loads and stores by place would touch one
-  // cache line per 8 lanes or fewer, so the group's lines move as one run of
-  // elements through LDS (300000 lines of 30 complex64: 53.7 -> 46.0 us).
-  m.flat = ps.op == OP_C2C && !a.lfast_in && !a.lfast_out && m.T <= 8 && a.nb <= 1 &&
-           a.esi == 2 && a.eso == 2 && !a.rot_in && !a.rot_out;
+  m.flat = flat_lines(ps.op, a, m);
+  if (m.flat && a.nb) {
+    m.flat_in = int(a.bsi[0]);
+    m.flat_out = int(a.bso[0]);
+  }
   return m;
 }
 

@@ -49,7 +49,8 @@ struct MixGeom {
   int nst;
   int ld;     // LDS elements per line
   int ngen;   // roots of larger primes copied to LDS behind the lines
-  int flat;   // the group's lines are loaded and stored as one run of elements
+  int flat;   // the group's lines are loaded and stored one after another
+  int flat_in, flat_out;  // ... and lie this many scalars apart
   float invT;
   MixStage st[kMixStages];
 };
@@ -225,6 +226,7 @@ MixGeom mix_geometry(const Desc &f, const int *pbo, bool dbl, int64_t nlines, bo
     const int G = dbl ? 16 : 32, slot = L < G ? G / L : 1;
     if (L > 1) ld += ((slot - ld) % (2 * slot) + 2 * slot) % (2 * slot);
   } else if (m.T <= 128) {
+    if (m.T <= 16) ld |= 1;  // the places of a wave's lines fall into different banks
     // groups of about 256 threads; among the sizes up to 512 threads the
     // first that leaves under a tenth of its last wave's lanes idle.  Groups
     // of 5 to 7 waves fill the four SIMDs unevenly: lines of 1000 (100

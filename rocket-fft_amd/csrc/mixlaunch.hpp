@@ -12,13 +12,6 @@
 
 namespace rfh {
 
-template <typename T, int OP>
-__global__ void __launch_bounds__(dev::kMixThreads<T>)
-    k_lines(const dev::LineArgs<T> a, const MixGeom m, int64_t tile0) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  dev::mix_body<T, OP>(a, m, tile0 + int64_t(dev::xcd_tile()), smem_raw);
-}
-
 // Lines of one small butterfly, bound by the loads a CU keeps in flight, which
 // are as short as the lines: the general form's registers (every radix to 17)
 // allow five waves per SIMD (complex128: three), this one eight for most
@@ -26,11 +19,12 @@ __global__ void __launch_bounds__(dev::kMixThreads<T>)
 // -> 20.8, rows of 3 27.4 -> 18.2, real lines of 3 along axis 0 of 2.8M 42.8 ->
 // 29.9, of 2 lines (DCT-II) of 4.2M 105.6 -> 77.5.
 constexpr int kShortThreads = 512;
-template <typename T, int OP>
-__global__ void __launch_bounds__(kShortThreads)
-    k_lines_short(const dev::LineArgs<T> a, const MixGeom m, int64_t tile0) {
+
+template <typename T, int OP, int FORM>
+__global__ void __launch_bounds__(FORM ? kShortThreads : dev::kMixThreads<T>)
+    k_lines(const dev::LineArgs<T> a, const MixGeom m, int64_t tile0) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  dev::mix_body<T, OP, true>(a, m, tile0 + int64_t(dev::xcd_tile()), smem_raw);
+  dev::mix_body<T, OP, FORM>(a, m, tile0 + int64_t(dev::xcd_tile()), smem_raw);
 }
 
 template <typename T, int OP>
@@ -48,16 +42,18 @@ void launch_mix_op(const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s) {
     HIP_CHECK(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(mu);
     if (!done.count(dev)) {
-      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_lines<T, OP>),
+      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_lines<T, OP, 0>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                     int(lds_limit())));
       done.insert(dev);
     }
   }
-  auto *fn = &k_lines<T, OP>;
-  if constexpr (OP != dev::OP_PASSA && OP != dev::OP_PASSB && OP != dev::OP_BLUE &&
-                OP != dev::OP_BLUEROW)
-    if (short_lines(m) && threads <= kShortThreads && lds <= 65536) fn = &k_lines_short<T, OP>;
+  auto *fn = &k_lines<T, OP, 0>;
+  if constexpr (dev::is_flat_op(OP))
+    if (threads <= kShortThreads && lds <= 65536) {
+      if (m.flat) fn = short_lines(m) ? &k_lines<T, OP, dev::kShort | dev::kFlat> : &k_lines<T, OP, dev::kFlat>;
+      else if (short_lines(m)) fn = &k_lines<T, OP, dev::kShort>;
+    }
   for_launches(groups, threads, [&](int64_t first, int64_t count) {
     hipLaunchKernelGGL(fn, dim3(unsigned(count)), dim3(unsigned(threads)), lds, s, a, m, first);
     const hipError_t e = hipGetLastError();

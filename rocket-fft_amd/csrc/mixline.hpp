@@ -54,6 +54,17 @@ template <int OP, typename T>
 __device__ __forceinline__ int op_of(const LineArgs<T> &a) {
   return OP == OP_ANY ? a.op : OP;
 }
+constexpr bool real_in(int op) { return op == OP_R2C_EVEN || op == OP_R2C_ODD || op == OP_R2R; }
+constexpr bool real_out(int op) { return op == OP_C2R_EVEN || op == OP_C2R_ODD || op == OP_R2R; }
+// Forms of the kernel beside the general one: lines of at most one butterfly of
+// a small radix (short_lines), without the other radices' registers; groups of
+// short contiguous lines that move flat (Walk).
+constexpr int kShort = 1, kFlat = 2;
+// operations that have a flat form
+constexpr bool is_flat_op(int op) {
+  return op == OP_C2C || op == OP_R2C_EVEN || op == OP_R2C_ODD || op == OP_C2R_EVEN ||
+         op == OP_C2R_ODD || op == OP_R2R;
+}
 __device__ __forceinline__ bool is_blue(int op) { return op == OP_BLUE || op == OP_BLUEROW; }
 // whether an op stores bin by bin, straight from the last stage's registers
 __device__ __forceinline__ bool elem_store(int op) { return op != OP_R2C_EVEN && op != OP_R2R; }
@@ -67,16 +78,43 @@ struct MixCtx {
   int j;        // place in the line
   bool ok;      // the line exists and the thread has a place in it
   bool line;    // ... the line exists (a line alone in its group: for every thread)
+  const T *in0;  // the group's first line, its lines and their LDS (FLAT only)
+  T *out0;
+  int nl;
+  C2<T> *lds;
 };
 
-// How the threads walk a line element by element: a line alone in its group
-// takes all of the group's threads, also those without a place in the stages.
-template <typename T>
+// How the threads walk `count` elements of each line: those of a line by its
+// own threads; a line alone in its group takes all of the group's threads, also
+// those without a place in the stages; FLAT: the group's lines one after
+// another, neighbours to neighbouring threads, whichever line they are in.
+template <typename T, int FORM>
 struct Walk {
-  int step;
+  static constexpr bool FLAT = (FORM & kFlat) != 0, SHORT = (FORM & kShort) != 0;
+  const MixGeom &m;
+  const MixCtx<T> &c;
+  int first, step, total, count;
+  float inv;
   bool on;
-  __device__ __forceinline__ Walk(const MixGeom &m, const MixCtx<T> &c)
-      : step(m.L == 1 ? int(blockDim.x) : m.T), on(m.L == 1 ? c.line : c.ok) {}
+  __device__ __forceinline__ Walk(const MixGeom &m_, const MixCtx<T> &c_, int count_)
+      : m(m_),
+        c(c_),
+        first(FLAT ? int(threadIdx.x) : c.j),
+        step(FLAT || (!SHORT && m.L == 1) ? int(blockDim.x) : m.T),
+        total(FLAT ? c.nl * count_ : count_),
+        count(count_),
+        inv(1.0f / float(count_)),
+        on(FLAT || (!SHORT && m.L == 1 ? c.line : c.ok)) {}
+  // element e's index in its line; the line's addresses
+  __device__ __forceinline__ int place(int e, MixCtx<T> &at) const {
+    at = c;
+    if (!FLAT) return e;
+    const int l = fdiv(e, count, inv);
+    at.in = c.in0 + unsigned(__mul24(l, m.flat_in));
+    at.out = c.out0 + unsigned(__mul24(l, m.flat_out));
+    at.ln = c.lds + __mul24(l, m.ld);
+    return e - __mul24(l, count);
+  }
 };
 
 template <typename T>
@@ -109,12 +147,13 @@ __device__ __forceinline__ C2<T> step_twiddle(const LineArgs<T> &a, int k, int a
 }
 
 // Inputs j + r NR (r < R) of a line, with the op's pre-processing.  CLAMP:
-// beyond the line its last element instead.
-template <typename T, int OP, int R, bool CLAMP = false>
+// beyond the line its last element instead.  FLAT: of adjacent elements.
+template <typename T, int OP, int R, bool CLAMP = false, bool FLAT = false>
 __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c, int j, int NR,
                                         C2<T> *v) {
   const bool cj = (a.sub & SUB_CONJ) != 0;
-  const int64_t es = a.esi;
+  using Es = std::conditional_t<FLAT, int, int64_t>;
+  const Es es = FLAT ? Es(real_in(OP) ? 1 : 2) : Es(a.esi);
   const int op = op_of<OP>(a);
   auto at = [&](int r) { return CLAMP ? min(j + r * NR, a.f.n - 1) : j + r * NR; };
   if (op == OP_C2C || op == OP_PASSB || op == OP_BLUEROW || op == OP_PASSA) {
@@ -140,7 +179,7 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
       for (int r = 0; r < R; ++r) v[r] = gload(c.in + rot_index(at(r), a.rot_in, a.nin) * es);
     } else {
       const T *p = c.in + j * es;
-      const int64_t step = NR * es;
+      const Es step = NR * es;
 #pragma unroll
       for (int r = 0; r < R; ++r) v[r] = gload(CLAMP ? c.in + at(r) * es : p + r * step);
     }
@@ -160,7 +199,7 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
     }
   } else if (op == OP_R2C_EVEN) {
     const T *p = c.in + 2 * j * es;
-    const int64_t step = 2 * NR * es;
+    const Es step = 2 * NR * es;
     if (es == 1) {
 #pragma unroll
       for (int r = 0; r < R; ++r) v[r] = gload(CLAMP ? c.in + 2 * at(r) * es : p + r * step);
@@ -177,7 +216,7 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
   } else if (op == OP_C2R_EVEN) {
     const int h = a.f.n;
     const T *p = c.in + j * es, *pm = c.in + (h - j) * es;
-    const int64_t step = NR * es;
+    const Es step = NR * es;
     C2<T> xm[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -201,20 +240,18 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
       v[r] = pre_elem<T, int>(a.sub & 0xff, c.in, es, int(a.bign), a.f.n, at(r),
                               (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_CONJ) != 0,
                               (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0});
-  } else {  // OP_C2R_ODD
+  } else {  // OP_C2R_ODD: bin j, or the conjugate of bin n - j
     const int n = a.f.n;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int jj = at(r);
-      if (jj == 0) {
-        v[r] = C2<T>{c.in[0], T(0)};
-      } else if (2 * jj < n) {
-        v[r] = gload(c.in + jj * es);
-        if (cj) v[r].y = -v[r].y;
-      } else {
-        v[r] = gload(c.in + (n - jj) * es);
-        if (!cj) v[r].y = -v[r].y;
-      }
+      v[r] = gload(c.in + (2 * jj < n ? jj : n - jj) * es);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int jj = at(r);
+      if ((2 * jj < n) == cj) v[r].y = -v[r].y;
+      if (jj == 0) v[r].y = T(0);
     }
   }
   if (op != OP_BLUE && op != OP_BLUEROW && op != OP_R2C_EVEN && op != OP_R2C_ODD) {
@@ -226,12 +263,13 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
 }
 
 // Bins j + r ns (r < R), with the op's post-processing.  CLAMP: those beyond
-// the line are left out.
-template <typename T, int OP, int R, bool CLAMP = false>
+// the line are left out.  FLAT: to adjacent elements.
+template <typename T, int OP, int R, bool CLAMP = false, bool FLAT = false>
 __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &c, int j, int ns,
                                          C2<T> *v) {
   const bool cj = (a.sub & SUB_CONJ) != 0;
-  const int64_t es = a.eso;
+  using Es = std::conditional_t<FLAT, int, int64_t>;
+  const Es es = FLAT ? Es(real_out(OP) ? 1 : 2) : Es(a.eso);
   const int op = op_of<OP>(a);
   auto in_line = [&](int r) { return !CLAMP || j + r * ns < a.f.n; };
   if (is_blue(op) || (op != OP_R2C_ODD && a.dir > T(0))) {  // the inverse transform ran on exchanged parts
@@ -239,7 +277,7 @@ __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &
     for (int r = 0; r < R; ++r) v[r] = C2<T>{v[r].y, v[r].x};
   }
   T *p = c.out + j * es;
-  const int64_t step = ns * es;
+  const Es step = ns * es;
   if (op == OP_C2C || op == OP_PASSB) {
     if (a.rot_out) {
 #pragma unroll
@@ -340,23 +378,41 @@ __device__ __forceinline__ void kernel_product(const LineArgs<T> &a, const MixCt
   }
 }
 
+// Bin k of a real line from bins k and h - k of its half-length spectrum.
+template <typename T>
+__device__ __forceinline__ void real_bin(const LineArgs<T> &a, int k, int h, C2<T> zk, C2<T> zm,
+                                         T *to) {
+  C2<T> X;
+  if (k == 0 || k == h) {
+    X = C2<T>{k == 0 ? zk.x + zk.y : zk.x - zk.y, T(0)};
+  } else {
+    zm = conjc(zm);
+    const C2<T> fe = T(0.5) * (zk + zm);
+    const C2<T> dd = zk - zm;
+    X = fe + cmul(a.t0[k], C2<T>{T(0.5) * dd.y, T(-0.5) * dd.x});
+  }
+  if ((a.sub & SUB_CONJ) != 0) X.y = -X.y;
+  gstore(to, a.fct * X);
+}
+
 // One forward stage of radix R (first: inputs from global memory; last:
 // outputs to global memory, or for Bluestein on through the kernel product
 // into the first backward stage).
-template <typename T, int OP, int R, bool SHORT = false>
+template <typename T, int OP, int R, int FORM = 0>
 __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m,
                                           const MixStage &st, const MixCtx<T> &c, bool first,
                                           bool last) {
-  constexpr int QM = !SHORT && kMaxElems<T> / R > 0 ? kMaxElems<T> / R : 1;
+  constexpr int QM = !(FORM & kShort) && kMaxElems<T> / R > 0 ? kMaxElems<T> / R : 1;
   const int op = op_of<OP>(a);
-  const int NR = st.nr, ns = st.ns;
-  const bool from_lds = !first || OP == OP_R2R || OP == OP_ANY || m.flat;
+  const int NR = FORM & kShort ? 1 : st.nr, ns = FORM & kShort ? 1 : st.ns;
+  constexpr bool FLAT = (FORM & kFlat) != 0;
+  const bool from_lds = !first || OP == OP_R2R || OP == OP_ANY || FLAT;
   const C2<T> *tw = a.tw + st.twoff;
   C2<T> v[QM][R];
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
     const int j = c.j + q * m.T;
-    if (q < st.q && c.ok && j < NR) {
+    if ((FORM & kShort || q < st.q) && c.ok && j < NR) {
       bool loaded = false;
       if constexpr (OP != OP_ANY)
         if (!from_lds) {
@@ -364,10 +420,11 @@ __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m
           loaded = true;
         }
       if (!loaded) {
-        const int b = fdiv(j, ns, st.invns), k = j - b * ns;
+        const int b = FORM & kShort ? 0 : fdiv(j, ns, st.invns), k = j - b * ns;
         const C2<T> *s = c.ln + b * st.pbi + k;
+        const int rs = FORM & kShort ? 1 : st.rs;
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[q][r] = s[r * st.rs];
+        for (int r = 0; r < R; ++r) v[q][r] = s[r * rs];
         if (!first) {
 #pragma unroll
           for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], tw[(r - 1) * ns + k]);
@@ -376,12 +433,21 @@ __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m
       bfly<R>(v[q]);
     }
   }
+  if constexpr (FORM == kShort && OP == OP_R2C_EVEN) {  // the whole spectrum is in v
+    if (c.ok) {
+#pragma unroll
+      for (int k = 0; k <= R; ++k)
+        real_bin(a, k, R, v[0][k % R], v[0][(R - k) % R], c.out + k * a.eso);
+    }
+    return;
+  }
   if constexpr (OP != OP_ANY) {
-    if (elem_store(op) && !is_blue(op) && last && !m.flat) {
+    if (elem_store(op) && !is_blue(op) && last && !FLAT) {
 #pragma unroll
       for (int q = 0; q < QM; ++q) {
         const int j = c.j + q * m.T;
-        if (q < st.q && c.ok && j < NR) op_store<T, OP, R>(a, c, j, ns, v[q]);
+        if ((FORM & kShort || q < st.q) && c.ok && j < NR)
+          op_store<T, OP, R>(a, c, j, ns, v[q]);
       }
       return;
     }
@@ -422,8 +488,8 @@ __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
     const int j = c.j + q * m.T;
-    if (q < st.q && c.ok && j < NR) {
-      const int b = fdiv(j, ns, st.invns), k = j - b * ns;
+    if ((FORM & kShort || q < st.q) && c.ok && j < NR) {
+      const int b = FORM & kShort ? 0 : fdiv(j, ns, st.invns), k = j - b * ns;
       C2<T> *d = c.ln + b * st.pbo + k;
 #pragma unroll
       for (int r = 0; r < R; ++r) d[r * ns] = swapri(v[q][r], sw);
@@ -497,69 +563,107 @@ __device__ __forceinline__ void with_post_mode(int mode, F &&f) {
   }
 }
 
-// The whole line to LDS, in order (with the batch executor's operations
-// and the real-to-real ones kLineBatch loads of a thread in flight).
+// The whole line to LDS, in order, a batch of loads of a thread in flight.
 constexpr int kLineBatch = 8;
-template <typename T, int OP>
+template <typename T, int OP, int FORM>
 __device__ __forceinline__ void load_line(const LineArgs<T> &a, const MixGeom &m,
                                           const MixCtx<T> &c) {
-  const Walk<T> w(m, c);
-  if constexpr (OP == OP_R2R) {
-    if (w.on)
+  constexpr bool FLAT = (FORM & kFlat) != 0;
+  const Walk<T, FORM> w(m, c, a.f.n);
+  // (short lines leave most of a large batch empty; two loads an element)
+  constexpr int B = FLAT && ((FORM & kShort) || OP == OP_C2R_EVEN) ? 4 : kLineBatch;
+  auto walk = [&](auto &&load) {
+    for (int e = w.first; e < w.total; e += B * w.step) {
+      C2<T> v[B], *to[B];
+#pragma unroll
+      for (int r = 0; r < B; ++r) {
+        MixCtx<T> at;
+        const int p = w.place(min(e + r * w.step, w.total - 1), at);
+        to[r] = at.ln + p;
+        load(at, p, &v[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < B; ++r)
+        if (e + r * w.step < w.total) *to[r] = v[r];
+    }
+  };
+  if (w.on) {
+    if constexpr (OP == OP_R2R) {
       with_pre_mode(a.sub & 0xff, [&](auto mode) {
-        for (int e = c.j; e < a.f.n; e += kLineBatch * w.step) {
-          C2<T> v[kLineBatch];
-#pragma unroll
-          for (int r = 0; r < kLineBatch; ++r)
-            v[r] = pre_elem<T, int>(mode, c.in, a.esi, int(a.bign), a.f.n,
-                                    min(e + r * w.step, a.f.n - 1), (a.sub & R2R_ORTHO) != 0,
-                                    (a.sub & R2R_CONJ) != 0, (a.sub & R2R_FLIP) != 0,
-                                    TableRoot<T>{a.t0});
-#pragma unroll
-          for (int r = 0; r < kLineBatch; ++r)
-            if (e + r * w.step < a.f.n) c.ln[e + r * w.step] = swapri(v[r], a.dir > T(0));
-        }
+        walk([&](const MixCtx<T> &at, int p, C2<T> *v) {
+          *v = swapri(pre_elem<T, int>(mode, at.in, FLAT ? 1 : a.esi, int(a.bign), a.f.n, p,
+                                       (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_CONJ) != 0,
+                                       (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0}),
+                      a.dir > T(0));
+        });
       });
-  } else {
-    constexpr int U = OP == OP_ANY ? kLineBatch : 1;
-    if (w.on)
-      for (int e = c.j; e < a.f.n; e += U * w.step) {
-        C2<T> v[U];
-        op_load<T, OP, U, (U > 1)>(a, c, e, w.step, v);
+    } else if constexpr (OP == OP_ANY) {
+      for (int e = c.j; e < a.f.n; e += B * w.step) {
+        C2<T> v[B];
+        op_load<T, OP, B, true>(a, c, e, w.step, v);
 #pragma unroll
-        for (int r = 0; r < U; ++r)
+        for (int r = 0; r < B; ++r)
           if (e + r * w.step < a.f.n) c.ln[e + r * w.step] = v[r];
       }
+    } else if constexpr (FLAT) {
+      walk([&](const MixCtx<T> &at, int p, C2<T> *v) { op_load<T, OP, 1, false, true>(a, at, p, 0, v); });
+    } else {
+      for (int e = c.j; e < a.f.n; e += w.step) {
+        C2<T> v;
+        op_load<T, OP, 1>(a, c, e, 0, &v);
+        c.ln[e] = v;
+      }
+    }
   }
   __syncthreads();
 }
 
 // ... and from LDS.
-template <typename T, int OP>
+template <typename T, int OP, int FORM>
 __device__ __forceinline__ void store_line(const LineArgs<T> &a, const MixGeom &m,
                                            const MixCtx<T> &c) {
-  const Walk<T> w(m, c);
-  if (w.on)
+  const int count = OP == OP_R2C_ODD ? a.nout : a.f.n;
+  const Walk<T, FORM> w(m, c, count);
+  if (!w.on) return;
+  if constexpr (OP == OP_ANY) {
     for (int e = c.j; e < a.f.n; e += kLineBatch * w.step) {
       C2<T> v[kLineBatch];
 #pragma unroll
       for (int r = 0; r < kLineBatch; ++r) v[r] = c.ln[min(e + r * w.step, a.f.n - 1)];
       op_store<T, OP, kLineBatch, true>(a, c, e, w.step, v);
     }
+  } else {
+    constexpr int B = 4;
+    for (int e = w.first; e < w.total; e += B * w.step) {
+      MixCtx<T> at[B];
+      C2<T> v[B];
+      int p[B];
+#pragma unroll
+      for (int r = 0; r < B; ++r) {
+        p[r] = w.place(min(e + r * w.step, w.total - 1), at[r]);
+        v[r] = at[r].ln[p[r]];
+      }
+#pragma unroll
+      for (int r = 0; r < B; ++r)
+        if (e + r * w.step < w.total)
+          op_store<T, OP, 1, false, (FORM & kFlat) != 0>(a, at[r], p[r], 0, &v[r]);
+    }
+  }
 }
 
 // A stage of a prime radix R above 17: st.q output pairs (kk, R - kk) of one
 // butterfly per thread, accumulated over the symmetric sums of its inputs,
 // which are read (and twiddled) once for all of them.  Unit u = chunk NR +
 // butterfly, so lanes share a chunk and the roots come from LDS as broadcasts.
-template <typename T, int OP>
+template <typename T, int OP, int FORM>
 __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixGeom &m,
                                                 const MixStage &st, const MixCtx<T> &c,
                                                 const C2<T> *roots, bool first, bool last) {
   constexpr int PM = kMaxElems<T> / 2;
   const int R = st.radix, NR = st.nr, ns = st.ns, H = (R - 1) / 2;
   const C2<T> *tw = a.tw + st.twoff;
-  if (first && OP != OP_R2R && OP != OP_ANY && !m.flat) load_line<T, OP>(a, m, c);  // an input serves several threads
+  constexpr bool FLAT = (FORM & kFlat) != 0;
+  if (first && OP != OP_R2R && OP != OP_ANY && !FLAT) load_line<T, OP, FORM>(a, m, c);  // an input serves several threads
   const int ch = fdiv(c.j, NR, 1.0f / float(NR)), j = c.j - ch * NR;
   const int k0 = ch * st.q;  // first pair of the chunk
   const bool on = c.ok && k0 <= H;
@@ -597,7 +701,7 @@ __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixG
     }
   }
   // outputs: bin kk and bin R - kk of the butterfly
-  const bool lds = OP == OP_ANY || !(elem_store(op_of<OP>(a)) && last && !m.flat);
+  const bool lds = OP == OP_ANY || !(elem_store(op_of<OP>(a)) && last && !FLAT);
   const bool sw = lds && last && OP == OP_R2R && a.dir > T(0);
   if (lds) __syncthreads();
   if (on) {
@@ -628,12 +732,14 @@ __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixG
 // The place of thread t in its group: the line it works on and its index in
 // it.  Contiguous lines: a line's threads are adjacent (runs along the line);
 // interleaved lines: adjacent threads take the same place of adjacent lines.
-template <typename T>
+// SHORT: a thread a line.
+template <typename T, bool SHORT>
 __device__ __forceinline__ MixCtx<T> mix_place(const LineArgs<T> &a, const MixGeom &m,
                                                int64_t tile, C2<T> *lds, bool lfast) {
   const int t = threadIdx.x;
-  int l, j;
-  if (lfast) {
+  int l = t, j = 0;
+  if (SHORT) {
+  } else if (lfast) {
     l = t & (m.L - 1);
     j = t >> m.log2L;
   } else {
@@ -643,7 +749,7 @@ __device__ __forceinline__ MixCtx<T> mix_place(const LineArgs<T> &a, const MixGe
   MixCtx<T> c;
   const int64_t b = tile * m.L + l;
   c.line = l < m.L && b < a.nlines;
-  c.ok = c.line && j < m.T;
+  c.ok = c.line && (SHORT || j < m.T);
   const LineOffsets o = c.line ? line_offsets(b, a.nb, a.bdim, a.bsi, a.bso, a.auxdim)
                              : LineOffsets{0, 0, 0};
   c.in = a.in + o.oi;
@@ -651,20 +757,23 @@ __device__ __forceinline__ MixCtx<T> mix_place(const LineArgs<T> &a, const MixGe
   c.aux = o.aux;
   c.j = j;
   c.ln = lds + (c.line ? l : 0) * m.ld;
+  c.in0 = a.in + (a.nb ? tile * m.L * a.bsi[0] : 0);
+  c.out0 = a.out + (a.nb ? tile * m.L * a.bso[0] : 0);
+  c.nl = int(min(int64_t(m.L), a.nlines - tile * m.L));
+  c.lds = lds;
   return c;
 }
 
 // One tile (m.L lines from line tile m.L on) of a line set.  Ends without a
-// barrier: a caller that runs several tiles puts one between them.  SHORT: the
-// form for short_lines(m), without the other radices' registers.
-template <typename T, int OP, bool SHORT = false>
+// barrier: a caller that runs several tiles puts one between them.
+template <typename T, int OP, int FORM = 0>
 __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m, int64_t tile,
                                          unsigned char *smem) {
   const int op = op_of<OP>(a);
   C2<T> *lds = reinterpret_cast<C2<T> *>(smem);
-  MixCtx<T> c = mix_place(a, m, tile, lds, a.lfast_in != 0);
+  MixCtx<T> c = mix_place<T, (FORM & kShort) != 0>(a, m, tile, lds, a.lfast_in != 0);
   C2<T> *roots = lds + m.L * m.ld;
-  if (m.ngen) {
+  if (!(FORM & kShort) && m.ngen) {
     for (int i = threadIdx.x; i < m.ngen; i += blockDim.x) roots[i] = a.gen[i];
     __syncthreads();
   }
@@ -678,42 +787,35 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
     }
     __syncthreads();
   }
-  if (OP == OP_C2C && m.flat) {
-    const int n = a.f.n, nl = int(min(int64_t(m.L), a.nlines - tile * m.L));
-    const float invn = 1.0f / float(n);
-    const int64_t bs = a.nb ? a.bsi[0] : 0;
-    const T *in = a.in + tile * m.L * bs;
-    for (int e = threadIdx.x; e < nl * n; e += blockDim.x) {
-      const int l = fdiv(e, n, invn), p = e - l * n;
-      lds[l * m.ld + p] = swapri(gload(in + l * bs + 2 * p), a.dir > T(0));
-    }
-    __syncthreads();
-  }
   // the real-to-real modes' heavier loads stay out of the unrolled stages
-  if ((OP == OP_R2R || OP == OP_ANY) && m.nst) load_line<T, OP>(a, m, c);
-  for (int s = 0; s < m.nst; ++s) {
-    const MixStage &st = m.st[s];
-    const bool first = s == 0, last = s == m.nst - 1;
+  constexpr bool FLAT = (FORM & kFlat) != 0;
+  if ((OP == OP_R2R || OP == OP_ANY || FLAT) && m.nst) load_line<T, OP, FORM>(a, m, c);
 #define RFH_CASE(R) \
-  case R: mix_stage<T, OP, R, SHORT>(a, m, st, c, first, last); break;
-    if constexpr (SHORT) {
+  case R: mix_stage<T, OP, R, FORM>(a, m, st, c, first, last); break;
+  if constexpr (FORM & kShort) {
+    const MixStage &st = m.st[0];
+    constexpr bool first = true, last = true;
+    if (m.nst) {
       switch (st.radix) {
         RFH_SHORT_RADICES(RFH_CASE)
         default: break;
       }
-      break;  // a single stage
     }
+  }
+  for (int s = 0; !(FORM & kShort) && s < m.nst; ++s) {
+    const MixStage &st = m.st[s];
+    const bool first = s == 0, last = s == m.nst - 1;
     switch (st.radix) {
       RFH_MIX_RADICES(RFH_CASE)
 #undef RFH_CASE
       default:
         if constexpr (OP != OP_BLUE && OP != OP_BLUEROW)
-          mix_prime_stage<T, OP>(a, m, st, c, roots, first, last);
+          mix_prime_stage<T, OP, FORM>(a, m, st, c, roots, first, last);
         break;
     }
     // from the first exchange on, threads take the places of the output side
     if (first && !last && a.lfast_out != a.lfast_in)
-      c = mix_place(a, m, tile, lds, a.lfast_out != 0);
+      c = mix_place<T, false>(a, m, tile, lds, a.lfast_out != 0);
   }
   if (is_blue(op)) {
     for (int s = m.nst - 2; s >= 0; --s) {
@@ -727,55 +829,41 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
       }
     }
   }
-  if (OP == OP_C2C && m.flat && m.nst) {  // the lines' bins are in LDS, in order
-    const int n = a.f.n, nl = int(min(int64_t(m.L), a.nlines - tile * m.L));
-    const float invn = 1.0f / float(n);
-    const int64_t bs = a.nb ? a.bso[0] : 0;
-    T *out = a.out + tile * m.L * bs;
-    for (int e = threadIdx.x; e < nl * n; e += blockDim.x) {
-      const int l = fdiv(e, n, invn), p = e - l * n;
-      gstore(out + l * bs + 2 * p, a.fct * swapri(lds[l * m.ld + p], a.dir > T(0)));
-    }
-  }
-  if constexpr (OP == OP_ANY)
-    if (m.nst && elem_store(op)) store_line<T, OP>(a, m, c);
-  if (op == OP_R2C_EVEN) {  // bins k and h - k of the half-length spectrum
-    const Walk<T> w(m, c);
+  if constexpr (OP == OP_ANY || FLAT)  // the bins are in LDS, in order
+    if (m.nst && elem_store(op)) store_line<T, OP, FORM>(a, m, c);
+  // bins k and h - k of the half-length spectrum (FORM == kShort: stored already)
+  if (op == OP_R2C_EVEN && !(FORM == kShort && m.nst)) {
+    const int h = a.f.n;
+    const Walk<T, FORM> w(m, c, h + 1);
     if (w.on) {
-      const int h = a.f.n;
-      const bool cj = (a.sub & SUB_CONJ) != 0;
-      for (int k = c.j; k <= h; k += w.step) {
-        C2<T> X;
-        if (k == 0 || k == h) {
-          const C2<T> z = c.ln[0];
-          X = C2<T>{k == 0 ? z.x + z.y : z.x - z.y, T(0)};
-        } else {
-          const C2<T> zk = c.ln[k], zm = conjc(c.ln[h - k]);
-          const C2<T> fe = T(0.5) * (zk + zm);
-          const C2<T> dd = zk - zm;
-          X = fe + cmul(a.t0[k], C2<T>{T(0.5) * dd.y, T(-0.5) * dd.x});
-        }
-        if (cj) X.y = -X.y;
-        gstore(c.out + k * a.eso, a.fct * X);
+      for (int e = w.first; e < w.total; e += w.step) {
+        MixCtx<T> at;
+        const int k = w.place(e, at);
+        const bool end = k == 0 || k == h;
+        real_bin(a, k, h, at.ln[end ? 0 : k], at.ln[end ? 0 : h - k],
+                 at.out + (FLAT ? 2 * k : k * a.eso));
       }
     }
   }
   if constexpr (OP == OP_R2R) {
-    const Walk<T> w(m, c);
+    const Walk<T, FORM> w(m, c, a.nout);
     if (w.on) {
-      const C2<T> *ln = c.ln;
       with_post_mode((a.sub >> 8) & 0xff, [&](auto mode) {
-        for (int k = c.j; k < a.nout; k += kLineBatch * w.step) {
-          T y[kLineBatch];
+        for (int e = w.first; e < w.total; e += kLineBatch * w.step) {
+          T y[kLineBatch], *to[kLineBatch];
 #pragma unroll
-          for (int r = 0; r < kLineBatch; ++r)
-            y[r] = a.fct * post_elem<T, int>(mode, [&](int q) { return ln[q]; }, int(a.bign),
-                                             min(k + r * w.step, a.nout - 1),
+          for (int r = 0; r < kLineBatch; ++r) {
+            MixCtx<T> at;
+            const int k = w.place(min(e + r * w.step, w.total - 1), at);
+            const C2<T> *ln = at.ln;
+            y[r] = a.fct * post_elem<T, int>(mode, [&](int q) { return ln[q]; }, int(a.bign), k,
                                              (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_FLIP) != 0,
                                              TableRoot<T>{a.t0});
+            to[r] = at.out + (FLAT ? k : k * a.eso);
+          }
 #pragma unroll
           for (int r = 0; r < kLineBatch; ++r)
-            if (k + r * w.step < a.nout) c.out[(k + r * w.step) * a.eso] = y[r];
+            if (e + r * w.step < w.total) *to[r] = y[r];
         }
       });
     }

@@ -90,12 +90,14 @@ def test_short_axis_groups(n, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
-@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 9, 10, 12, 17, 18, 19, 24, 30, 48, 62, 96])
-def test_short_rows(n, dtype):
-    """Contiguous rows, the last group a part of one; a padded output keeps its gaps."""
+@pytest.mark.parametrize("lines", [3, 257 * 9 + 1, 512 * 64 + 5])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 9, 10, 12, 17, 18, 19, 24, 30, 37, 48, 62, 96])
+def test_short_rows(n, lines, dtype):
+    """Contiguous rows, groups of one line and of many, the last group a part
+    of one; a padded output keeps its gaps."""
     import scipy.fft
     import torch
-    lines, ax = 257 * 9 + 1, np.array([1])
+    ax = np.array([1])
     print(f"case rows ({lines}, {n}) {dtype.__name__}", flush=True)
     rs = np.random.RandomState(100 + n)
     z = (rs.standard_normal((lines, n)) + 1j * rs.standard_normal((lines, n))).astype(dtype)
