@@ -60,6 +60,18 @@ inline bool short_lines(const MixGeom &m) {
   return m.nst == 0 || (m.nst == 1 && m.st[0].radix <= 9 && m.st[0].q == 1);
 }
 
+// Whether a thread takes at most kFewPairs of the output pairs of a butterfly of
+// a prime above 17: sums in a form of the kernel of their own, without the
+// branches and registers of more pairs, a lone pair's loads several iterations
+// ahead.  us, before the general kernel was rewritten / since / now: 24 lines of
+// 122 complex64 11.6 / 16.6 / 10.9, of 194 complex128 15.0 / 24.8 / 13.6.
+constexpr int kFewPairs = 3;
+inline bool few_pairs(const MixGeom &m) {
+  for (int s = 0; s < m.nst; ++s)
+    if (m.st[s].radix > 17 && m.st[s].q > kFewPairs) return false;
+  return true;
+}
+
 // Threads a line of n needs when each may hold 16 elements of a stage's
 // butterflies, and how evenly the stages use them: the sum over the stages of
 // (elements held by all threads, idle places included) / n; among equals the
@@ -180,12 +192,14 @@ MixGeom mix_geometry(const Desc &f, const int *pbo, bool dbl, int64_t nlines, bo
   if (!inter) want = 1;
   else if (!want) want = int(128 / elem);
   // 16 elements per thread; more where a group would not fit its threads
-  // otherwise, fewer while the launch leaves SIMDs without a wave
+  // otherwise, fewer while the launch leaves SIMDs without a wave.  Two (a lone
+  // output pair of a prime above 17) only for an eighth of that: 400 lines of 529
+  // complex128, 110000 threads instead of 55000, 16.5 -> 23.3 us
   m.T = threads_for(16);
   if (m.T * want > max_t) m.T = threads_for(max_e);
   const bool full = nlines * m.T >= kFillThreads;
-  for (int E : {10, 6, 4})
-    if (nlines * m.T < kFillThreads) {
+  for (int E : {10, 6, 4, 2})
+    if (nlines * m.T < (E == 2 ? kFillThreads / 8 : kFillThreads)) {
       const int t = threads_for(E);
       if (t * want <= max_t && t <= 512) m.T = std::max(m.T, t);
     }

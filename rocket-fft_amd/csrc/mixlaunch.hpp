@@ -20,8 +20,12 @@ namespace rfh {
 // 29.9, of 2 lines (DCT-II) of 4.2M 105.6 -> 77.5.
 constexpr int kShortThreads = 512;
 
+// (Five waves per SIMD for the sums of many complex64 lines with a prime: 29 of
+// 144631 lines 33.6 us at four, 30.9 at five.)
 template <typename T, int OP, int FORM>
-__global__ void __launch_bounds__(FORM ? kShortThreads : dev::kMixThreads<T>)
+__global__ void __launch_bounds__(FORM == 0 || FORM & dev::kPrime ? dev::kMixThreads<T>
+                                                                  : kShortThreads,
+                                  FORM == dev::kPrime && sizeof(T) == 4 ? 5 : 1)
     k_lines(const dev::LineArgs<T> a, const MixGeom m, int64_t tile0) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   dev::mix_body<T, OP, FORM>(a, m, tile0 + int64_t(dev::xcd_tile()), smem_raw);
@@ -35,25 +39,31 @@ void launch_mix_op(const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s) {
   if (threads > dev::kMixThreads<T> || lds > lds_limit())
     RFH_THROW(3, "line group of " + std::to_string(a.f.n) + " needs " + std::to_string(threads) +
                      " threads and " + std::to_string(lds) + " B of LDS");
-  if (lds > 65536) {  // raise the kernel's dynamic-LDS ceiling once per device
-    static std::mutex mu;
-    static std::set<int> done;
-    int dev = 0;
-    HIP_CHECK(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lk(mu);
-    if (!done.count(dev)) {
-      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_lines<T, OP, 0>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    int(lds_limit())));
-      done.insert(dev);
-    }
-  }
   auto *fn = &k_lines<T, OP, 0>;
+  if constexpr (!dev::is_blue_op(OP))
+    if (!few_pairs(m)) fn = &k_lines<T, OP, dev::kPrime>;
   if constexpr (dev::is_flat_op(OP))
     if (threads <= kShortThreads && lds <= 65536) {
-      if (m.flat) fn = short_lines(m) ? &k_lines<T, OP, dev::kShort | dev::kFlat> : &k_lines<T, OP, dev::kFlat>;
-      else if (short_lines(m)) fn = &k_lines<T, OP, dev::kShort>;
+      if (m.flat && !(m.ngen && few_pairs(m)))
+        fn = short_lines(m) ? &k_lines<T, OP, dev::kShort | dev::kFlat>
+             : m.ngen       ? &k_lines<T, OP, dev::kFlat | dev::kPrime>
+                            : &k_lines<T, OP, dev::kFlat>;
+      else if (short_lines(m))
+        fn = &k_lines<T, OP, dev::kShort>;
     }
+  if (lds > 65536) {  // raise the kernel's dynamic-LDS ceiling once per device
+    static std::mutex mu;
+    static std::set<std::pair<int, const void *>> done;
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    const void *f = reinterpret_cast<const void *>(fn);
+    std::lock_guard<std::mutex> lk(mu);
+    if (!done.count({dev, f})) {
+      HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    int(lds_limit())));
+      done.insert({dev, f});
+    }
+  }
   for_launches(groups, threads, [&](int64_t first, int64_t count) {
     hipLaunchKernelGGL(fn, dim3(unsigned(count)), dim3(unsigned(threads)), lds, s, a, m, first);
     const hipError_t e = hipGetLastError();

@@ -58,14 +58,16 @@ constexpr bool real_in(int op) { return op == OP_R2C_EVEN || op == OP_R2C_ODD ||
 constexpr bool real_out(int op) { return op == OP_C2R_EVEN || op == OP_C2R_ODD || op == OP_R2R; }
 // Forms of the kernel beside the general one: lines of at most one butterfly of
 // a small radix (short_lines), without the other radices' registers; groups of
-// short contiguous lines that move flat (Walk).
-constexpr int kShort = 1, kFlat = 2;
+// short contiguous lines that move flat (Walk); lines with a prime above 17 of
+// more than kFewPairs output pairs a thread, whose sums take registers.
+constexpr int kShort = 1, kFlat = 2, kPrime = 4;
 // operations that have a flat form
 constexpr bool is_flat_op(int op) {
   return op == OP_C2C || op == OP_R2C_EVEN || op == OP_R2C_ODD || op == OP_C2R_EVEN ||
          op == OP_C2R_ODD || op == OP_R2R;
 }
-__device__ __forceinline__ bool is_blue(int op) { return op == OP_BLUE || op == OP_BLUEROW; }
+constexpr bool is_blue_op(int op) { return op == OP_BLUE || op == OP_BLUEROW; }
+__device__ __forceinline__ bool is_blue(int op) { return is_blue_op(op); }
 // whether an op stores bin by bin, straight from the last stage's registers
 __device__ __forceinline__ bool elem_store(int op) { return op != OP_R2C_EVEN && op != OP_R2R; }
 
@@ -651,6 +653,47 @@ __device__ __forceinline__ void store_line(const LineArgs<T> &a, const MixGeom &
   }
 }
 
+// Inputs mm and R - mm of a prime stage's butterfly, twiddled, into the sums of
+// output pairs k0 .. k0 + q - 1 (q <= Q).
+template <typename T, int Q, int PM>
+__device__ __forceinline__ void prime_step(const MixStage &st, const C2<T> *s, const C2<T> *tw,
+                                           int k, const C2<T> *g, int k0, int mm, C2<T> &sum,
+                                           C2<T> (&A)[PM], C2<T> (&B)[PM], int (&idx)[PM]) {
+  const int R = st.radix, ns = st.ns;
+  C2<T> xp = s[mm * st.rs], xm = s[(R - mm) * st.rs];
+  if (ns > 1) {
+    xp = cmul(xp, tw[(mm - 1) * ns + k]);
+    xm = cmul(xm, tw[(R - mm - 1) * ns + k]);
+  }
+  const C2<T> t = xp + xm, d = xp - xm;
+  sum = sum + t;
+#pragma unroll
+  for (int p = 0; p < Q; ++p) {
+    if (Q == 1 || p < st.q) {
+      idx[p] += k0 + p;
+      if (idx[p] >= R) idx[p] -= R;
+      const C2<T> w = g[idx[p]];
+      A[p] = A[p] + w.x * t;
+      B[p] = B[p] + w.y * d;
+    }
+  }
+}
+template <typename T, int Q, int PM>
+__device__ __forceinline__ void prime_sums(const MixStage &st, const C2<T> *s, const C2<T> *tw,
+                                           int k, const C2<T> *g, int k0, C2<T> &sum,
+                                           C2<T> (&A)[PM], C2<T> (&B)[PM], int (&idx)[PM]) {
+  const int H = (st.radix - 1) / 2;
+  int mm = 1;
+  if constexpr (Q <= 3) {  // few lines: a chain of loads, some iterations' in flight
+    constexpr int U = Q == 1 ? 4 : 2;
+    for (; mm + U - 1 <= H; mm += U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) prime_step<T, Q, PM>(st, s, tw, k, g, k0, mm + u, sum, A, B, idx);
+    }
+  }
+  for (; mm <= H; ++mm) prime_step<T, Q, PM>(st, s, tw, k, g, k0, mm, sum, A, B, idx);
+}
+
 // A stage of a prime radix R above 17: st.q output pairs (kk, R - kk) of one
 // butterfly per thread, accumulated over the symmetric sums of its inputs,
 // which are read (and twiddled) once for all of them.  Unit u = chunk NR +
@@ -659,7 +702,8 @@ template <typename T, int OP, int FORM>
 __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixGeom &m,
                                                 const MixStage &st, const MixCtx<T> &c,
                                                 const C2<T> *roots, bool first, bool last) {
-  constexpr int PM = kMaxElems<T> / 2;
+  constexpr bool FEW = !(FORM & kPrime) && OP != OP_ANY;
+  constexpr int PM = FEW ? kFewPairs : kMaxElems<T> / 2;
   const int R = st.radix, NR = st.nr, ns = st.ns, H = (R - 1) / 2;
   const C2<T> *tw = a.tw + st.twoff;
   constexpr bool FLAT = (FORM & kFlat) != 0;
@@ -680,25 +724,8 @@ __device__ __forceinline__ void mix_prime_stage(const LineArgs<T> &a, const MixG
       B[p] = C2<T>{T(0), T(0)};
       idx[p] = 0;
     }
-    for (int mm = 1; mm <= H; ++mm) {
-      C2<T> xp = s[mm * st.rs], xm = s[(R - mm) * st.rs];
-      if (ns > 1) {
-        xp = cmul(xp, tw[(mm - 1) * ns + k]);
-        xm = cmul(xm, tw[(R - mm - 1) * ns + k]);
-      }
-      const C2<T> t = xp + xm, d = xp - xm;
-      sum = sum + t;
-#pragma unroll
-      for (int p = 0; p < PM; ++p) {
-        if (p < st.q) {
-          idx[p] += k0 + p;
-          if (idx[p] >= R) idx[p] -= R;
-          const C2<T> w = g[idx[p]];
-          A[p] = A[p] + w.x * t;
-          B[p] = B[p] + w.y * d;
-        }
-      }
-    }
+    if (FEW && st.q == 1) prime_sums<T, 1, PM>(st, s, tw, k, g, k0, sum, A, B, idx);
+    else prime_sums<T, PM, PM>(st, s, tw, k, g, k0, sum, A, B, idx);
   }
   // outputs: bin kk and bin R - kk of the butterfly
   const bool lds = OP == OP_ANY || !(elem_store(op_of<OP>(a)) && last && !FLAT);
@@ -809,7 +836,7 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
       RFH_MIX_RADICES(RFH_CASE)
 #undef RFH_CASE
       default:
-        if constexpr (OP != OP_BLUE && OP != OP_BLUEROW)
+        if constexpr (!is_blue_op(OP) && !(FORM == kFlat))
           mix_prime_stage<T, OP, FORM>(a, m, st, c, roots, first, last);
         break;
     }

@@ -128,3 +128,24 @@ def test_short_rows(n, lines, dtype):
     R.r2r_separable_hartley(x, y, ax, 1.0)
     f = np.fft.fft(r.astype(np.float64), axis=1)
     assert rel_l2(y.cpu().numpy(), f.real + f.imag) <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n", [19, 23, 38, 61, 97, 122, 194, 361, 437, 529, 1147, 1220, 1681])
+def test_prime_radices_few_and_many_lines(n, dtype):
+    """Lines with a prime above 17: one output pair a thread (few lines), several
+    (more of them) and many, rows and columns."""
+    import torch
+    for lines in (1, 24, 400, 5000):
+        print(f"case primes {lines} x {n} {dtype.__name__}", flush=True)
+        rs = np.random.RandomState(n + lines)
+        z = (rs.standard_normal((lines, n)) + 1j * rs.standard_normal((lines, n))).astype(dtype)
+        want = np.fft.fft(z.astype(np.complex128), axis=1)
+        t = torch.from_numpy(z).cuda()
+        y = torch.empty_like(t)
+        R.c2c(t, y, np.array([1]), True, 1.0)
+        assert rel_l2(y.cpu().numpy(), want) <= tol_of(dtype)
+        c = t.T.contiguous()
+        R.c2c(c, c, np.array([0]), True, 1.0)
+        assert rel_l2(c.T.cpu().numpy(), want) <= tol_of(dtype)
