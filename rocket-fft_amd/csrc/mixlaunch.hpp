@@ -25,7 +25,7 @@ constexpr int kShortThreads = 512;
 template <typename T, int OP, int FORM>
 __global__ void __launch_bounds__(FORM == 0 || FORM & dev::kPrime ? dev::kMixThreads<T>
                                                                   : kShortThreads,
-                                  FORM == dev::kPrime && sizeof(T) == 4 ? 5 : 1)
+                                  FORM == dev::kPrime && sizeof(T) == 4 && OP != dev::OP_PASSA ? 5 : 1)
     k_lines(const dev::LineArgs<T> a, const MixGeom m, int64_t tile0) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   dev::mix_body<T, OP, FORM>(a, m, tile0 + int64_t(dev::xcd_tile()), smem_raw);

@@ -148,11 +148,20 @@ __device__ __forceinline__ C2<T> step_twiddle(const LineArgs<T> &a, int k, int a
   return cmul(a.t0[unsigned(e) & mask], a.t1[e >> a.shift]);
 }
 
+// Factors (chirps, four-step twiddles) a thread holds beside its elements: all R
+// of them took registers that a kernel of every radix spilled (four-step columns
+// 203 complex64 and 433 complex128 ones, Bluestein lines 40 and 649): us, all /
+// these, 2000 lines of 30000 complex64 673 / 592, 64 of 10^6 907 / 801, 400
+// columns of 30000 129 / 113, 256 lines of 4099 complex128 51.9 / 40.6.
+template <typename T, int OP, int R>
+constexpr int kFactors = OP == OP_ANY ? R : (sizeof(T) == 8 ? 4 : 8);
+
 // Inputs j + r NR (r < R) of a line, with the op's pre-processing.  CLAMP:
 // beyond the line its last element instead.  FLAT: of adjacent elements.
 template <typename T, int OP, int R, bool CLAMP = false, bool FLAT = false>
 __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c, int j, int NR,
                                         C2<T> *v) {
+  constexpr int S = kFactors<T, OP, R>;
   const bool cj = (a.sub & SUB_CONJ) != 0;
   using Es = std::conditional_t<FLAT, int, int64_t>;
   const Es es = FLAT ? Es(real_in(OP) ? 1 : 2) : Es(a.esi);
@@ -161,20 +170,23 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
   if (op == OP_C2C || op == OP_PASSB || op == OP_BLUEROW || op == OP_PASSA) {
     if (op == OP_PASSA && (a.sub & SUB_CHIRP)) {  // x[m] conj(chirp[m]), zero from m = n on
       // (loads without a condition around them, so that all are in flight)
-      C2<T> w[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int64_t m = int64_t(at(r)) * a.other + c.aux;
-        const int jj = m < a.bign ? at(r) : 0;
-        const int64_t mc = m < a.bign ? m : c.aux;
-        w[r] = a.t2[mc];
-        v[r] = gload(c.in + blue_col_offset(jj, mc, a.rot_in, a.bign, c.aux, es, a.other));
-      }
+      for (int s = 0; s < R; s += S) {
+        C2<T> w[S];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const bool on = int64_t(at(r)) * a.other + c.aux < a.bign;
-        const C2<T> y = cmul(v[r], cj ? w[r] : conjc(w[r]));
-        v[r] = on ? y : C2<T>{T(0), T(0)};
+        for (int r = s; r < R && r < s + S; ++r) {
+          const int64_t m = int64_t(at(r)) * a.other + c.aux;
+          const int jj = m < a.bign ? at(r) : 0;
+          const int64_t mc = m < a.bign ? m : c.aux;
+          w[r - s] = a.t2[mc];
+          v[r] = gload(c.in + blue_col_offset(jj, mc, a.rot_in, a.bign, c.aux, es, a.other));
+        }
+#pragma unroll
+        for (int r = s; r < R && r < s + S; ++r) {
+          const bool on = int64_t(at(r)) * a.other + c.aux < a.bign;
+          const C2<T> y = cmul(v[r], cj ? w[r - s] : conjc(w[r - s]));
+          v[r] = on ? y : C2<T>{T(0), T(0)};
+        }
       }
     } else if ((op == OP_C2C || op == OP_PASSA) && a.rot_in) {
 #pragma unroll
@@ -187,17 +199,20 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
     }
   } else if (op == OP_BLUE) {
     const int n = int(a.bign);
-    C2<T> w[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {  // element (j + rot_in) mod n, times the chirp at j
-      const int jj = at(r) < n ? at(r) : 0;
-      w[r] = a.t0[jj];
-      v[r] = gload(c.in + rot_index(jj, a.rot_in, n) * es);
-    }
+    for (int s = 0; s < R; s += S) {
+      C2<T> w[S];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const C2<T> y = cmul(v[r], cj ? w[r] : conjc(w[r]));
-      v[r] = at(r) < n ? y : C2<T>{T(0), T(0)};
+      for (int r = s; r < R && r < s + S; ++r) {  // element (j + rot_in) mod n, times the chirp at j
+        const int jj = at(r) < n ? at(r) : 0;
+        w[r - s] = a.t0[jj];
+        v[r] = gload(c.in + rot_index(jj, a.rot_in, n) * es);
+      }
+#pragma unroll
+      for (int r = s; r < R && r < s + S; ++r) {
+        const C2<T> y = cmul(v[r], cj ? w[r - s] : conjc(w[r - s]));
+        v[r] = at(r) < n ? y : C2<T>{T(0), T(0)};
+      }
     }
   } else if (op == OP_R2C_EVEN) {
     const T *p = c.in + 2 * j * es;
@@ -269,6 +284,7 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
 template <typename T, int OP, int R, bool CLAMP = false, bool FLAT = false>
 __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &c, int j, int ns,
                                          C2<T> *v) {
+  constexpr int S = kFactors<T, OP, R>;
   const bool cj = (a.sub & SUB_CONJ) != 0;
   using Es = std::conditional_t<FLAT, int, int64_t>;
   const Es es = FLAT ? Es(real_out(OP) ? 1 : 2) : Es(a.eso);
@@ -292,48 +308,62 @@ __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &
         if (in_line(r)) gstore(p + r * step, a.fct * v[r]);
     }
   } else if (op == OP_PASSA) {
-    // the factors of all bins first, without a condition around their loads
-    C2<T> w[R];
+    // a slice's factors first, without a condition around their loads
     if (a.sub & SUB_FINAL) {  // Bluestein columns, last pass: chirp and fct, m < n
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int64_t m = c.aux + int64_t(j + r * ns) * a.other;
-        w[r] = a.t0[m < a.bign ? m : c.aux];
-      }
+      for (int s = 0; s < R; s += S) {
+        C2<T> w[S];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int k = j + r * ns;
-        const int64_t m = c.aux + int64_t(k) * a.other;
-        if (in_line(r) && m < a.bign)
-          gstore(c.out + blue_col_offset(k, m, a.rot_out, a.bign, c.aux, es, a.other),
-                 a.fct * cmul(v[r], cj ? w[r] : conjc(w[r])));
+        for (int r = s; r < R && r < s + S; ++r) {
+          const int64_t m = c.aux + int64_t(j + r * ns) * a.other;
+          w[r - s] = a.t0[m < a.bign ? m : c.aux];
+        }
+#pragma unroll
+        for (int r = s; r < R && r < s + S; ++r) {
+          const int k = j + r * ns;
+          const int64_t m = c.aux + int64_t(k) * a.other;
+          if (in_line(r) && m < a.bign)
+            gstore(c.out + blue_col_offset(k, m, a.rot_out, a.bign, c.aux, es, a.other),
+                   a.fct * cmul(v[r], cj ? w[r - s] : conjc(w[r - s])));
+        }
       }
     } else {
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        w[r] = step_twiddle(a, CLAMP ? min(j + r * ns, a.f.n - 1) : j + r * ns, c.aux);
+      for (int s = 0; s < R; s += S) {
+        C2<T> w[S];
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (in_line(r)) gstore(p + r * step, cmul(v[r], dirw(w[r], a.dir)));
+        for (int r = s; r < R && r < s + S; ++r)
+          w[r - s] = step_twiddle(a, CLAMP ? min(j + r * ns, a.f.n - 1) : j + r * ns, c.aux);
+#pragma unroll
+        for (int r = s; r < R && r < s + S; ++r)
+          if (in_line(r)) gstore(p + r * step, cmul(v[r], dirw(w[r - s], a.dir)));
+      }
     }
   } else if (op == OP_BLUEROW) {
-    C2<T> w[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      w[r] = step_twiddle(a, CLAMP ? min(j + r * ns, a.f.n - 1) : j + r * ns, c.aux);
+    for (int s = 0; s < R; s += S) {
+      C2<T> w[S];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (in_line(r)) gstore(p + r * step, cmul(v[r], conjc(w[r])));
+      for (int r = s; r < R && r < s + S; ++r)
+        w[r - s] = step_twiddle(a, CLAMP ? min(j + r * ns, a.f.n - 1) : j + r * ns, c.aux);
+#pragma unroll
+      for (int r = s; r < R && r < s + S; ++r)
+        if (in_line(r)) gstore(p + r * step, cmul(v[r], conjc(w[r - s])));
+    }
   } else if (op == OP_BLUE) {  // bin k < n, chirped, to (k + rot_out) mod n
-    C2<T> w[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) w[r] = a.t0[j + r * ns < a.nout ? j + r * ns : 0];
+    for (int s = 0; s < R; s += S) {
+      C2<T> w[S];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int k = j + r * ns;
-      if (in_line(r) && k < a.nout)
-        gstore(c.out + rot_index(k, a.rot_out, a.nout) * es,
-               a.fct * cmul(v[r], cj ? w[r] : conjc(w[r])));
+      for (int r = s; r < R && r < s + S; ++r)
+        w[r - s] = a.t0[j + r * ns < a.nout ? j + r * ns : 0];
+#pragma unroll
+      for (int r = s; r < R && r < s + S; ++r) {
+        const int k = j + r * ns;
+        if (in_line(r) && k < a.nout)
+          gstore(c.out + rot_index(k, a.rot_out, a.nout) * es,
+                 a.fct * cmul(v[r], cj ? w[r - s] : conjc(w[r - s])));
+      }
     }
   } else if (op == OP_R2C_ODD) {
 #pragma unroll
