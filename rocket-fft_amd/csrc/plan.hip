@@ -686,9 +686,10 @@ static std::shared_ptr<RealPlan> materialize(const RealRec &r) {
 // budget, stride class) and GPU architecture, so that a later process skips
 // the FP64 table generation (the Bluestein kernel's host DFT above all):
 //   <dir>/plan_<arch>_<c2c|real>_<n>_<c64|c128>_b<budget>_<i|c>.bin
-// Format: "RFHPLAN1", the key fields, the record, an FNV-1a checksum of all
-// that; a file that does not parse, checksum or match its key is ignored
-// (and rewritten).  Files are written to a temporary name and renamed.
+// Format: "RFHPLAN1", the key fields, the record, the schedule's version, an
+// FNV-1a checksum of all that; a file that does not parse, checksum or match its
+// key and version is ignored (and rewritten).  Files are written to a temporary
+// name and renamed.
 
 namespace {
 
@@ -749,9 +750,16 @@ uint64_t fnv1a(const char *p, size_t n) {
 
 const char kMagic[8] = {'R', 'F', 'H', 'P', 'L', 'A', 'N', '1'};
 
+// The version of the schedules that records hold (radices and their order, how a
+// length is split, Bluestein lengths): one more with every change, so that a
+// directory of an earlier build does not keep its schedules alive.  (Records
+// without the field: radix 16 first, Bluestein columns of 1024 first.)
+constexpr uint32_t kScheduleVersion = 2;
+
 std::string seal(const Writer &w) {
   std::string out(kMagic, 8);
   out += w.b;
+  out.append(reinterpret_cast<const char *>(&kScheduleVersion), sizeof kScheduleVersion);
   const uint64_t h = fnv1a(out.data(), out.size());
   out.append(reinterpret_cast<const char *>(&h), sizeof h);
   return out;
@@ -759,11 +767,14 @@ std::string seal(const Writer &w) {
 
 // the payload of a sealed file, or empty when it does not check
 std::string unseal(const std::string &f) {
-  if (f.size() < 16 || std::memcmp(f.data(), kMagic, 8) != 0) return {};
+  if (f.size() < 20 || std::memcmp(f.data(), kMagic, 8) != 0) return {};
   uint64_t h = 0;
   std::memcpy(&h, f.data() + f.size() - 8, 8);
   if (h != fnv1a(f.data(), f.size() - 8)) return {};
-  return f.substr(8, f.size() - 16);
+  uint32_t v = 0;
+  std::memcpy(&v, f.data() + f.size() - 12, 4);
+  if (v != kScheduleVersion) return {};
+  return f.substr(8, f.size() - 20);
 }
 
 std::string encode(const PlanRec &r) {

@@ -517,8 +517,13 @@ std::vector<uint64_t> signature(const Batch &bt) {
   return sig;
 }
 
+// The version of the kernels and candidates that a tuning result holds for: one
+// more with every change.  It is part of the key, so that lines of an earlier
+// build are not found and their batches timed again.
+constexpr uint64_t kTuneVersion = 2;
+
 DiskKey disk_key(const std::vector<uint64_t> &sig) {
-  uint64_t h1 = 1469598103934665603ull, h2 = 0x9e3779b97f4a7c15ull;
+  uint64_t h1 = 1469598103934665603ull, h2 = 0x9e3779b97f4a7c15ull ^ kTuneVersion;
   for (uint64_t v : sig) {
     for (int b = 0; b < 8; ++b) {
       h1 = (h1 ^ ((v >> (8 * b)) & 0xff)) * 1099511628211ull;
