@@ -162,6 +162,7 @@ enum LineOp {
 };
 // OP_R2R packs its modes into LineArgs::sub
 constexpr int R2R_ORTHO = 1 << 16, R2R_CONJ = 1 << 17, R2R_FLIP = 1 << 18;
+constexpr int R2R_SINCOS = 1 << 19;  // the factors are computed, there is no table
 enum SubFlags {
   SUB_CHIRP = 1,   // pass A: multiply loads by the chirp, zero beyond n
   SUB_KERNEL = 2,  // pass B: multiply by the Bluestein kernel (natural order)

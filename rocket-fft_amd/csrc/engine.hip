@@ -355,9 +355,21 @@ void r2r_axis(Ctx &c, const int64_t *shape, int nd, int ax, const int64_t *si,
   LineSet g = lines_for_axis(shape, nd, ax, si, so, in, out);
   rr.n = shape[ax];
   rr.m = m;
-  // the whole work line fits in LDS: one launch
-  if (auto plan = get_r2r_plan(uint64_t(rr.n), uint64_t(m), c.dbl)) {
-    launch_r2r_fused(*plan, g, pre, post, rr, fft_forward, fct, c.s);
+  if (r2r_one_pass(uint64_t(m), c.dbl)) {  // the whole work line fits in LDS: one launch
+    const uint64_t n = mode_has_factors(pre, post) ? uint64_t(rr.n) : 0;
+    // a call that is being captured cannot build a plan: it takes the work
+    // length's complex one, with its factors computed, where that is there
+    if (c.ws->capturing && !find_r2r_plan(n, uint64_t(m), c.dbl)) {
+      auto shared = find_c2c_plan(uint64_t(m), c.dbl, 0, false);
+      if (!shared || shared->kind != kDirect)
+        RFH_THROW(3, "no plan for a real-to-real line of " + std::to_string(rr.n) +
+                         " while the stream is capturing a graph; run the same call once before "
+                         "capture");
+      launch_r2r_fused(shared->main, nullptr, c.dbl, g, pre, post, rr, fft_forward, fct, c.s);
+      return;
+    }
+    auto plan = get_r2r_plan(n, uint64_t(m), c.dbl);
+    launch_r2r_fused(plan->d, plan->roots.p, c.dbl, g, pre, post, rr, fft_forward, fct, c.s);
     return;
   }
   void *work = complex_work(c, g.nlines, m);

@@ -831,20 +831,42 @@ void launch_c2c(const C2CPlan &p, const LineSet &g, int dir, double fct, hipStre
   for (const PassLaunch &pl : passes) run_pass_any(p.dbl, pl.ps, pl.g, s);
 }
 
-void launch_r2r_fused(const R2RPlan &p, const LineSet &g, PreMode pre, PostMode post,
-                      const RealPrePost &rr, bool fft_forward, double fct, hipStream_t s) {
+bool mode_has_factors(PreMode pre, PostMode post) {
+  switch (pre) {
+    case kPreDct3:
+    case kPreDst3:
+    case kPreType4:
+    case kPreDct3N:
+    case kPreDst3N: return true;
+    default: break;
+  }
+  switch (post) {
+    case kPostDct2:
+    case kPostDst2:
+    case kPostDct4:
+    case kPostDst4:
+    case kPostDct2N:
+    case kPostDst2N: return true;
+    default: return false;
+  }
+}
+
+void launch_r2r_fused(const Direct &d, const void *roots, bool dbl, const LineSet &g, PreMode pre,
+                      PostMode post, const RealPrePost &rr, bool fft_forward, double fct,
+                      hipStream_t s) {
   PassSpec ps;
-  ps.d = &p.d;
-  ps.t0 = p.roots.p;
+  ps.d = &d;
+  ps.t0 = roots;
+  if (!roots && mode_has_factors(pre, post)) ps.sub = R2R_SINCOS;
   ps.op = OP_R2R;
   ps.dir = fft_forward ? -1 : +1;
   ps.fct = fct;
   ps.bign = rr.n;
-  ps.sub = int(pre) | (int(post) << 8) | (rr.ortho ? R2R_ORTHO : 0) |
-           (rr.conj ? R2R_CONJ : 0) | (rr.flip ? R2R_FLIP : 0);
+  ps.sub |= int(pre) | (int(post) << 8) | (rr.ortho ? R2R_ORTHO : 0) |
+            (rr.conj ? R2R_CONJ : 0) | (rr.flip ? R2R_FLIP : 0);
   ps.nin = int(rr.m);
   ps.nout = int(rr.n);
-  run_pass_any(p.dbl, ps, g, s);
+  run_pass_any(dbl, ps, g, s);
 }
 
 PassLaunch describe_real_fused(const RealPlan &rp, RealOp op, const LineSet &g, bool conj_flag,

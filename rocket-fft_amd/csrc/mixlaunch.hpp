@@ -51,6 +51,8 @@ void launch_mix_op(const dev::LineArgs<T> &a, const MixGeom &m, hipStream_t s) {
       else if (short_lines(m))
         fn = &k_lines<T, OP, dev::kShort>;
     }
+  if constexpr (OP == dev::OP_R2R)
+    if (a.sub & dev::R2R_SINCOS) fn = &k_lines<T, OP, dev::kPrime | dev::kSinCos>;
   if (lds > 65536) {  // raise the kernel's dynamic-LDS ceiling once per device
     static std::mutex mu;
     static std::set<std::pair<int, const void *>> done;

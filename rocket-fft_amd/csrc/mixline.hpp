@@ -56,11 +56,18 @@ __device__ __forceinline__ int op_of(const LineArgs<T> &a) {
 }
 constexpr bool real_in(int op) { return op == OP_R2C_EVEN || op == OP_R2C_ODD || op == OP_R2R; }
 constexpr bool real_out(int op) { return op == OP_C2R_EVEN || op == OP_C2R_ODD || op == OP_R2R; }
+// factors e^{i pi q / 4n} of a real-to-real line
+template <bool SINCOS, typename T>
+__device__ __forceinline__ auto root_of(const LineArgs<T> &a) {
+  if constexpr (SINCOS) return ComputedRoot<T>{a.bign};
+  else return TableRoot<T>{a.t0};
+}
 // Forms of the kernel beside the general one: lines of at most one butterfly of
 // a small radix (short_lines), without the other radices' registers; groups of
 // short contiguous lines that move flat (Walk); lines with a prime above 17 of
-// more than kFewPairs output pairs a thread, whose sums take registers.
-constexpr int kShort = 1, kFlat = 2, kPrime = 4;
+// more than kFewPairs output pairs a thread, whose sums take registers; real-to-
+// real lines without a table of their factors.
+constexpr int kShort = 1, kFlat = 2, kPrime = 4, kSinCos = 8;
 // operations that have a flat form
 constexpr bool is_flat_op(int op) {
   return op == OP_C2C || op == OP_R2C_EVEN || op == OP_R2C_ODD || op == OP_C2R_EVEN ||
@@ -251,12 +258,6 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
       const C2<T> B = cmul(x - y, conjc(a.t0[jj]));
       v[r] = C2<T>{A.x - B.y, A.y + B.x};
     }
-  } else if constexpr (OP == OP_R2R) {
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      v[r] = pre_elem<T, int>(a.sub & 0xff, c.in, es, int(a.bign), a.f.n, at(r),
-                              (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_CONJ) != 0,
-                              (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0});
   } else {  // OP_C2R_ODD: bin j, or the conjugate of bin n - j
     const int n = a.f.n;
 #pragma unroll
@@ -446,7 +447,7 @@ __device__ __forceinline__ void mix_stage(const LineArgs<T> &a, const MixGeom &m
     const int j = c.j + q * m.T;
     if ((FORM & kShort || q < st.q) && c.ok && j < NR) {
       bool loaded = false;
-      if constexpr (OP != OP_ANY)
+      if constexpr (OP != OP_ANY && OP != OP_R2R)
         if (!from_lds) {
           op_load<T, OP, R>(a, c, j, NR, v[q]);
           loaded = true;
@@ -625,7 +626,7 @@ __device__ __forceinline__ void load_line(const LineArgs<T> &a, const MixGeom &m
         walk([&](const MixCtx<T> &at, int p, C2<T> *v) {
           *v = swapri(pre_elem<T, int>(mode, at.in, FLAT ? 1 : a.esi, int(a.bign), a.f.n, p,
                                        (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_CONJ) != 0,
-                                       (a.sub & R2R_FLIP) != 0, TableRoot<T>{a.t0}),
+                                       (a.sub & R2R_FLIP) != 0, root_of<(FORM & kSinCos) != 0>(a)),
                       a.dir > T(0));
         });
       });
@@ -837,10 +838,15 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
   if (m.nst == 0) {  // lines of one element
     if (c.ok && c.j == 0) {
       C2<T> v[1];
-      op_load<T, OP, 1>(a, c, 0, 0, v);
+      if constexpr (OP == OP_R2R)
+        v[0] = pre_elem<T, int>(a.sub & 0xff, c.in, a.esi, int(a.bign), a.f.n, 0,
+                                (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_CONJ) != 0,
+                                (a.sub & R2R_FLIP) != 0, root_of<(FORM & kSinCos) != 0>(a));
+      else
+        op_load<T, OP, 1>(a, c, 0, 0, v);
       if (is_blue(op)) kernel_product<T, OP, 1>(a, c, 0, 0, v);
       if (elem_store(op)) op_store<T, OP, 1>(a, c, 0, 0, v);
-      else c.ln[0] = swapri(v[0], OP == OP_R2R && a.dir > T(0));
+      else c.ln[0] = v[0];
     }
     __syncthreads();
   }
@@ -915,7 +921,7 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
             const C2<T> *ln = at.ln;
             y[r] = a.fct * post_elem<T, int>(mode, [&](int q) { return ln[q]; }, int(a.bign), k,
                                              (a.sub & R2R_ORTHO) != 0, (a.sub & R2R_FLIP) != 0,
-                                             TableRoot<T>{a.t0});
+                                             root_of<(FORM & kSinCos) != 0>(a));
             to[r] = at.out + (FLAT ? k : k * a.eso);
           }
 #pragma unroll

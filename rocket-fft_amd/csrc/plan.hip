@@ -334,6 +334,13 @@ struct RealRec {
   std::vector<std::complex<double>> rtw;
 };
 
+struct R2RRec {
+  uint64_t n = 0, m = 0;
+  bool dbl = false;
+  DirectRec d;
+  std::vector<std::complex<double>> roots;
+};
+
 static void make_direct(DirectRec &d, uint64_t n, const std::vector<int> &rad) {
   if (rad.size() > size_t(kMaxStages)) RFH_THROW(3, "too many FFT stages");
   d.desc = FftDesc{};
@@ -634,6 +641,16 @@ static RealRec build_real_rec(uint64_t n, bool dbl, size_t budget) {
   return p;
 }
 
+static R2RRec build_r2r_rec(uint64_t n, uint64_t m, bool dbl) {
+  R2RRec r;
+  r.n = n;
+  r.m = m;
+  r.dbl = dbl;
+  make_direct(r.d, m, even_radices(m));
+  for (uint64_t q = 0; n && q <= 2 * n; ++q) r.roots.push_back(std::conj(wfwd(q, 8 * n)));
+  return r;
+}
+
 static std::shared_ptr<C2CPlan> materialize(const PlanRec &r) {
   auto p = std::make_shared<C2CPlan>();
   p->n = r.n;
@@ -686,6 +703,7 @@ static std::shared_ptr<RealPlan> materialize(const RealRec &r) {
 // budget, stride class) and GPU architecture, so that a later process skips
 // the FP64 table generation (the Bluestein kernel's host DFT above all):
 //   <dir>/plan_<arch>_<c2c|real>_<n>_<c64|c128>_b<budget>_<i|c>.bin
+//   <dir>/plan_<arch>_r2r_<n>_<c64|c128>_b<work length>_c.bin
 // Format: "RFHPLAN1", the key fields, the record, the schedule's version, an
 // FNV-1a checksum of all that; a file that does not parse, checksum or match its
 // key and version is ignored (and rewritten).  Files are written to a temporary
@@ -815,6 +833,18 @@ std::string encode(const RealRec &r) {
   return seal(w);
 }
 
+std::string encode(const R2RRec &r) {
+  Writer w;
+  w.put(uint8_t(2));  // real-to-real
+  w.put(r.n);
+  w.put(uint8_t(r.dbl));
+  w.put(r.m);
+  w.put(uint8_t(0));
+  w.direct(r.d);
+  w.vec(r.roots);
+  return seal(w);
+}
+
 // key fields of a record file; false when they do not match
 bool read_key(Reader &rd, uint8_t kind, uint64_t n, bool dbl, size_t budget, bool inter) {
   uint8_t k = 255, d = 255, it = 255;
@@ -875,6 +905,20 @@ bool decode(const std::string &f, uint64_t n, bool dbl, size_t budget, RealRec *
   r->fused = fu != 0;
   r->half = ha != 0;
   return rd.ok && rd.at == pay.size();
+}
+
+bool decode(const std::string &f, uint64_t n, bool dbl, size_t m, R2RRec *r) {
+  const std::string pay = unseal(f);
+  if (pay.empty()) return false;
+  Reader rd{pay};
+  if (!read_key(rd, 2, n, dbl, m, false)) return false;
+  r->n = n;
+  r->m = m;
+  r->dbl = dbl;
+  rd.direct(r->d);
+  rd.vec(r->roots);
+  return rd.ok && rd.at == pay.size() && uint64_t(r->d.desc.n) == m &&
+         r->roots.size() == (n ? 2 * n + 1 : 0);
 }
 
 std::mutex g_cache_mu;
@@ -1010,29 +1054,34 @@ std::shared_ptr<RealPlan> get_real_plan(uint64_t n, bool dbl, size_t budget) {
   });
 }
 
-std::shared_ptr<R2RPlan> get_r2r_plan(uint64_t n, uint64_t m, bool dbl) {
+bool r2r_one_pass(uint64_t m, bool dbl) {
   uint64_t bn2 = 0;
-  if (m > direct_max(dbl, 1) || (m > 1 && plan_bluestein(m, false, &bn2))) return nullptr;
+  return m <= direct_max(dbl, 1) && !(m > 1 && plan_bluestein(m, false, &bn2));
+}
+
+std::shared_ptr<R2RPlan> find_r2r_plan(uint64_t n, uint64_t m, bool dbl) {
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
-  const auto key = std::make_tuple(dev, n, m, dbl);
-  {
-    std::lock_guard<std::mutex> lk(g_cache_mu);
-    auto it = g_r2r.find(key);
-    if (it != g_r2r.end()) return it->second;
-  }
+  std::lock_guard<std::mutex> lk(g_cache_mu);
+  auto it = g_r2r.find(std::make_tuple(dev, n, m, dbl));
+  return it == g_r2r.end() ? nullptr : it->second;
+}
+
+std::shared_ptr<R2RPlan> get_r2r_plan(uint64_t n, uint64_t m, bool dbl) {
+  if (auto p = find_r2r_plan(n, m, dbl)) return p;
+  int dev = 0;
+  HIP_CHECK(hipGetDevice(&dev));
+  // (a record's key has one length and a budget: here n and m)
+  const R2RRec r = cached_record<R2RRec>("r2r", n, dbl, size_t(m), false,
+                                         [&] { return build_r2r_rec(n, m, dbl); });
   auto p = std::make_shared<R2RPlan>();
   p->n = n;
   p->m = m;
   p->dbl = dbl;
-  DirectRec d;
-  make_direct(d, m, even_radices(m));
-  upload_direct(p->d, d, dbl);
-  std::vector<std::complex<double>> roots(2 * n + 1);
-  for (uint64_t q = 0; q <= 2 * n; ++q) roots[q] = std::conj(wfwd(q, 8 * n));
-  upload_any(p->roots, roots, dbl);
+  upload_direct(p->d, r.d, dbl);
+  if (!r.roots.empty()) upload_any(p->roots, r.roots, dbl);
   std::lock_guard<std::mutex> lk(g_cache_mu);
-  return g_r2r.emplace(key, p).first->second;
+  return g_r2r.emplace(std::make_tuple(dev, n, m, dbl), p).first->second;
 }
 
 void plan_cache_dir(const std::string &dir, bool clear_memory) {

@@ -126,7 +126,8 @@ struct RealPlan {
 };
 
 // Real-to-real line of n in one LDS pass through a complex FFT of m points:
-// the FFT and the table e^{i pi q / 4n}, q <= 2n, of the DCT / DST factors.
+// the FFT and the table e^{i pi q / 4n}, q <= 2n, of the DCT / DST factors (n = 0:
+// no table, for the modes without factors).
 struct R2RPlan {
   uint64_t n = 0, m = 0;
   bool dbl = false;
@@ -148,9 +149,12 @@ bool fast_interleaved_ok(uint64_t n, bool dbl);
 std::shared_ptr<C2CPlan> get_c2c_plan(uint64_t n, bool dbl, size_t lds_budget = 0,
                                       bool interleaved = false);
 std::shared_ptr<RealPlan> get_real_plan(uint64_t n, bool dbl, size_t lds_budget = 0);
-// ... of a real-to-real line, or null when a complex FFT of m points does not
-// run in one LDS pass (or runs as Bluestein).
+// Whether a real-to-real line's complex FFT of m points runs in one LDS pass
+// (and not as Bluestein); the plan of such a line of n (0: without factors), and
+// the one there is, or null.
+bool r2r_one_pass(uint64_t m, bool dbl);
 std::shared_ptr<R2RPlan> get_r2r_plan(uint64_t n, uint64_t m, bool dbl);
+std::shared_ptr<R2RPlan> find_r2r_plan(uint64_t n, uint64_t m, bool dbl);
 // The cached plan of get_c2c_plan's arguments on the current device, or
 // null when none was built yet (never allocates).
 std::shared_ptr<C2CPlan> find_c2c_plan(uint64_t n, bool dbl, size_t lds_budget = 0,
@@ -280,8 +284,12 @@ struct RealPrePost {
   bool conj = false;  // pre: conjugate input spectrum; post: conjugate output
   bool flip = false;  // negate entries 2, 4, 6, ... (FFTPACK sign rule)
 };
-// pre -> FFT of length rr.m -> post in one LDS pass (p of rr.n and rr.m).
-void launch_r2r_fused(const R2RPlan &p, const LineSet &g, PreMode pre, PostMode post,
+// whether a mode multiplies by the DCT / DST factors
+bool mode_has_factors(PreMode pre, PostMode post);
+// pre -> FFT of length rr.m (d) -> post in one LDS pass; roots: the factors' table
+// of rr.n, or null (computed in the kernel).
+void launch_r2r_fused(const Direct &d, const void *roots, bool dbl, const LineSet &g, PreMode pre,
+                      PostMode post,
                       const RealPrePost &rr, bool fft_forward, double fct, hipStream_t s);
 void launch_pre(PreMode mode, const RealPrePost &rp, const LineSet &g, bool dbl,
                 void *tmp_complex, hipStream_t s);
