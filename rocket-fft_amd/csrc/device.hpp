@@ -165,8 +165,7 @@ constexpr int R2R_ORTHO = 1 << 16, R2R_CONJ = 1 << 17, R2R_FLIP = 1 << 18;
 constexpr int R2R_SINCOS = 1 << 19;  // the factors are computed, there is no table
 enum SubFlags {
   SUB_CHIRP = 1,   // pass A: multiply loads by the chirp, zero beyond n
-  SUB_KERNEL = 2,  // pass B: multiply by the Bluestein kernel (natural order)
-  SUB_FINAL = 4,   // pass A or B: multiply by the chirp and fct, keep m = aux + k other < n
+  SUB_FINAL = 4,   // pass A: multiply by the chirp and fct, keep m = aux + k other < n
   SUB_CONJ = 8,    // Bluestein backward / r2c conj output / c2r conj input
 };
 

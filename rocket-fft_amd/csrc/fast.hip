@@ -103,9 +103,7 @@ __device__ __forceinline__ C2<T> fload(const FCtx<T> &c, int p) {
   } else if constexpr (OP == OP_C2R_EVEN) {
     const int h = a.f.n;
     return c2r_pre(a, c.rtw, ldc<VIN>(c.gin + p * a.esi), ldc<VIN>(c.gin + (h - p) * a.esi), p);
-  } else if constexpr (OP == OP_PASSA) {
-    return ldc<VIN>(c.gin + ((p + a.rot_in) & (a.f.n - 1)) * a.esi);
-  } else {  // OP_C2C (power-of-two lengths: the rotation is a mask)
+  } else {  // (power-of-two lengths: the rotation is a mask)
     return ldc<VIN>(c.gin + ((p + a.rot_in) & (a.f.n - 1)) * a.esi);
   }
 }
@@ -178,7 +176,7 @@ __device__ __forceinline__ C2<T> ftwiddle(const LineArgs<T> &a, const C2<T> *twl
 template <typename T, int OP, bool VOUT>
 __device__ __forceinline__ void fstore(const LineArgs<T> &a, const C2<T> *twl, T *gout, int aux,
                                        int p, C2<T> v) {
-  if constexpr (OP == OP_C2C) {
+  if constexpr (OP == OP_C2C || OP == OP_PASSB) {
     stc<VOUT>(gout + ((p + a.rot_out) & (a.f.n - 1)) * a.eso, a.fct * v);
   } else if constexpr (OP == OP_PASSA) {
     if (a.sub & SUB_FINAL) {  // Bluestein columns, last pass: chirp and fct, m < n
@@ -195,20 +193,6 @@ __device__ __forceinline__ void fstore(const LineArgs<T> &a, const C2<T> *twl, T
   } else if constexpr (OP == OP_BLUEROW) {  // inverse four-step twiddle, in place
     const C2<T> w = dirw(big_twiddle(a, int64_t(p) * aux), T(1));
     stc<VOUT>(gout + p * a.eso, cmul(v, w));
-  } else if constexpr (OP == OP_PASSB) {
-    const int64_t m = aux + int64_t(p) * a.other;
-    const bool cj = (a.sub & SUB_CONJ) != 0;
-    if (a.sub & SUB_KERNEL) {
-      const C2<T> w = a.t1[m];
-      stc<VOUT>(gout + p * a.eso, cmul(v, cj ? conjc(w) : w));
-    } else if (a.sub & SUB_FINAL) {
-      if (m < a.bign) {
-        const C2<T> ch = a.t0[m];
-        stc<VOUT>(gout + p * a.eso, a.fct * cmul(v, cj ? ch : conjc(ch)));
-      }
-    } else {
-      stc<VOUT>(gout + ((p + a.rot_out) & (a.f.n - 1)) * a.eso, a.fct * v);
-    }
   } else if constexpr (OP == OP_C2R_EVEN) {
     const C2<T> z = a.fct * v;
     if constexpr (VOUT) {

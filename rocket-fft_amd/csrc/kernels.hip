@@ -553,7 +553,8 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 // Lines per group of a four-step pass over lines of n: at least `base`
 // adjacent lines (64-byte row segments), more for short lines until a group
-// holds 2048 elements or its two LDS buffers reach 64 KB (or the plan's budget).
+// holds 2048 elements or its LDS reaches 32 KB (or half the plan's budget), so
+// that several groups share a CU.
 int pass_lines(const C2CPlan &p, uint64_t n, int base) {
   const size_t elem = p.dbl ? 16 : 8;
   const size_t cap = std::min<size_t>(p.budget ? p.budget : 65536, 65536);

@@ -841,8 +841,7 @@ bool launch_pass1024_pipe(int mode, bool pass_a, const dev::LineArgs<float> &a0,
 const char *launch_pass1024(int mode, int op, const dev::LineArgs<float> &a, bool lf_in,
                             bool lf_out, hipStream_t s) {
   const bool pass_a = op == OP_PASSA && lf_in && lf_out && !(a.sub & (SUB_CHIRP | SUB_FINAL));
-  const bool pass_b = op == OP_PASSB && !lf_in && lf_out &&
-                      !(a.sub & (SUB_KERNEL | SUB_FINAL));
+  const bool pass_b = op == OP_PASSB && !lf_in && lf_out;
   if (!pass_a && !pass_b) return nullptr;
   if (a.f.nst != 3 || a.f.st[0].radix != 16 || a.f.st[1].radix != 16 || a.f.st[2].radix != 4)
     return nullptr;

@@ -284,7 +284,7 @@ std::unique_ptr<Built> build(const std::vector<rfh_job_t> &jobs, bool dbl, size_
   // pass 3: device tables; tiles by level and workgroup size
   struct Item {  // one pass
     double cost;  // of all its tiles: elements x stages, a prime stage by its sums
-  double time;  // of one tile, in the same units over its threads
+    double time;  // of one tile, in the same units over its threads
     int pass, tiles, level, cls;
     size_t lds;
   };
