@@ -246,17 +246,21 @@ MixGeom mix_geometry(const Desc &f, const int *pbo, bool dbl, int64_t nlines, bo
     // of 5 to 7 waves fill the four SIMDs unevenly: lines of 1000 (100
     // threads) in threes / fives, 65536 of them c64 263 / 240 us, 32000 c128
     // 297 / 250; of 600 (40 threads) in eights / sixes 16000 c64 41.6 / 36.5
+    // (no more lines than leave every CU two groups, nor than fit: 2730 lines of
+    // 1536 double in fives, half of the nines that fill their waves best, 41.4 us,
+    // in threes 23.8)
+    const int64_t most = std::min({int64_t(kMixLines), int64_t(512 / m.T), nlines / 512,
+                                   int64_t(cap / (size_t(ld) * elem))});
     double best = 0;
-    for (int l = std::max(1, 192 / m.T); l * m.T <= 512 && l <= kMixLines; ++l) {
-      const int t = l * m.T, waves = (t + 63) / 64;
+    for (int64_t l = std::max<int64_t>(1, std::min<int64_t>(192 / m.T, most)); l <= most; ++l) {
+      const int t = int(l) * m.T, waves = (t + 63) / 64;
       const double use = double(t) / double(64 * waves) * (waves > 4 && waves < 8 ? 0.9 : 1.0);
       if (use > best + 0.02) {
         best = use;
-        L = l;
+        L = int(l);
       }
       if (best >= 0.92) break;
     }
-    while (L > 1 && (nlines < int64_t(L) * 512 || size_t(L) * ld * elem > cap)) L = (L + 1) / 2;
   }
   m.L = L;
   while ((1 << m.log2L) < L) ++m.log2L;

@@ -1,6 +1,7 @@
 """Groups of short lines.  Host: an interleaved group of short lines fills more
 than half of its waves' lanes and stays inside the workgroup and its LDS, at
-every length to 100.  GPU: short lengths along axis 0 with enough lines for
+every length to 100; a contiguous group fills its waves as well as any smaller
+one.  GPU: short lengths along axis 0 with enough lines for
 whole waves, the last group a part of one, against numpy in FP64, forward and
 inverse, complex, real and back.  Bar: rel-L2 <= 1e-6 / 1e-13."""
 import subprocess
@@ -48,6 +49,33 @@ DRIVER = textwrap.dedent(r"""
                 return 1;
               }
             }
+      // contiguous lines: a set too small for the group that fills its waves best
+      // takes the best of those it has two a CU of, not a part of that group
+      for (int dbl = 0; dbl < 2; ++dbl)
+        for (int n = 2; n <= 1000; ++n)
+          for (int64_t lines : {int64_t(600), int64_t(2730), int64_t(9000)}) {
+            const std::vector<int> rad = even_radices(uint64_t(n));
+            Desc f{};
+            f.n = n;
+            int pbo[24] = {}, ns = 1;
+            for (int R : rad) {
+              f.st[f.nst] = St{R, ns, 0, 0};
+              pbo[f.nst++] = block_pitch(ns * R, ns, dbl);
+              ns *= R;
+            }
+            if (rad.back() > 17) continue;
+            const MixGeom m = line_geometry(f, pbo, dbl, lines, false, 0, 160 * 1024);
+            auto use = [&](int l) {
+              const int t = l * m.T, waves = (t + 63) / 64;
+              return double(t) / (64 * waves) * (waves > 4 && waves < 8 ? 0.9 : 1.0);
+            };
+            bool ok = m.L >= 1 && (m.L == 1 || m.L * 512 <= lines) && m.L * m.T <= 1024;
+            for (int l = std::max(1, 192 / m.T); l < m.L; ++l) ok = ok && use(l) <= use(m.L);
+            if (!ok) {
+              std::printf("FAIL n=%d dbl=%d lines=%d: %d lines of %d\n", n, dbl, int(lines), m.L, m.T);
+              return 1;
+            }
+          }
       std::printf("OK\n");
       return 0;
     }
