@@ -20,12 +20,20 @@ namespace rfh {
 // 29.9, of 2 lines (DCT-II) of 4.2M 105.6 -> 77.5.
 constexpr int kShortThreads = 512;
 
-// (Five waves per SIMD for the sums of many complex64 lines with a prime: 29 of
-// 144631 lines 33.6 us at four, 30.9 at five.)
+// Waves per SIMD that the compiler is held to (1: what the threads allow).  Five
+// for the sums of many complex64 lines with a prime: 29 of 144631 lines 33.6 us at
+// four, 30.9 at five.  Six for complex64 groups that move flat, by three registers:
+// r2c of 24 on 349525 lines 25.2 -> 21.3, 64M pairs of reals in lines of 48 332 -> 311.
+constexpr int kernel_waves(bool dbl, int op, int form) {
+  if (dbl) return 1;
+  if (form == dev::kFlat) return 6;
+  return form == dev::kPrime && op != dev::OP_PASSA ? 5 : 1;
+}
+
 template <typename T, int OP, int FORM>
 __global__ void __launch_bounds__(FORM == 0 || FORM & dev::kPrime ? dev::kMixThreads<T>
                                                                   : kShortThreads,
-                                  FORM == dev::kPrime && sizeof(T) == 4 && OP != dev::OP_PASSA ? 5 : 1)
+                                  kernel_waves(sizeof(T) == 8, OP, FORM))
     k_lines(const dev::LineArgs<T> a, const MixGeom m, int64_t tile0) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   dev::mix_body<T, OP, FORM>(a, m, tile0 + int64_t(dev::xcd_tile()), smem_raw);
