@@ -397,8 +397,8 @@ def lengths_config(torch, R, stream, reps):
 
 def ragged_config(torch, R, stream):
     """4096 transforms of log-uniform lengths 64..65536 (70% good sizes, 30%
-    raw incl. primes; 60% c2c complex64, 40% r2c float32) in one persistent
-    launch, against one drop-in call per transform."""
+    raw incl. primes; 60% c2c complex64, 40% r2c float32) in a few
+    launches, against one drop-in call per transform."""
     spec = R.ragged_workload(njobs=4096, seed=5)
     jobs, nbytes = [], 0
     g = torch.Generator(device="cuda")
