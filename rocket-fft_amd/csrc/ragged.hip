@@ -117,7 +117,7 @@ __device__ void post_line(const LineArgs<T> &a, int tile) {
 // One tile per workgroup.  Bound by a tile's latency (about 20 us for 4096
 // elements of a column pass: arguments, loads, two twiddled exchanges, stores,
 // each waiting for the one before) times the 16 waves per CU that 128
-// registers allow: 4096 jobs 1857 -> 912 us, 2.4 GB of traffic at 2.6 TB/s,
+// registers allow: 4096 jobs 1857 -> 865 us, 1.8 GB of traffic at 2.1 TB/s,
 // against 256-thread workgroups that pulled units from a queue and ran every
 // tile, long or short, with two line buffers.
 template <typename T>
