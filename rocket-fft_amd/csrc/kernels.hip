@@ -99,17 +99,20 @@ LineArgs<T> make_line_args(const PassSpec &ps, const LineSet &g) {
 // 24 60.2 / 24.1.  More: a prime of 37 48.5 / 33.4, 61 49.7 / 40.6, r2c of 96
 // 36.4 / 26.9, but 48 20.6 / 24.0 (16.6 / 20.0), 77 20.4 / 24.4: such lines of
 // complex64 move flat only where they are beyond the 256 MB of the last cache
-// (64M elements of 36 302 / 255, of 60 310 / 242).
+// (64M elements of 36 302 / 255, of 60 310 / 242).  Lines of every other element
+// likewise (12 41.2 / 24, 24 29.2 / 28.2).
 template <typename T>
 bool flat_lines(int op, const LineArgs<T> &a, const MixGeom &m) {
   const int64_t bi = a.nb ? a.bsi[0] : 0, bo = a.nb ? a.bso[0] : 0;
   if (!is_flat_op(op) || a.lfast_in || a.lfast_out || a.nb > 1 || m.L < 2 || m.nst == 0 ||
-      a.esi != (real_in(op) ? 1 : 2) || a.eso != (real_out(op) ? 1 : 2) || a.rot_in || a.rot_out ||
+      std::min(a.esi, a.eso) < 1 || std::max(a.esi, a.eso) >= (1 << 20) || a.rot_in || a.rot_out ||
       std::min(bi, bo) < 0 || std::max(bi, bo) >= (1 << 20))  // (places are 24-bit products)
     return false;
+  // (pairs of reals are one load or store)
+  if ((op == OP_R2C_EVEN && a.esi != 1) || (op == OP_C2R_EVEN && a.eso != 1)) return false;
   // the factors of a work line longer than the real one (types 1 and 4) outweigh
   // its loads: DCT-IV of 15 float 51.2 by place, 63.4 flat
-  if (op == OP_R2R && a.f.n != a.bign) return false;
+  if (op == OP_R2R && (a.f.n != a.bign || a.esi != 1 || a.eso != 1)) return false;
   if (m.T == 1)
     return a.f.n > (op == OP_R2C_ODD || op == OP_C2R_ODD || op == OP_C2R_EVEN ? 5 : 2);
   if (m.T == 2) return true;

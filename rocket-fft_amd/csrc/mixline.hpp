@@ -163,15 +163,23 @@ __device__ __forceinline__ C2<T> step_twiddle(const LineArgs<T> &a, int k, int a
 template <typename T, int OP, int R>
 constexpr int kFactors = OP == OP_ANY ? R : (sizeof(T) == 8 ? 4 : 8);
 
+// The element stride of a line that moves flat: 24-bit products (flat_lines).
+struct Stride24 {
+  int v;
+  __device__ __forceinline__ explicit Stride24(int64_t s) : v(int(s)) {}
+  __device__ __forceinline__ operator int() const { return v; }
+};
+__device__ __forceinline__ int operator*(int i, Stride24 s) { return __mul24(i, s.v); }
+
 // Inputs j + r NR (r < R) of a line, with the op's pre-processing.  CLAMP:
-// beyond the line its last element instead.  FLAT: of adjacent elements.
+// beyond the line its last element instead.  FLAT: 24-bit strides.
 template <typename T, int OP, int R, bool CLAMP = false, bool FLAT = false>
 __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c, int j, int NR,
                                         C2<T> *v) {
   constexpr int S = kFactors<T, OP, R>;
   const bool cj = (a.sub & SUB_CONJ) != 0;
-  using Es = std::conditional_t<FLAT, int, int64_t>;
-  const Es es = FLAT ? Es(real_in(OP) ? 1 : 2) : Es(a.esi);
+  using Es = std::conditional_t<FLAT, Stride24, int64_t>;
+  const Es es = Es(a.esi);
   const int op = op_of<OP>(a);
   auto at = [&](int r) { return CLAMP ? min(j + r * NR, a.f.n - 1) : j + r * NR; };
   if (op == OP_C2C || op == OP_PASSB || op == OP_BLUEROW || op == OP_PASSA) {
@@ -200,7 +208,7 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
       for (int r = 0; r < R; ++r) v[r] = gload(c.in + rot_index(at(r), a.rot_in, a.nin) * es);
     } else {
       const T *p = c.in + j * es;
-      const Es step = NR * es;
+      const auto step = NR * es;
 #pragma unroll
       for (int r = 0; r < R; ++r) v[r] = gload(CLAMP ? c.in + at(r) * es : p + r * step);
     }
@@ -223,8 +231,8 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
     }
   } else if (op == OP_R2C_EVEN) {
     const T *p = c.in + 2 * j * es;
-    const Es step = 2 * NR * es;
-    if (es == 1) {
+    const auto step = 2 * NR * es;
+    if (FLAT || es == 1) {
 #pragma unroll
       for (int r = 0; r < R; ++r) v[r] = gload(CLAMP ? c.in + 2 * at(r) * es : p + r * step);
     } else {
@@ -240,7 +248,7 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
   } else if (op == OP_C2R_EVEN) {
     const int h = a.f.n;
     const T *p = c.in + j * es, *pm = c.in + (h - j) * es;
-    const Es step = NR * es;
+    const auto step = NR * es;
     C2<T> xm[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -281,14 +289,14 @@ __device__ __forceinline__ void op_load(const LineArgs<T> &a, const MixCtx<T> &c
 }
 
 // Bins j + r ns (r < R), with the op's post-processing.  CLAMP: those beyond
-// the line are left out.  FLAT: to adjacent elements.
+// the line are left out.  FLAT: 24-bit strides.
 template <typename T, int OP, int R, bool CLAMP = false, bool FLAT = false>
 __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &c, int j, int ns,
                                          C2<T> *v) {
   constexpr int S = kFactors<T, OP, R>;
   const bool cj = (a.sub & SUB_CONJ) != 0;
-  using Es = std::conditional_t<FLAT, int, int64_t>;
-  const Es es = FLAT ? Es(real_out(OP) ? 1 : 2) : Es(a.eso);
+  using Es = std::conditional_t<FLAT, Stride24, int64_t>;
+  const Es es = Es(a.eso);
   const int op = op_of<OP>(a);
   auto in_line = [&](int r) { return !CLAMP || j + r * ns < a.f.n; };
   if (is_blue(op) || (op != OP_R2C_ODD && a.dir > T(0))) {  // the inverse transform ran on exchanged parts
@@ -296,7 +304,7 @@ __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &
     for (int r = 0; r < R; ++r) v[r] = C2<T>{v[r].y, v[r].x};
   }
   T *p = c.out + j * es;
-  const Es step = ns * es;
+  const auto step = ns * es;
   if (op == OP_C2C || op == OP_PASSB) {
     if (a.rot_out) {
 #pragma unroll
@@ -375,7 +383,7 @@ __device__ __forceinline__ void op_store(const LineArgs<T> &a, const MixCtx<T> &
       }
   } else if (op == OP_C2R_EVEN) {
     T *q = c.out + 2 * j * es;
-    if (es == 1) {
+    if (FLAT || es == 1) {
 #pragma unroll
       for (int r = 0; r < R; ++r)
         if (in_line(r)) gstore(q + 2 * r * step, a.fct * v[r]);
@@ -904,7 +912,7 @@ __device__ __forceinline__ void mix_body(const LineArgs<T> &a, const MixGeom &m,
         const int k = w.place(e, at);
         const bool end = k == 0 || k == h;
         real_bin(a, k, h, at.ln[end ? 0 : k], at.ln[end ? 0 : h - k],
-                 at.out + (FLAT ? 2 * k : k * a.eso));
+                 at.out + (FLAT ? k * Stride24(a.eso) : k * a.eso));
       }
     }
   }

@@ -177,3 +177,34 @@ def test_prime_radices_few_and_many_lines(n, dtype):
         c = t.T.contiguous()
         R.c2c(c, c, np.array([0]), True, 1.0)
         assert rel_l2(c.T.cpu().numpy(), want) <= tol_of(dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n", [3, 6, 9, 12, 17, 24, 30, 37])
+def test_short_rows_of_spread_elements(n, dtype):
+    """Rows of every third input element to every second output one; what lies
+    between the outputs stays."""
+    import torch
+    lines, ax = 512 * 64 + 5, np.array([1])
+    print(f"case spread rows ({lines}, {n}) {dtype.__name__}", flush=True)
+    rs = np.random.RandomState(200 + n)
+    z = (rs.standard_normal((lines, 3 * n)) + 1j * rs.standard_normal((lines, 3 * n))).astype(dtype)
+    r = rs.standard_normal((lines, 3 * n)).astype(RTYPE[dtype])
+    t, x = torch.from_numpy(z).cuda()[:, ::3], torch.from_numpy(r).cuda()[:, ::3]
+    tol, h = tol_of(dtype), n // 2 + 1
+    wide = torch.full((lines, 2 * n), 7, dtype=t.dtype, device="cuda")
+    R.c2c(t, wide[:, ::2], ax, False, 1.0 / n)
+    assert rel_l2(wide[:, ::2].cpu().numpy(), np.fft.ifft(z[:, ::3].astype(np.complex128), axis=1)) <= tol
+    assert bool((wide[:, 1::2] == 7).all())
+    half = torch.full((lines, 2 * h), 7, dtype=t.dtype, device="cuda")
+    R.r2c(x, half[:, ::2], ax, True, 1.0)
+    assert rel_l2(half[:, ::2].cpu().numpy(), np.fft.rfft(r[:, ::3].astype(np.float64), axis=1)) <= tol
+    assert bool((half[:, 1::2] == 7).all())
+    back = torch.full((lines, 2 * n), 7, dtype=x.dtype, device="cuda")
+    R.c2r(half[:, ::2], back[:, ::2], ax, False, 1.0 / n)
+    assert rel_l2(back[:, ::2].cpu().numpy(), r[:, ::3]) <= 2 * tol and bool((back[:, 1::2] == 7).all())
+    y = torch.empty((lines, n), dtype=x.dtype, device="cuda")
+    R.r2r_separable_hartley(x, y, ax, 1.0)
+    f = np.fft.fft(r[:, ::3].astype(np.float64), axis=1)
+    assert rel_l2(y.cpu().numpy(), f.real + f.imag) <= tol
